@@ -192,3 +192,15 @@ def test_head_sample(O, tglib):
             assert tok.value == S.sample(ref_logits, T, top_p, u)[0]
     finally:
         tglib.tg_head_destroy(h)
+
+
+@pytest.mark.parametrize("V", [1023, 1024, 1025, 1032, 8191, 9215, 9216, 9217, 17408, 17409])
+def test_sample_ordered_sum_edges(tglib, sampler_factory, V):
+    """The parallel ordered sums at the edges of the one-wave head (1024 values) and of the block tiles (8192 after
+    it): every token a candidate, tied values (ties to even on half ulps), spread and nearly equal ones."""
+    gpu_note(f"tg_sampler_run ordered sums V={V}")
+    s = sampler_factory(V)
+    for name, T in (("llm", 1.0), ("ties", 1.3), ("flat", 0.02)):
+        check_case(tglib, s, logit_set(name, V, V + 1), T, 1.0, us=(0.0, 0.3, 0.77, 0.9999999))
+        check_case(tglib, s, logit_set(name, V, V + 1), T, 0.97, us=(0.5,))
+    check_case(tglib, s, np.zeros(V, np.float32), 1.0, 1.0, us=(0.25, 0.9999999))

@@ -38,7 +38,7 @@
 //                 running sum past top_p (they hold the candidates); when
 //                 they hold at most 8192 elements, their keys (descending q,
 //                 ascending id) gathered into LDS, sorted by a bitonic network
-//                 8 keys per thread, and the scans by one wave
+//                 8 keys per thread, and the ordered sums as block scans
 // More candidates (flat distributions, top_p near 1): the host then gathers
 // the keys in global memory (k_smp_compact), sorts them (8192-key tiles in
 // registers and LDS, longer steps one launch each), and k_smp_unpack,
@@ -146,111 +146,217 @@ TG_DEV float wave_pw_sum(const float *v, int n, PwTree &t) {
     return t.v[0][0];
 }
 
-// ------------------------------------------------ one-wave ordered scans
-// First k in [0, n) whose fp32 running sum s_k = s_{k-1} + v[k] (s_{-1} = 0)
-// satisfies (double)s_k >= top_p, or -1.  The wave forms the sums in order
-// (each value read from its lane), 64 per step; the sums only grow, so a
-// step whose last sum stays below top_p holds no crossing, and the step that
-// crosses is formed again keeping each lane's own sum.
-TG_DEV int wave_cut(const float *v, int n, double top_p) {
-    constexpr int B = 8;  // values per lane per batch; the next batch is loaded while one is summed
-    const int lane = __lane_id();
-    float run = 0.0f;
-    float x[B], xn[B];
+// ------------------------------------------------ ordered running sums, in parallel
+// The running sum s_k = round(s_{k-1} + v_k) of descending values v_k >= 0
+// (fp32, or float64 of fp32 values) is defined by its order; walked by one
+// wave, 151,936 of them took 1,230 us in fp32 and two walks 1,690 us in
+// float64.  While the sum stays inside one binade [2^e, 2^(e+1)) it is a
+// multiple of the binade's ulp, and what a run of additions adds to it depends
+// on where it starts only through the parity of that multiple (it decides the
+// ties).  So each lane adds its run to 2^e and to 2^e + ulp: the differences
+// are what the run adds to an even and to an odd sum, and these pairs compose
+// associatively.  A scan over the lanes' pairs gives every lane the exact sum
+// before its run, and the lane then makes its own additions from there.  The
+// first lane whose sum reaches 2^(e+1) still ends on the true sum (it made
+// every addition itself); the lanes after it are scanned again from that sum,
+// once per binade.  v_k <= v_0 <= s throughout; pairs past a crossing may be
+// inexact and are not used.  The same 151,936 values now take 36 us (fp32 cut)
+// and 72 us (float64 draw): one block, bound by its additions and 19 tiles of
+// two barriers each.  (Values loaded one dword at a time instead of two float4
+// per lane: 95 and 113 us.  Ulps counted as 64-bit integers: 166 and 192 us.)
+template <class F> struct Grid;  // the sum's binade as 2^e, its ulp, a value's parity in ulps
+template <> struct Grid<float> {
+    TG_DEV static float binade(float s) { return __uint_as_float(__float_as_uint(s) & 0x7F800000u); }
+    static constexpr float ULP = 0x1p-23f;
+    TG_DEV static bool odd(float v) { return __float_as_uint(v) & 1u; }
+};
+template <> struct Grid<double> {
+    TG_DEV static double binade(double s) {
+        return __longlong_as_double(__double_as_longlong(s) & 0x7FF0000000000000ll);
+    }
+    static constexpr double ULP = 0x1p-52;
+    TG_DEV static bool odd(double v) { return __double_as_longlong(v) & 1; }
+};
+// what a run of additions adds to a sum that is an even / odd number of ulps
+template <class F> struct Hop { F d0, d1; };
+// run a, then run b, in binade c
+template <class F> TG_DEV Hop<F> hop_join(F c, const Hop<F> &a, const Hop<F> &b) {
+    return {a.d0 + (Grid<F>::odd(c + a.d0) ? b.d1 : b.d0), a.d1 + (Grid<F>::odd(c + a.d1) ? b.d0 : b.d1)};
+}
+// lanes without a source read 0
+template <int CTRL, int ROWS> TG_DEV float dpp_0(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, ROWS, 0xF, false));
+}
+template <int CTRL, int ROWS> TG_DEV double dpp_0(double v) {
+    const unsigned long long b = __double_as_longlong(v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, CTRL, ROWS, 0xF, false);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), CTRL, ROWS, 0xF, false);
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+template <int CTRL, int ROWS, class F> TG_DEV Hop<F> hop_from(const Hop<F> &v) {
+    return {dpp_0<CTRL, ROWS>(v.d0), dpp_0<CTRL, ROWS>(v.d1)};
+}
+// inclusive scan over groups of 16 lanes, then over the wave ({0, 0} is the identity)
+template <class F> TG_DEV Hop<F> hop_scan16(F c, Hop<F> v) {
+    v = hop_join(c, hop_from<0x111, 0xF>(v), v);  // row_shr:1
+    v = hop_join(c, hop_from<0x112, 0xF>(v), v);  // row_shr:2
+    v = hop_join(c, hop_from<0x114, 0xF>(v), v);  // row_shr:4
+    v = hop_join(c, hop_from<0x118, 0xF>(v), v);  // row_shr:8
+    return v;
+}
+template <class F> TG_DEV Hop<F> hop_scan(F c, Hop<F> v) {
+    v = hop_scan16(c, v);
+    v = hop_join(c, hop_from<0x142, 0xA>(v), v);  // row_bcast:15 into rows 1 and 3
+    v = hop_join(c, hop_from<0x143, 0xC>(v), v);  // row_bcast:31 into rows 2 and 3
+    return v;
+}
+
+constexpr int ORD_R = 8;        // values per lane and scan
+constexpr int ORD_NW = 16;      // waves of a block scan
+constexpr int ORD_HEAD = 1024;  // values summed by one wave first (most of the binades lie there)
+constexpr int ORD_TILE = ORD_NW * WAVE * ORD_R;
+constexpr int ORD_LOG = 2 + SMP_VMAX / ORD_TILE;
+struct OrdLds {
+    Hop<double> t[ORD_NW];  // the waves' totals
+    double s[ORD_NW];       // per wave, its first event: the sum after that lane's run (no event: after its last),
+    int end[ORD_NW];        // that lane's end (INT_MAX: no event)
+    int hit[ORD_NW];        // and the index that satisfies the predicate (-1: the binade's end)
+    double s0;              // the head's result
+    float s2;               // the candidates' sum
+    int pos0, pick;
+    double log[ORD_LOG];    // the sum before each tile
+};
+
+// Continues the running sum s of the values before pos (a multiple of 8; at 0,
+// s = v[0] and the sum goes on from v[1]) over v[pos..n) (each divided by div
+// when DIV), by NW waves (NW == 1: any one wave; else the whole block of ORD_NW
+// waves).  v is 16-byte aligned and readable to the next multiple of 8 values.
+// Returns the first index whose running sum satisfies pred (monotone), or -1
+// with s the sum of all.  log: the sum before each tile.
+template <class F, int NW, bool DIV, class Pred>
+TG_DEV int ord_run(const float *v, float div, int n, int pos, F &s, Pred pred, OrdLds &L, double *log) {
+    constexpr int TILE = NW * WAVE * ORD_R;
+    const int lane = __lane_id(), w = NW == 1 ? 0 : (int)threadIdx.x / WAVE, slot = (w * WAVE + lane) * ORD_R;
+    float raw[ORD_R];
+    F x[ORD_R];
+    // two 16-byte loads, unconditional (at the last group of 8 past the end,
+    // whose values are not used), so that they stay in flight during a scan
+    auto load = [&](int p0) {
+        const float4 *g = reinterpret_cast<const float4 *>(v + min(p0 + slot, (n - 1) & ~(ORD_R - 1)));
+        const float4 a = g[0], b = g[1];
+        raw[0] = a.x; raw[1] = a.y; raw[2] = a.z; raw[3] = a.w;
+        raw[4] = b.x; raw[5] = b.y; raw[6] = b.z; raw[7] = b.w;
+    };
+    load(pos);
+    for (; pos < n; pos += TILE) {
 #pragma unroll
-    for (int r = 0; r < B; r++) x[r] = r * WAVE + lane < n ? v[r * WAVE + lane] : 0.0f;
-    for (int b = 0; b < n; b += B * WAVE) {
-#pragma unroll
-        for (int r = 0; r < B; r++) {
-            const int i = b + (B + r) * WAVE + lane;
-            xn[r] = i < n ? v[i] : 0.0f;
+        for (int j = 0; j < ORD_R; j++) {
+            const int i = pos + slot + j;
+            const float q = DIV ? raw[j] / div : raw[j];
+            x[j] = i > 0 && i < n ? (F)q : (F)0;
         }
+        load(pos + TILE);
+        if (NW > 1 && log && threadIdx.x == 0) *log++ = (double)s;
+        const int end = min(pos + slot + ORD_R, n);  // of this lane's run
+        for (;;) {
+            // x: this tile's values not yet in s (those that are, and past n: 0)
+            const F c = Grid<F>::binade(s), c1 = c + c * Grid<F>::ULP;
+            F a0 = c, a1 = c1;
 #pragma unroll
-        for (int r = 0; r < B; r++) {
-            const float start = run;
-#pragma unroll
-            for (int i = 0; i < WAVE; i++) run = run + rdl(x[r], i);
-            if ((double)run >= top_p) {
-                float s = start, mine = 0.0f;
-#pragma unroll
-                for (int i = 0; i < WAVE; i++) {
-                    s = s + rdl(x[r], i);
-                    mine = lane == i ? s : mine;
-                }
-                const int base = b + r * WAVE;
-                const uint64_t hit = __ballot(base + lane < n && (double)mine >= top_p);
-                return base + __ffsll((long long)hit) - 1;
+            for (int j = 0; j < ORD_R; j++) {
+                a0 = a0 + x[j];
+                a1 = a1 + x[j];
             }
-        }
+            const Hop<F> inc = hop_scan(c, Hop<F>{a0 - c, a1 - c1});
+            Hop<F> ex = hop_from<0x138, 0xF>(inc);  // wave_shr:1
+            if (NW > 1) {
+                if (lane == WAVE - 1) L.t[w] = {(double)inc.d0, (double)inc.d1};
+                lds_barrier();  // (the next tile's loads stay in flight)
+                const Hop<double> td = L.t[lane & (NW - 1)];
+                const Hop<F> ti = hop_scan16(c, Hop<F>{(F)td.d0, (F)td.d1});
+                if (w > 0) ex = hop_join(c, Hop<F>{rdl(ti.d0, w - 1), rdl(ti.d1, w - 1)}, ex);
+            }
+            const F sl = s + (Grid<F>::odd(s) ? ex.d1 : ex.d0);
+            F se = sl;
 #pragma unroll
-        for (int r = 0; r < B; r++) x[r] = xn[r];
+            for (int j = 0; j < ORD_R; j++) se = se + x[j];
+            const uint64_t m = __ballot(se >= c + c || pred(se));
+            int first = WAVE - 1, at = INT_MAX, hit = -1;
+            if (m) {
+                first = __ffsll((unsigned long long)m) - 1;
+                at = __builtin_amdgcn_readlane(end, first);
+                F r = sl;
+                int k = 0;
+#pragma unroll
+                for (int j = 0; j < ORD_R; j++) {
+                    r = r + x[j];
+                    k += pred(r) ? 0 : 1;
+                }
+                k = __builtin_amdgcn_readlane(k, first);
+                if (k < ORD_R) hit = pos + (w * WAVE + first) * ORD_R + k;
+            }
+            F sn = rdl(se, first);
+            if (NW > 1) {
+                if (lane == 0) { L.end[w] = at; L.s[w] = (double)sn; L.hit[w] = hit; }
+                lds_barrier();
+                const uint64_t me = __ballot(lane < NW && L.end[lane & (NW - 1)] != INT_MAX);
+                const int fw = me ? __ffsll((unsigned long long)me) - 1 : NW - 1;
+                at = L.end[fw];
+                sn = (F)L.s[fw];
+                hit = L.hit[fw];
+            }
+            s = sn;
+            if (at == INT_MAX) break;  // the whole tile is in s
+            if (hit >= 0) return hit;
+#pragma unroll
+            for (int j = 0; j < ORD_R; j++)
+                if (end <= at) x[j] = (F)0;
+        }
     }
     return -1;
 }
 
-// The float64 running sum of (double)(v[k] / s2) over k < n: its last value
-// (cdf[-1] of RandomState.choice).
-TG_DEV double wave_total(const float *v, int n, float s2) {
-    const int lane = __lane_id();
-    double run = 0.0;
-    for (int b = 0; b < n; b += WAVE) {
-        const double x = b + lane < n ? (double)(v[b + lane] / s2) : 0.0;
-#pragma unroll
-        for (int i = 0; i < WAVE; i++) run = run + rdl(x, i);
+// The running sum of v[0..n) (n >= 1) by a block of ORD_NW waves: its first
+// index that satisfies pred, or -1 and s the whole sum.
+template <class F, bool DIV, class Pred>
+TG_DEV int ord_block(const float *v, float div, int n, F &s, Pred pred, OrdLds &L, double *log) {
+    if (threadIdx.x < WAVE) {
+        F h = (F)(DIV ? v[0] / div : v[0]);
+        int at = 0;
+        if (!pred(h)) at = ord_run<F, 1, DIV>(v, div, min(n, ORD_HEAD), 0, h, pred, L, nullptr);
+        if (threadIdx.x == 0) { L.s0 = (double)h; L.pos0 = at; }
     }
-    return run;
+    __syncthreads();
+    s = (F)L.s0;
+    const int at = L.pos0;
+    if (at >= 0 || n <= ORD_HEAD) return at;
+    return ord_run<F, ORD_NW, DIV>(v, div, n, ORD_HEAD, s, pred, L, log);
 }
 
-// First k whose float64 running sum divided by tot exceeds u
-// (cdf.searchsorted(u, side='right')); n - 1 if none (u < 1 never gets there).
-TG_DEV int wave_draw(const float *v, int n, float s2, double tot, double u) {
-    const int lane = __lane_id();
-    double run = 0.0;
-    for (int b = 0; b < n; b += WAVE) {
-        const double x = b + lane < n ? (double)(v[b + lane] / s2) : 0.0;
-        const double start = run;
-#pragma unroll
-        for (int i = 0; i < WAVE; i++) run = run + rdl(x, i);
-        if (run / tot > u) {
-            double r = start, mine = 0.0;
-#pragma unroll
-            for (int i = 0; i < WAVE; i++) {
-                r = r + rdl(x, i);
-                mine = lane == i ? r : mine;
-            }
-            const uint64_t hit = __ballot(b + lane < n && mine / tot > u);
-            return b + __ffsll((long long)hit) - 1;
-        }
+// First k whose float64 running sum of (double)(v[k] / s2), divided by the
+// last one, exceeds u (cdf.searchsorted(u, side='right')), by a block of
+// ORD_NW waves: the sums of the tiles, then the tile that holds the draw.
+TG_DEV int ord_draw(const float *v, int n, float s2, double u, OrdLds &L) {
+    double tot;
+    ord_block<double, true>(v, s2, n, tot, [](double) { return false; }, L, L.log + 1);
+    const int nt = 1 + (n > ORD_HEAD ? (n - ORD_HEAD + ORD_TILE - 1) / ORD_TILE : 0);  // the head, then tiles
+    if (threadIdx.x == 0) L.pick = nt - 1;
+    __syncthreads();
+    for (int t = threadIdx.x; t + 1 < nt; t += ORD_NW * WAVE)
+        if (L.log[t + 1] / tot > u) atomicMin(&L.pick, t);
+    __syncthreads();
+    const int t = L.pick;
+    auto hit = [=](double s) { return s / tot > u; };
+    double s;
+    int at;
+    if (t == 0) {
+        at = ord_block<double, true>(v, s2, min(n, ORD_HEAD), s, hit, L, nullptr);
+    } else {
+        const int p0 = ORD_HEAD + (t - 1) * ORD_TILE;
+        s = L.log[t];
+        at = ord_run<double, ORD_NW, true>(v, s2, min(n, p0 + ORD_TILE), p0, s, hit, L, nullptr);
     }
-    return n - 1;
-}
-
-// The same draw when every (double)(v[k] / s2) is >= 2^-29: each is then a
-// multiple of 2^-52 (24 significant bits), every running sum a multiple of
-// 2^-52 below 2, so the float64 running sums are exact and equal the integer
-// prefix sums in units of 2^-52, formed here in parallel.
-TG_DEV int wave_draw_exact(const float *v, int n, float s2, double u) {
-    const int lane = __lane_id();
-    unsigned long long tot = 0;
-    for (int b = 0; b < n; b += WAVE) {
-        unsigned long long x = b + lane < n ? (unsigned long long)((double)(v[b + lane] / s2) * 0x1p52) : 0ull;
-        for (int s = WAVE / 2; s >= 1; s >>= 1) x += __shfl_xor(x, s, WAVE);
-        tot += x;
-    }
-    const double dt = (double)tot * 0x1p-52;
-    unsigned long long run = 0;
-    for (int b = 0; b < n; b += WAVE) {
-        unsigned long long x = b + lane < n ? (unsigned long long)((double)(v[b + lane] / s2) * 0x1p52) : 0ull;
-        for (int s = 1; s < WAVE; s <<= 1) {  // inclusive scan over the wave
-            const unsigned long long o = __shfl_up(x, s, WAVE);
-            if (lane >= s) x += o;
-        }
-        const double cdf = (double)(run + x) * 0x1p-52;
-        const uint64_t hit = __ballot(b + lane < n && cdf / dt > u);
-        if (hit) return b + __ffsll((long long)hit) - 1;
-        run += __shfl(x, WAVE - 1, WAVE);
-    }
-    return n - 1;
+    return at < 0 ? n - 1 : at;
 }
 
 // np.sum of v[0..n) as buffers of 8192 added from 0, by one wave
@@ -260,29 +366,30 @@ TG_DEV float wave_np_sum(const float *v, int n, PwTree &t) {
     return s;
 }
 
-// The position drawn among the first cut values (cp = v / s2, descending).
-TG_DEV int wave_pick(const float *v, int cut, float s2, double u) {
-    if (v[cut - 1] / s2 >= 0x1p-29f) return wave_draw_exact(v, cut, s2, u);
-    return wave_draw(v, cut, s2, wave_total(v, cut, s2), u);
-}
-
-// The candidates' draw from their q in descending order (v[0..n)): writes
-// cut and the token drawn.
-TG_DEV void wave_finish(const float *v, int n, int V, double top_p, double u, PwTree &t, SmpCtl *ctl,
-                        const uint32_t *ids) {
-    int cut = wave_cut(v, n, top_p);
+// The candidates' draw from their q in descending order (v[0..n), n <= 8192)
+// by a block of ORD_NW waves: writes cut and the token drawn.
+TG_DEV void block_finish(const float *v, int n, int V, double top_p, double u, PwTree &t, OrdLds &L, SmpCtl *ctl,
+                         const uint32_t *ids) {
+    float s;
+    int cut = ord_block<float, false>(v, 1.0f, n, s, [=](float r) { return (double)r >= top_p; }, L, nullptr);
     if (cut < 0) {
         if (n != V) {  // the selection bound guarantees a crossing inside a strict prefix
-            if (__lane_id() == 0) ctl->status = SMP_ST_BOUND;
+            if (threadIdx.x == 0) ctl->status = SMP_ST_BOUND;
             return;
         }
         cut = V;  // searchsorted past the end: every token is a candidate
     } else {
         cut += 1;
     }
-    const float s2 = wave_np_sum(v, cut, t);
-    const int pos = wave_pick(v, cut, s2, u);
-    if (__lane_id() == 0) {
+    __syncthreads();
+    if (threadIdx.x < WAVE) {
+        const float s2 = wave_np_sum(v, cut, t);
+        if (threadIdx.x == 0) L.s2 = s2;
+    }
+    __syncthreads();
+    const float s2 = L.s2;
+    const int pos = ord_draw(v, cut, s2, u, L);
+    if (threadIdx.x == 0) {
         ctl->cut = cut;
         ctl->token = (int)ids[pos];
         ctl->status = SMP_ST_OK;
@@ -574,7 +681,8 @@ __global__ __launch_bounds__(1024) void k_smp_final(const unsigned long long *__
         }
     }
     __syncthreads();
-    if (tid < WAVE) wave_finish(sq, (int)C, V, top_p, u, t, ctl, sid);
+    __shared__ OrdLds ord;
+    block_finish(sq, (int)C, V, top_p, u, t, ord, ctl, sid);
 }
 
 // ------------------------------------------------ more than 8192 candidates
@@ -655,9 +763,11 @@ __global__ __launch_bounds__(SMP_T) void k_smp_unpack(const unsigned long long *
     }
 }
 
-__global__ __launch_bounds__(WAVE) void k_smp_cut(const float *__restrict__ sq, int C, int V, double top_p,
+__global__ __launch_bounds__(1024) void k_smp_cut(const float *__restrict__ sq, int C, int V, double top_p,
                                                   SmpCtl *ctl) {
-    const int c = wave_cut(sq, C, top_p);
+    __shared__ OrdLds ord;
+    float s;
+    const int c = ord_block<float, false>(sq, 1.0f, C, s, [=](float r) { return (double)r >= top_p; }, ord, nullptr);
     if (threadIdx.x == 0) {
         if (c >= 0) ctl->cut = c + 1;
         else if (C == V) ctl->cut = V;
@@ -665,66 +775,16 @@ __global__ __launch_bounds__(WAVE) void k_smp_cut(const float *__restrict__ sq, 
     }
 }
 
-// The draw over cut candidates in global memory.  When every cp >= 2^-29
-// (the exact case of wave_draw_exact) the block's 16 waves take one segment
-// each: segment totals, their prefix, then each wave finds its first hit and
-// the lowest position wins; otherwise wave 0 alone, in order.
+// The draw over cut candidates in global memory.
 __global__ __launch_bounds__(1024) void k_smp_draw(const float *__restrict__ sq, const uint32_t *__restrict__ sid,
                                                    const float *__restrict__ sums, double u, SmpCtl *ctl) {
-    constexpr int NW = 1024 / WAVE;
-    __shared__ unsigned long long seg[NW];
-    __shared__ int s_pos;
+    __shared__ OrdLds ord;
     if (ctl->status != SMP_ST_PENDING) return;
-    const int cut = ctl->cut, tid = threadIdx.x, lane = tid & (WAVE - 1), w = tid / WAVE;
+    const int cut = ctl->cut;
     float s2 = 0.0f;
     for (int c = 0; c * NP_BUFSIZE < cut; c++) s2 = s2 + sums[c];
-    if (!(sq[cut - 1] / s2 >= 0x1p-29f)) {
-        if (tid < WAVE) {
-            const int pos = wave_draw(sq, cut, s2, wave_total(sq, cut, s2), u);
-            if (tid == 0) {
-                ctl->token = (int)sid[pos];
-                ctl->status = SMP_ST_OK;
-            }
-        }
-        return;
-    }
-    const int len = ((cut + NW - 1) / NW + WAVE - 1) / WAVE * WAVE;
-    const int lo = min(cut, w * len), hi = min(cut, lo + len);
-    auto units = [&](int i) -> unsigned long long {
-        return i < hi ? (unsigned long long)((double)(sq[i] / s2) * 0x1p52) : 0ull;
-    };
-    unsigned long long tot = 0;
-    for (int b = lo; b < hi; b += WAVE) {
-        unsigned long long x = units(b + lane);
-        for (int s = WAVE / 2; s >= 1; s >>= 1) x += __shfl_xor(x, s, WAVE);
-        tot += x;
-    }
-    if (lane == 0) seg[w] = tot;
-    if (tid == 0) s_pos = INT_MAX;
-    __syncthreads();
-    unsigned long long run = 0, all = 0;
-    for (int j = 0; j < NW; j++) {
-        if (j < w) run += seg[j];
-        all += seg[j];
-    }
-    const double dt = (double)all * 0x1p-52;
-    for (int b = lo; b < hi; b += WAVE) {
-        unsigned long long x = units(b + lane);
-        for (int s = 1; s < WAVE; s <<= 1) {
-            const unsigned long long o = __shfl_up(x, s, WAVE);
-            if (lane >= s) x += o;
-        }
-        const double cdf = (double)(run + x) * 0x1p-52;
-        const uint64_t hit = __ballot(b + lane < hi && cdf / dt > u);
-        if (hit) {
-            if (lane == 0) atomicMin(&s_pos, b + __ffsll((long long)hit) - 1);
-            break;
-        }
-        run += __shfl(x, WAVE - 1, WAVE);
-    }
-    __syncthreads();
-    if (tid == 0) {
-        const int pos = s_pos == INT_MAX ? cut - 1 : s_pos;
+    const int pos = ord_draw(sq, cut, s2, u, ord);
+    if (threadIdx.x == 0) {
         ctl->token = (int)sid[pos];
         ctl->status = SMP_ST_OK;
     }
@@ -765,7 +825,7 @@ hipError_t launch_sample_large(const SmpBufs &b, int V, int C, double top_p, dou
     }
     const int nchunks = (V + NP_BUFSIZE - 1) / NP_BUFSIZE;
     TG_LAUNCH(k_smp_unpack, dim3(smp_grid(C, SMP_T * 4)), dim3(SMP_T), 0, st, b.keys, C, b.sq, b.sid);
-    TG_LAUNCH(k_smp_cut, dim3(1), dim3(WAVE), 0, st, b.sq, C, V, top_p, b.ctl);
+    TG_LAUNCH(k_smp_cut, dim3(1), dim3(1024), 0, st, b.sq, C, V, top_p, b.ctl);
     TG_LAUNCH(k_smp_chunks, dim3(nchunks), dim3(WAVE), 0, st, b.sq, 0, 1, b.ctl, b.sums);
     TG_LAUNCH(k_smp_draw, dim3(1), dim3(1024), 0, st, b.sq, b.sid, b.sums, u, b.ctl);
     return hipGetLastError();
