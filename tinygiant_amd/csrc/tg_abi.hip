@@ -2263,8 +2263,6 @@ static int sampler_new(int vocab, tg_sampler **out) {
     tg_sampler *s = new tg_sampler{};
     s->vocab = vocab;
     s->dev = g_lg_dev;
-    size_t nk = 16384;
-    while (nk < (size_t)vocab) nk <<= 1;
     const size_t V = (size_t)vocab;
     LgCarve c{nullptr};
     for (int pass = 0; pass < 2; pass++) {
@@ -2276,7 +2274,9 @@ static int sampler_new(int vocab, tg_sampler **out) {
         s->b.sums = c.take<float>(sizeof(float) * 64);
         s->b.hcnt = c.take<uint32_t>(sizeof(uint32_t) * tg::SMP_BUCKETS);
         s->b.hmass = c.take<unsigned long long>(sizeof(unsigned long long) * tg::SMP_BUCKETS);
-        s->b.keys = c.take<unsigned long long>(sizeof(unsigned long long) * nk);
+        s->b.keys = c.take<unsigned long long>(sizeof(unsigned long long) * V);
+        s->b.keys2 = c.take<unsigned long long>(sizeof(unsigned long long) * V);
+        s->b.table = c.take<uint32_t>(sizeof(uint32_t) * tg::SMP_RS_TABLE);
         s->b.sq = c.take<float>(sizeof(float) * V);
         s->b.sid = c.take<uint32_t>(sizeof(uint32_t) * V);
         s->b.ctl = c.take<tg::SmpCtl>(sizeof(tg::SmpCtl));
@@ -2304,7 +2304,11 @@ static int sampler_run(tg_sampler *s, const float *dl, float temperature, double
         return lg_finish(token, s->tok, sizeof(int32_t));
     }
     if (!(u >= 0.0 && u < 1.0)) return set_err(TG_E_INVALID, "sample: u = %g is not in [0, 1)", u);
-    PROFILED("sample", st, tg::launch_sample_main(s->b, dl, s->vocab, temperature, top_p, u, st));
+    const bool all = !(top_p < 1.0) && s->vocab > tg::SMP_SMALL;
+    if (all)
+        PROFILED("sample", st, tg::launch_sample_all(s->b, dl, s->vocab, temperature, top_p, u, st));
+    else
+        PROFILED("sample", st, tg::launch_sample_main(s->b, dl, s->vocab, temperature, top_p, u, st));
     HIP_TRY(hipMemcpyAsync(s->hctl, s->b.ctl, sizeof(tg::SmpCtl), hipMemcpyDeviceToHost, st));
     if (probs) HIP_TRY(hipMemcpyAsync(probs, s->b.q, sizeof(float) * (size_t)s->vocab, hipMemcpyDeviceToHost, st));
     int rc = lg_sync();
@@ -2313,7 +2317,7 @@ static int sampler_run(tg_sampler *s, const float *dl, float temperature, double
     if (c.bad || c.status == tg::SMP_ST_INPUT)
         return set_err(TG_E_INVALID, "sample: the logits hold NaN or +inf, or every logit is -inf");
     if (c.large) {
-        PROFILED("sample_large", st, tg::launch_sample_large(s->b, s->vocab, (int)c.C, top_p, u, st));
+        PROFILED("sample_large", st, tg::launch_sample_large(s->b, s->vocab, top_p, u, st));
         HIP_TRY(hipMemcpyAsync(s->hctl, s->b.ctl, sizeof(tg::SmpCtl), hipMemcpyDeviceToHost, st));
         if ((rc = lg_sync())) return rc;
         c = *s->hctl;

@@ -194,6 +194,7 @@ constexpr int SMP_VMAX = 1 << 19;        // largest vocabulary
 constexpr int SMP_BUCKETS = 4096;        // histogram over q's bits 30..19
 constexpr int SMP_BUCKET_SHIFT = 19;
 constexpr int SMP_SMALL = 8192;          // candidates sorted in one block's LDS
+constexpr int SMP_RS_TABLE = (SMP_VMAX / 4096) * 1024;  // 128 blocks x 1024 digits
 constexpr int NP_BUFSIZE = 8192;         // np.sum reduces in buffers of this many values
 constexpr int SMP_ST_PENDING = -1, SMP_ST_OK = 0, SMP_ST_INPUT = 1, SMP_ST_BOUND = 2;
 struct SmpCtl {
@@ -215,7 +216,8 @@ struct SmpBufs {
     float *sums;                  // 64 buffer sums
     uint32_t *hcnt;               // SMP_BUCKETS
     unsigned long long *hmass;    // SMP_BUCKETS
-    unsigned long long *keys;     // next power of two >= max(vocab, 16384)
+    unsigned long long *keys, *keys2;  // vocab each: the candidates' keys, the sort's passes
+    uint32_t *table;              // SMP_RS_TABLE: the sort's digit counts per block
     float *sq;                    // vocab: sorted probabilities (more than SMP_SMALL candidates)
     uint32_t *sid;                // vocab: their token ids
     SmpCtl *ctl;
@@ -224,7 +226,10 @@ hipError_t sample_prepare();
 // k_smp_max .. k_smp_small; afterwards ctl->large says whether launch_sample_large must finish
 hipError_t launch_sample_main(const SmpBufs &b, const float *logits, int V, float T, double top_p, double u,
                               hipStream_t st);
-hipError_t launch_sample_large(const SmpBufs &b, int V, int C, double top_p, double u, hipStream_t st);
+hipError_t launch_sample_large(const SmpBufs &b, int V, double top_p, double u, hipStream_t st);
+// the whole call over the full sort at once (top_p >= 1 or NaN: every token may be a candidate)
+hipError_t launch_sample_all(const SmpBufs &b, const float *logits, int V, float T, double top_p, double u,
+                             hipStream_t st);
 
 // One-token layer with routing inside (k_layer_dec) and the prologue that
 // forms the first layer's router partials (k_dec_part).  part buffers hold

@@ -39,10 +39,10 @@
 //                 they hold at most 8192 elements, their keys (descending q,
 //                 ascending id) gathered into LDS, sorted by a bitonic network
 //                 8 keys per thread, and the ordered sums as block scans
-// More candidates (flat distributions, top_p near 1): the host then gathers
-// the keys in global memory (k_smp_compact), sorts them (8192-key tiles in
-// registers and LDS, longer steps one launch each), and k_smp_unpack,
-// k_smp_cut, k_smp_chunks and k_smp_draw finish.
+// More candidates (flat distributions, top_p near 1): the host then launches a
+// radix sort of every q (k_rs_count, k_rs_place), and k_smp_cut, k_smp_chunks
+// and k_smp_draw finish.  top_p >= 1 or NaN with more than 8192 tokens goes
+// there at once, without the selection and its wait.
 #include <algorithm>
 
 #include "tg_device.h"
@@ -52,7 +52,6 @@ namespace tg {
 
 constexpr int SMP_T = 256;
 constexpr int PW_LEVELS = 8;   // depth of numpy's pairwise tree over <= 8192 values is 7
-constexpr int BT_TILE = 8192;  // bitonic keys per LDS tile (64 KiB)
 
 TG_DEV uint32_t smp_bucket(float q) {
     const uint32_t b = __float_as_uint(q) >> SMP_BUCKET_SHIFT;
@@ -528,16 +527,19 @@ TG_DEV void smp_select(const uint32_t *hcnt, const unsigned long long *hmass, in
     }
 }
 
+// q = p / S; SELECT: also the histogram, and the candidate buckets from it
+template <bool SELECT>
 __global__ __launch_bounds__(SMP_T) void k_smp_norm(const float *__restrict__ p, int V,
                                                     const float *__restrict__ sums, int nchunks, double top_p,
                                                     SmpCtl *ctl, float *__restrict__ q, uint32_t *hcnt,
                                                     unsigned long long *hmass) {
-    __shared__ uint32_t lc[SMP_BUCKETS];
-    __shared__ unsigned long long lm[SMP_BUCKETS];
+    __shared__ uint32_t lc[SELECT ? SMP_BUCKETS : 1];
+    __shared__ unsigned long long lm[SELECT ? SMP_BUCKETS : 1];
     __shared__ float s_S;
     __shared__ int s_last;
     const int tid = threadIdx.x;
-    for (int b = tid; b < SMP_BUCKETS; b += SMP_T) { lc[b] = 0; lm[b] = 0; }
+    if constexpr (SELECT)
+        for (int b = tid; b < SMP_BUCKETS; b += SMP_T) { lc[b] = 0; lm[b] = 0; }
     if (tid == 0) {
         float S = 0.0f;
         for (int c = 0; c < nchunks; c++) S = S + sums[c];
@@ -549,10 +551,13 @@ __global__ __launch_bounds__(SMP_T) void k_smp_norm(const float *__restrict__ p,
     for (int i = blockIdx.x * SMP_T + tid; i < V; i += gridDim.x * SMP_T) {
         const float v = p[i] / S;
         q[i] = v;
-        const uint32_t b = smp_bucket(v);
-        atomicAdd(&lc[b], 1u);
-        atomicAdd(&lm[b], smp_mass(v));
+        if constexpr (SELECT) {
+            const uint32_t b = smp_bucket(v);
+            atomicAdd(&lc[b], 1u);
+            atomicAdd(&lm[b], smp_mass(v));
+        }
     }
+    if constexpr (!SELECT) return;
     __syncthreads();
     for (int b = tid; b < SMP_BUCKETS; b += SMP_T)
         if (lc[b]) {
@@ -722,57 +727,121 @@ __global__ __launch_bounds__(SMP_T) void k_smp_compact(const float *__restrict__
     }
 }
 
-__global__ __launch_bounds__(SMP_T) void k_fill_u64(unsigned long long *__restrict__ p, int from, int to,
-                                                    unsigned long long v) {
-    for (int i = from + blockIdx.x * SMP_T + threadIdx.x; i < to; i += gridDim.x * SMP_T) p[i] = v;
+// All V probabilities in descending order, ties by ascending id: a stable
+// radix sort of 0x3F800000 - bits(q) (q <= 1: 30 bits) in three passes of 10
+// bits.  Per pass one launch counts each block's digits (table [block][digit])
+// and one places the block's RS_TILE keys: every block sums the table's columns
+// itself (no scan launch between), and inside a block a key's rank among its
+// equals is its wave's count so far plus its lane's place among the lanes with
+// the same digit (one ballot per digit bit).  Bound by the latency of these
+// steps, not by its 1.2 MB a pass: at 151,936 values (38 blocks) 2.6-4.5 us to
+// count and 12-15 us to place, 53 us in all; the bitonic network it replaces
+// took 21 launches and 215 us there, and grew with the next power of two.
+constexpr int RS_T = 1024, RS_R = 4, RS_TILE = RS_T * RS_R, RS_BITS = 10, RS_BINS = 1 << RS_BITS;
+static_assert(RS_BINS == RS_T, "one digit per thread");
+static_assert(SMP_RS_TABLE >= (SMP_VMAX + RS_TILE - 1) / RS_TILE * RS_BINS, "table size");
+template <int PASS>
+TG_DEV unsigned long long rs_load(const float *q, const unsigned long long *src, int i) {
+    if constexpr (PASS == 0) return ((unsigned long long)(0x3F800000u - __float_as_uint(q[i])) << 32) | (uint32_t)i;
+    return src[i];
 }
+template <int PASS>
+TG_DEV uint32_t rs_digit(unsigned long long k) { return (uint32_t)(k >> (32 + PASS * RS_BITS)) & (RS_BINS - 1); }
 
-// Each 8192-key tile through the stages kk = 2..8192 of the global network,
-// or, with kfix, the steps j = 4096..1 of stage kfix.
-__global__ __launch_bounds__(1024) void k_bitonic_tile(unsigned long long *__restrict__ keys, int kfix) {
-    __shared__ unsigned long long x[BT_TILE];
-    const uint32_t g0 = blockIdx.x * BT_TILE;
-    unsigned long long k[8];
+template <int PASS>
+__global__ __launch_bounds__(RS_T) void k_rs_count(const float *__restrict__ q,
+                                                   const unsigned long long *__restrict__ src, int n,
+                                                   uint32_t *__restrict__ table) {
+    __shared__ uint32_t h[RS_BINS];
+    const int tid = threadIdx.x, i0 = blockIdx.x * RS_TILE;
+    unsigned long long k[RS_R];
 #pragma unroll
-    for (int r = 0; r < 8; r++) k[r] = keys[g0 + (threadIdx.x << 3) + r];
-    if (kfix) {
-        for (int j = BT_TILE / 2; j > 0; j >>= 1) bt_step(k, BT_TILE, g0, kfix, j, x);
-    } else {
-        for (int kk = 2; kk <= BT_TILE; kk <<= 1)
-            for (int j = kk >> 1; j > 0; j >>= 1) bt_step(k, BT_TILE, g0, kk, j, x);
-    }
+    for (int r = 0; r < RS_R; r++) k[r] = rs_load<PASS>(q, src, min(i0 + r * RS_T + tid, n - 1));
+    h[tid] = 0;
+    __syncthreads();
 #pragma unroll
-    for (int r = 0; r < 8; r++) keys[g0 + (threadIdx.x << 3) + r] = k[r];
+    for (int r = 0; r < RS_R; r++)
+        if (i0 + r * RS_T + tid < n) atomicAdd(&h[rs_digit<PASS>(k[r])], 1u);
+    __syncthreads();
+    table[(size_t)blockIdx.x * RS_BINS + tid] = h[tid];
 }
 
-// One step (kk, j >= 8192) of the network: one pair per thread.
-__global__ __launch_bounds__(SMP_T) void k_bitonic_step(unsigned long long *__restrict__ keys, int j, int k) {
-    const uint32_t t = blockIdx.x * SMP_T + threadIdx.x;
-    const uint32_t i = ((t / (uint32_t)j) * 2u * (uint32_t)j) + (t % (uint32_t)j), l = i + (uint32_t)j;
-    const unsigned long long a = keys[i], b = keys[l];
-    const bool asc = (i & (uint32_t)k) == 0;
-    if ((a > b) == asc) { keys[i] = b; keys[l] = a; }
-}
-
-__global__ __launch_bounds__(SMP_T) void k_smp_unpack(const unsigned long long *__restrict__ keys, int C,
-                                                      float *__restrict__ sq, uint32_t *__restrict__ sid) {
-    for (int i = blockIdx.x * SMP_T + threadIdx.x; i < C; i += gridDim.x * SMP_T) {
-        const unsigned long long k = keys[i];
-        sq[i] = smp_key_q(k);
-        sid[i] = (uint32_t)k;
+template <int PASS>
+__global__ __launch_bounds__(RS_T) void k_rs_place(const float *__restrict__ q,
+                                                   const unsigned long long *__restrict__ src, int n,
+                                                   const uint32_t *__restrict__ table,
+                                                   unsigned long long *__restrict__ dst, float *__restrict__ sq,
+                                                   uint32_t *__restrict__ sid) {
+    constexpr int NW = RS_T / WAVE;
+    __shared__ uint16_t cnt[NW][RS_BINS];  // per wave and digit: its keys so far, then the keys of earlier waves
+    __shared__ uint32_t base[RS_BINS], wt[NW];
+    const int tid = threadIdx.x, lane = tid & (WAVE - 1), w = tid / WAVE;
+    const int i0 = blockIdx.x * RS_TILE + w * (RS_TILE / NW);  // a wave's keys are contiguous
+    unsigned long long k[RS_R];
+#pragma unroll
+    for (int r = 0; r < RS_R; r++) k[r] = rs_load<PASS>(q, src, min(i0 + r * WAVE + lane, n - 1));
+    uint32_t tot = 0, before = 0;
+#pragma unroll 8
+    for (int b = 0; b < (int)gridDim.x; b++) {
+        const uint32_t c = table[(size_t)b * RS_BINS + tid];
+        tot += c;
+        before += b < (int)blockIdx.x ? c : 0u;
+    }
+    for (int j = 0; j < NW; j++) cnt[j][tid] = 0;
+    uint32_t inc = tot;  // exclusive scan of the digits' totals over the block
+    for (int s = 1; s < WAVE; s <<= 1) {
+        const uint32_t o = __shfl_up(inc, s, WAVE);
+        if (lane >= s) inc += o;
+    }
+    if (lane == WAVE - 1) wt[w] = inc;
+    __syncthreads();
+    uint32_t off = inc - tot + before;
+    for (int j = 0; j < w; j++) off += wt[j];
+    base[tid] = off;
+    uint32_t rank[RS_R];
+#pragma unroll
+    for (int r = 0; r < RS_R; r++) {
+        const bool live = i0 + r * WAVE + lane < n;
+        const uint32_t d = rs_digit<PASS>(k[r]);
+        uint64_t peers = __ballot(live);
+#pragma unroll
+        for (int bit = 0; bit < RS_BITS; bit++) {
+            const bool set = (d >> bit) & 1u;
+            const uint64_t m = __ballot(set);
+            peers &= set ? m : ~m;
+        }
+        const uint32_t below = (uint32_t)__popcll(peers & ((1ull << lane) - 1));
+        rank[r] = cnt[w][d] + below;
+        wave_lds_sync();
+        if (live && below == 0) cnt[w][d] = (uint16_t)(cnt[w][d] + __popcll(peers));
+        wave_lds_sync();
+    }
+    __syncthreads();
+    uint32_t run = 0;
+    for (int j = 0; j < NW; j++) {
+        const uint32_t c = cnt[j][tid];
+        cnt[j][tid] = (uint16_t)run;
+        run += c;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < RS_R; r++) {
+        if (i0 + r * WAVE + lane >= n) continue;
+        const uint32_t d = rs_digit<PASS>(k[r]), at = base[d] + cnt[w][d] + rank[r];
+        if constexpr (PASS == 2) {
+            sq[at] = __uint_as_float(0x3F800000u - (uint32_t)(k[r] >> 32));
+            sid[at] = (uint32_t)k[r];
+        } else {
+            dst[at] = k[r];
+        }
     }
 }
 
-__global__ __launch_bounds__(1024) void k_smp_cut(const float *__restrict__ sq, int C, int V, double top_p,
-                                                  SmpCtl *ctl) {
+__global__ __launch_bounds__(1024) void k_smp_cut(const float *__restrict__ sq, int V, double top_p, SmpCtl *ctl) {
     __shared__ OrdLds ord;
     float s;
-    const int c = ord_block<float, false>(sq, 1.0f, C, s, [=](float r) { return (double)r >= top_p; }, ord, nullptr);
-    if (threadIdx.x == 0) {
-        if (c >= 0) ctl->cut = c + 1;
-        else if (C == V) ctl->cut = V;
-        else ctl->status = SMP_ST_BOUND;
-    }
+    const int c = ord_block<float, false>(sq, 1.0f, V, s, [=](float r) { return (double)r >= top_p; }, ord, nullptr);
+    if (threadIdx.x == 0) ctl->cut = c >= 0 ? c + 1 : V;
 }
 
 // The draw over cut candidates in global memory.
@@ -795,40 +864,53 @@ static unsigned smp_grid(long n, long per) { return (unsigned)std::max<long>(1, 
 
 size_t smp_small_lds() { return sizeof(unsigned long long) * SMP_SMALL + sizeof(PwTree); }
 
-hipError_t launch_sample_main(const SmpBufs &b, const float *logits, int V, float T, double top_p, double u,
-                              hipStream_t st) {
-    if (V <= 0 || V > SMP_VMAX) return hipErrorInvalidValue;
+// p and the buffer sums; then q with or without the candidate selection
+static void launch_probs(const SmpBufs &b, const float *logits, int V, float T, double top_p, bool select,
+                         hipStream_t st) {
     const unsigned nb = smp_grid(V, SMP_T * 4);
     const int nchunks = (V + NP_BUFSIZE - 1) / NP_BUFSIZE;
     TG_LAUNCH(k_smp_max, dim3(nb), dim3(SMP_T), 0, st, logits, V, b.pmax, b.pbad, b.hcnt, b.hmass, b.ctl);
     TG_LAUNCH(k_smp_exp, dim3(smp_grid(V, SMP_T * 2)), dim3(SMP_T), 0, st, logits, V, b.pmax, b.pbad, (int)nb, T,
               b.p, b.ctl);
     TG_LAUNCH(k_smp_chunks, dim3(nchunks), dim3(WAVE), 0, st, b.p, V, 0, b.ctl, b.sums);
-    TG_LAUNCH(k_smp_norm, dim3(smp_grid(V, SMP_T * 8)), dim3(SMP_T), 0, st, b.p, V, b.sums, nchunks, top_p, b.ctl,
-              b.q, b.hcnt, b.hmass);
+    if (select)
+        TG_LAUNCH(k_smp_norm<true>, dim3(smp_grid(V, SMP_T * 8)), dim3(SMP_T), 0, st, b.p, V, b.sums, nchunks,
+                  top_p, b.ctl, b.q, b.hcnt, b.hmass);
+    else
+        TG_LAUNCH(k_smp_norm<false>, dim3(smp_grid(V, SMP_T * 2)), dim3(SMP_T), 0, st, b.p, V, b.sums, nchunks,
+                  top_p, b.ctl, b.q, b.hcnt, b.hmass);
+}
+
+hipError_t launch_sample_main(const SmpBufs &b, const float *logits, int V, float T, double top_p, double u,
+                              hipStream_t st) {
+    if (V <= 0 || V > SMP_VMAX) return hipErrorInvalidValue;
+    launch_probs(b, logits, V, T, top_p, true, st);
     TG_LAUNCH(k_smp_compact, dim3(smp_grid(V, SMP_T * 8)), dim3(SMP_T), 0, st, b.q, V, b.ctl, b.keys);
     TG_LAUNCH(k_smp_final, dim3(1), dim3(1024), smp_small_lds(), st, b.keys, V, top_p, u, b.ctl);
     return hipGetLastError();
 }
 
-hipError_t launch_sample_large(const SmpBufs &b, int V, int C, double top_p, double u, hipStream_t st) {
-    if (C <= SMP_SMALL || C > V || V > SMP_VMAX) return hipErrorInvalidValue;
-    int P = BT_TILE;
-    while (P < C) P <<= 1;
-    TG_LAUNCH(k_fill_u64, dim3(smp_grid(P - C, SMP_T)), dim3(SMP_T), 0, st, b.keys, C, P, ~0ull);
-    const int tiles = P / BT_TILE;
-    TG_LAUNCH(k_bitonic_tile, dim3(tiles), dim3(1024), 0, st, b.keys, 0);
-    for (int k = 2 * BT_TILE; k <= P; k <<= 1) {
-        for (int j = k >> 1; j >= BT_TILE; j >>= 1)
-            TG_LAUNCH(k_bitonic_step, dim3(P / 2 / SMP_T), dim3(SMP_T), 0, st, b.keys, j, k);
-        TG_LAUNCH(k_bitonic_tile, dim3(tiles), dim3(1024), 0, st, b.keys, k);
-    }
+hipError_t launch_sample_large(const SmpBufs &b, int V, double top_p, double u, hipStream_t st) {
+    if (V <= 0 || V > SMP_VMAX) return hipErrorInvalidValue;
+    const dim3 grid((unsigned)((V + RS_TILE - 1) / RS_TILE)), block(RS_T);
+    TG_LAUNCH(k_rs_count<0>, grid, block, 0, st, b.q, b.keys, V, b.table);
+    TG_LAUNCH(k_rs_place<0>, grid, block, 0, st, b.q, b.keys, V, b.table, b.keys, b.sq, b.sid);
+    TG_LAUNCH(k_rs_count<1>, grid, block, 0, st, b.q, b.keys, V, b.table);
+    TG_LAUNCH(k_rs_place<1>, grid, block, 0, st, b.q, b.keys, V, b.table, b.keys2, b.sq, b.sid);
+    TG_LAUNCH(k_rs_count<2>, grid, block, 0, st, b.q, b.keys2, V, b.table);
+    TG_LAUNCH(k_rs_place<2>, grid, block, 0, st, b.q, b.keys2, V, b.table, b.keys, b.sq, b.sid);
     const int nchunks = (V + NP_BUFSIZE - 1) / NP_BUFSIZE;
-    TG_LAUNCH(k_smp_unpack, dim3(smp_grid(C, SMP_T * 4)), dim3(SMP_T), 0, st, b.keys, C, b.sq, b.sid);
-    TG_LAUNCH(k_smp_cut, dim3(1), dim3(1024), 0, st, b.sq, C, V, top_p, b.ctl);
+    TG_LAUNCH(k_smp_cut, dim3(1), dim3(1024), 0, st, b.sq, V, top_p, b.ctl);
     TG_LAUNCH(k_smp_chunks, dim3(nchunks), dim3(WAVE), 0, st, b.sq, 0, 1, b.ctl, b.sums);
     TG_LAUNCH(k_smp_draw, dim3(1), dim3(1024), 0, st, b.sq, b.sid, b.sums, u, b.ctl);
     return hipGetLastError();
+}
+
+hipError_t launch_sample_all(const SmpBufs &b, const float *logits, int V, float T, double top_p, double u,
+                             hipStream_t st) {
+    if (V <= 0 || V > SMP_VMAX) return hipErrorInvalidValue;
+    launch_probs(b, logits, V, T, top_p, false, st);
+    return launch_sample_large(b, V, top_p, u, st);
 }
 
 hipError_t sample_prepare() {
