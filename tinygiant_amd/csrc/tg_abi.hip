@@ -2252,14 +2252,6 @@ static int sampler_new(int vocab, tg_sampler **out) {
     *out = nullptr;
     if (vocab <= 0 || vocab > tg::SMP_VMAX)
         return set_err(TG_E_INVALID, "sampler: vocab %d outside 1..%d", vocab, tg::SMP_VMAX);
-    static bool prepared = false;
-    if (!prepared) {
-        if (tg::sample_prepare() != hipSuccess) {
-            (void)hipGetLastError();
-            return set_err(TG_E_HIP, "sampler: LDS attribute of the sort kernel");
-        }
-        prepared = true;
-    }
     tg_sampler *s = new tg_sampler{};
     s->vocab = vocab;
     s->dev = g_lg_dev;

@@ -191,9 +191,9 @@ hipError_t launch_argmax(const float *x, int n, float *pv, int *pi, int *out, hi
 
 // Temperature / top-p sampling (tg_sample.hip).
 constexpr int SMP_VMAX = 1 << 19;        // largest vocabulary
-constexpr int SMP_BUCKETS = 4096;        // histogram over q's bits 30..19
-constexpr int SMP_BUCKET_SHIFT = 19;
-constexpr int SMP_SMALL = 8192;          // candidates sorted in one block's LDS
+constexpr int SMP_BUCKETS = 1024;        // histogram over q's bits 30..19, from 2^-63
+constexpr int SMP_BUCKET_SHIFT = 19, SMP_BUCKET_LOW = (127 - 63) << 4;
+constexpr int SMP_SMALL = 8192;          // candidates ranked by counting
 constexpr int SMP_RS_TABLE = (SMP_VMAX / 4096) * 1024;  // 128 blocks x 1024 digits
 constexpr int NP_BUFSIZE = 8192;         // np.sum reduces in buffers of this many values
 constexpr int SMP_ST_PENDING = -1, SMP_ST_OK = 0, SMP_ST_INPUT = 1, SMP_ST_BOUND = 2;
@@ -222,8 +222,7 @@ struct SmpBufs {
     uint32_t *sid;                // vocab: their token ids
     SmpCtl *ctl;
 };
-hipError_t sample_prepare();
-// k_smp_max .. k_smp_small; afterwards ctl->large says whether launch_sample_large must finish
+// k_smp_max .. k_smp_final; afterwards ctl->large says whether launch_sample_large must finish
 hipError_t launch_sample_main(const SmpBufs &b, const float *logits, int V, float T, double top_p, double u,
                               hipStream_t st);
 hipError_t launch_sample_large(const SmpBufs &b, int V, double top_p, double u, hipStream_t st);

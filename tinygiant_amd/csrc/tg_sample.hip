@@ -31,19 +31,21 @@
 //   k_smp_max     per-block max of the logits and a non-finite flag; clears
 //                 the histogram
 //   k_smp_exp     p
-//   k_smp_chunks  one wave per 8192-value buffer: its pairwise sum
-//   k_smp_norm    S from the buffer sums; q = p / S; a histogram of q's top
-//                 12 bits with counts and exact mass (units of 2^-40)
-//   k_smp_final   the fewest top buckets whose mass provably carries the fp32
-//                 running sum past top_p (they hold the candidates); when
-//                 they hold at most 8192 elements, their keys (descending q,
-//                 ascending id) gathered into LDS, sorted by a bitonic network
-//                 8 keys per thread, and the ordered sums as block scans
+//   k_smp_chunks  one block per 8192-value buffer: its pairwise sum
+//   k_smp_norm_select  S from the buffer sums; q = p / S; a histogram of q in
+//                 1/16 binades with counts and exact mass (units of 2^-40),
+//                 and from it the fewest top buckets whose mass provably
+//                 carries the fp32 running sum past top_p (they hold the
+//                 candidates)
+//   k_smp_compact their keys (descending q, ascending id)
+//   k_smp_rank    at most 8192 of them: each key to its place
+//   k_smp_final   the cutoff, the candidates' sum and the draw
 // More candidates (flat distributions, top_p near 1): the host then launches a
 // radix sort of every q (k_rs_count, k_rs_place), and k_smp_cut, k_smp_chunks
 // and k_smp_draw finish.  top_p >= 1 or NaN with more than 8192 tokens goes
 // there at once, without the selection and its wait.
 #include <algorithm>
+#include <type_traits>
 
 #include "tg_device.h"
 #include "tg_internal.h"
@@ -53,9 +55,10 @@ namespace tg {
 constexpr int SMP_T = 256;
 constexpr int PW_LEVELS = 8;   // depth of numpy's pairwise tree over <= 8192 values is 7
 
+// 1/16 binades below 1; everything below 2^-63 (and zero) in bucket 0
 TG_DEV uint32_t smp_bucket(float q) {
-    const uint32_t b = __float_as_uint(q) >> SMP_BUCKET_SHIFT;
-    return b < (uint32_t)SMP_BUCKETS ? b : (uint32_t)SMP_BUCKETS - 1;  // NaN with the sign bit
+    const int b = (int)(__float_as_uint(q) >> SMP_BUCKET_SHIFT) - SMP_BUCKET_LOW;
+    return (uint32_t)min(max(b, 0), SMP_BUCKETS - 1);
 }
 // q in [0, 1] in units of 2^-40, rounded down (exact: a power-of-two scale)
 TG_DEV unsigned long long smp_mass(float q) {
@@ -76,22 +79,26 @@ TG_DEV double rdl(double v, int i) {
 }
 
 // ------------------------------------------------ numpy's pairwise sum
-// Base case of numpy's pairwise summation, n <= 128 values v[0..n).
-TG_DEV float pw_leaf(const float *v, int n) {
+// Base case of numpy's pairwise summation, n <= 128 values v[0..n), by 8
+// adjacent lanes (j = lane % 8): each keeps one of the 8 interleaved
+// accumulators; every lane returns the sum.
+TG_DEV float pw_leaf8(const float *v, int n, int j) {
     if (n < 8) {
         float r = 0.0f;
         for (int i = 0; i < n; i++) r = r + v[i];
         return r;
     }
-    float r0 = v[0], r1 = v[1], r2 = v[2], r3 = v[3], r4 = v[4], r5 = v[5], r6 = v[6], r7 = v[7];
     const int main = n & ~7;
-    for (int i = 8; i < main; i += 8) {
-        r0 = r0 + v[i]; r1 = r1 + v[i + 1]; r2 = r2 + v[i + 2]; r3 = r3 + v[i + 3];
-        r4 = r4 + v[i + 4]; r5 = r5 + v[i + 5]; r6 = r6 + v[i + 6]; r7 = r7 + v[i + 7];
-    }
-    float res = ((r0 + r1) + (r2 + r3)) + ((r4 + r5) + (r6 + r7));
-    for (int i = main; i < n; i++) res = res + v[i];
-    return res;
+    float r = v[j];
+    for (int i = 8; i < main; i += 8) r = r + v[i + j];
+    auto dpp = [](float x, auto c) {
+        return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), decltype(c)::value, 0xF, 0xF, false));
+    };
+    r = r + dpp(r, std::integral_constant<int, 0xB1>{});   // lane ^ 1
+    r = r + dpp(r, std::integral_constant<int, 0x4E>{});   // lane ^ 2
+    r = r + dpp(r, std::integral_constant<int, 0x141>{});  // the other quad of 8
+    for (int i = main; i < n; i++) r = r + v[i];
+    return r;
 }
 
 // The recursion's nodes level by level (at most 64 per level for n <= 8192):
@@ -101,47 +108,64 @@ TG_DEV float pw_leaf(const float *v, int n) {
 struct PwTree {
     short st[PW_LEVELS][WAVE], ln[PW_LEVELS][WAVE], ch[PW_LEVELS][WAVE];
     float v[PW_LEVELS][WAVE];
+    short leaf[PW_LEVELS * WAVE];  // level * 64 + index
+    int nleaf;
 };
 
-// numpy's pairwise sum of v[0..n), 1 <= n <= 8192, by one whole wave (every
-// lane returns it).  Leaves are summed one per lane, inner nodes level by
-// level from the bottom, each as left + right.
-TG_DEV float wave_pw_sum(const float *v, int n, PwTree &t) {
-    const int lane = __lane_id();
+// numpy's pairwise sum of v[0..n), 1 <= n <= 8192, by the whole block (1024
+// threads; every thread returns it): wave 0 lays out the tree, every leaf is
+// summed by 8 lanes, and wave 0 adds the inner nodes up, each as left + right.
+// (Leaves one per lane of one wave read 64 lines per load: 6.1 us a buffer.)
+TG_DEV float block_pw_sum(const float *v, int n, PwTree &t) {
+    const int tid = threadIdx.x, lane = tid & (WAVE - 1);
     int cnt[PW_LEVELS];
-    if (lane == 0) { t.st[0][0] = 0; t.ln[0][0] = (short)n; }
-    wave_lds_sync();
-    int c = 1;
-#pragma unroll
-    for (int d = 0; d < PW_LEVELS; d++) {
-        cnt[d] = c;
-        const bool have = lane < c;
-        const int s0 = have ? t.st[d][lane] : 0, l0 = have ? t.ln[d][lane] : 0;
-        const bool split = have && l0 > 128 && d + 1 < PW_LEVELS;
-        const uint64_t m = __ballot(split);
-        const int r = __popcll(m & ((1ull << lane) - 1));
-        if (split) {
-            const int n2 = (l0 >> 1) & ~7;
-            t.st[d + 1][2 * r] = (short)s0;
-            t.ln[d + 1][2 * r] = (short)n2;
-            t.st[d + 1][2 * r + 1] = (short)(s0 + n2);
-            t.ln[d + 1][2 * r + 1] = (short)(l0 - n2);
-        }
-        if (have) t.ch[d][lane] = (short)(split ? 2 * r : -1);
-        c = 2 * __popcll(m);
+    if (tid < WAVE) {
+        if (lane == 0) { t.st[0][0] = 0; t.ln[0][0] = (short)n; }
         wave_lds_sync();
-    }
+        int c = 1, nl = 0;
 #pragma unroll
-    for (int d = PW_LEVELS - 1; d >= 0; d--) {
-        if (lane < cnt[d]) {
-            const int ch = t.ch[d][lane];
-            const int dn = d + 1 < PW_LEVELS ? d + 1 : d;  // children exist only above the last level
-            const float val = ch < 0 ? pw_leaf(v + t.st[d][lane], t.ln[d][lane])
-                                     : t.v[dn][ch] + t.v[dn][ch + 1];
-            t.v[d][lane] = val;
+        for (int d = 0; d < PW_LEVELS; d++) {
+            cnt[d] = c;
+            const bool have = lane < c;
+            const int s0 = have ? t.st[d][lane] : 0, l0 = have ? t.ln[d][lane] : 0;
+            const bool split = have && l0 > 128 && d + 1 < PW_LEVELS;
+            const uint64_t m = __ballot(split), mf = __ballot(have && !split), lt = (1ull << lane) - 1;
+            const int r = __popcll(m & lt);
+            if (split) {
+                const int n2 = (l0 >> 1) & ~7;
+                t.st[d + 1][2 * r] = (short)s0;
+                t.ln[d + 1][2 * r] = (short)n2;
+                t.st[d + 1][2 * r + 1] = (short)(s0 + n2);
+                t.ln[d + 1][2 * r + 1] = (short)(l0 - n2);
+            } else if (have) {
+                t.leaf[nl + __popcll(mf & lt)] = (short)(d * WAVE + lane);
+            }
+            if (have) t.ch[d][lane] = (short)(split ? 2 * r : -1);
+            c = 2 * __popcll(m);
+            nl += __popcll(mf);
+            wave_lds_sync();
         }
-        wave_lds_sync();
+        if (lane == 0) t.nleaf = nl;
     }
+    __syncthreads();
+    const int nl = t.nleaf;
+    for (int g = tid >> 3; g < nl; g += (int)blockDim.x >> 3) {
+        const int at = t.leaf[g], d = at / WAVE, i = at % WAVE;
+        const float r = pw_leaf8(v + t.st[d][i], t.ln[d][i], tid & 7);
+        if ((tid & 7) == 0) t.v[d][i] = r;
+    }
+    __syncthreads();
+    if (tid < WAVE) {
+#pragma unroll
+        for (int d = PW_LEVELS - 2; d >= 0; d--) {
+            if (lane < cnt[d]) {
+                const int ch = t.ch[d][lane];
+                if (ch >= 0) t.v[d][lane] = t.v[d + 1][ch] + t.v[d + 1][ch + 1];
+            }
+            wave_lds_sync();
+        }
+    }
+    __syncthreads();
     return t.v[0][0];
 }
 
@@ -358,43 +382,6 @@ TG_DEV int ord_draw(const float *v, int n, float s2, double u, OrdLds &L) {
     return at < 0 ? n - 1 : at;
 }
 
-// np.sum of v[0..n) as buffers of 8192 added from 0, by one wave
-TG_DEV float wave_np_sum(const float *v, int n, PwTree &t) {
-    float s = 0.0f;
-    for (int c0 = 0; c0 < n; c0 += NP_BUFSIZE) s = s + wave_pw_sum(v + c0, min(NP_BUFSIZE, n - c0), t);
-    return s;
-}
-
-// The candidates' draw from their q in descending order (v[0..n), n <= 8192)
-// by a block of ORD_NW waves: writes cut and the token drawn.
-TG_DEV void block_finish(const float *v, int n, int V, double top_p, double u, PwTree &t, OrdLds &L, SmpCtl *ctl,
-                         const uint32_t *ids) {
-    float s;
-    int cut = ord_block<float, false>(v, 1.0f, n, s, [=](float r) { return (double)r >= top_p; }, L, nullptr);
-    if (cut < 0) {
-        if (n != V) {  // the selection bound guarantees a crossing inside a strict prefix
-            if (threadIdx.x == 0) ctl->status = SMP_ST_BOUND;
-            return;
-        }
-        cut = V;  // searchsorted past the end: every token is a candidate
-    } else {
-        cut += 1;
-    }
-    __syncthreads();
-    if (threadIdx.x < WAVE) {
-        const float s2 = wave_np_sum(v, cut, t);
-        if (threadIdx.x == 0) L.s2 = s2;
-    }
-    __syncthreads();
-    const float s2 = L.s2;
-    const int pos = ord_draw(v, cut, s2, u, L);
-    if (threadIdx.x == 0) {
-        ctl->cut = cut;
-        ctl->token = (int)ids[pos];
-        ctl->status = SMP_ST_OK;
-    }
-}
-
 // ------------------------------------------------ kernels
 __global__ __launch_bounds__(SMP_T) void k_smp_max(const float *__restrict__ l, int V, float *__restrict__ pmax,
                                                    int *__restrict__ pbad, uint32_t *__restrict__ hcnt,
@@ -450,9 +437,9 @@ __global__ __launch_bounds__(SMP_T) void k_smp_exp(const float *__restrict__ l, 
     }
 }
 
-// One wave per 8192-value buffer of v[0..n): its pairwise sum.  n is the
+// One block per 8192-value buffer of v[0..n): its pairwise sum.  n is the
 // argument, or, when n_from_ctl, the candidate count ctl->cut.
-__global__ __launch_bounds__(WAVE) void k_smp_chunks(const float *__restrict__ v, int n, int n_from_ctl,
+__global__ __launch_bounds__(1024) void k_smp_chunks(const float *__restrict__ v, int n, int n_from_ctl,
                                                      const SmpCtl *ctl, float *__restrict__ sums) {
     __shared__ PwTree t;
     if (n_from_ctl) {
@@ -461,8 +448,17 @@ __global__ __launch_bounds__(WAVE) void k_smp_chunks(const float *__restrict__ v
     }
     const int c0 = blockIdx.x * NP_BUFSIZE;
     if (c0 >= n) return;
-    const float s = wave_pw_sum(v + c0, min(NP_BUFSIZE, n - c0), t);
+    const float s = block_pw_sum(v + c0, min(NP_BUFSIZE, n - c0), t);
     if (threadIdx.x == 0) sums[blockIdx.x] = s;
+}
+// np.sum from the buffer sums: added one after another from 0 (n <= 64; every
+// lane of the wave)
+TG_DEV float smp_total(const float *sums, int n) {
+    const int lane = __lane_id();
+    const float x = lane < n ? sums[lane] : 0.0f;
+    float s = 0.0f;
+    for (int c = 0; c < n; c++) s = s + rdl(x, c);
+    return s;
 }
 
 // The candidates lie in the top buckets: with C elements and exact mass M
@@ -471,262 +467,210 @@ __global__ __launch_bounds__(WAVE) void k_smp_chunks(const float *__restrict__ v
 // M 2^-40 - C 2^-24 (each addition rounds by at most half an ulp of a sum
 // below 2), so M 2^-40 >= top_p + C 2^-24 puts the crossing inside them.
 // The largest such b is taken; none (top_p near or above 1, or NaN) = all.
-// A block of NT threads; the histogram is read at device scope (other
+// A block of SL_T threads; the histogram is read at device scope (other
 // blocks' atomics).  Leaves bstar and C in ctl.
-template <int NT>
+constexpr int SL_T = 1024, SL_R = 8;  // threads, values per thread of the selection's launches
+static_assert(SMP_BUCKETS == SL_T, "one bucket per thread");
 TG_DEV void smp_select(const uint32_t *hcnt, const unsigned long long *hmass, int V, double top_p, SmpCtl *ctl) {
-    constexpr int PER = SMP_BUCKETS / NT;
-    __shared__ uint32_t wc[NT / WAVE];
-    __shared__ unsigned long long wm[NT / WAVE];
-    __shared__ int s_best;
-    __shared__ uint32_t s_C;
+    constexpr int NW = SL_T / WAVE;
+    __shared__ uint32_t wc[NW], hC[NW];
+    __shared__ unsigned long long wm[NW];
+    __shared__ int hd[NW];
     const int tid = threadIdx.x, lane = tid & (WAVE - 1), w = tid / WAVE;
-    // descending position d = PER tid + k holds bucket SMP_BUCKETS - 1 - d
-    uint32_t c[PER];
-    unsigned long long ms[PER];
-    uint32_t tc = 0;
-    unsigned long long tm = 0;
-#pragma unroll
-    for (int k = 0; k < PER; k++) {
-        const int b = SMP_BUCKETS - 1 - (PER * tid + k);
-        c[k] = __hip_atomic_load(hcnt + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        ms[k] = __hip_atomic_load(hmass + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        tc += c[k];
-        tm += ms[k];
-    }
-    uint32_t ic = tc;  // inclusive scan of the thread totals over the wave, then over waves
-    unsigned long long im = tm;
+    // descending position tid holds bucket SMP_BUCKETS - 1 - tid
+    const int b = SMP_BUCKETS - 1 - tid;
+    const uint32_t c = __hip_atomic_load(hcnt + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned long long m = __hip_atomic_load(hmass + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    uint32_t cc = c;  // inclusive scan over the wave, then over waves
+    unsigned long long cm = m;
     for (int s = 1; s < WAVE; s <<= 1) {
-        const uint32_t oc = __shfl_up(ic, s, WAVE);
-        const unsigned long long om = __shfl_up(im, s, WAVE);
-        if (lane >= s) { ic += oc; im += om; }
+        const uint32_t oc = __shfl_up(cc, s, WAVE);
+        const unsigned long long om = __shfl_up(cm, s, WAVE);
+        if (lane >= s) { cc += oc; cm += om; }
     }
-    if (lane == WAVE - 1) { wc[w] = ic; wm[w] = im; }
-    if (tid == 0) { s_best = INT_MAX; s_C = (uint32_t)V; }
+    if (lane == WAVE - 1) { wc[w] = cc; wm[w] = cm; }
     __syncthreads();
-    uint32_t cc = ic - tc;
-    unsigned long long cm = im - tm;
     for (int j = 0; j < w; j++) { cc += wc[j]; cm += wm[j]; }
-    int best = INT_MAX;
-    uint32_t bestC = 0;
-#pragma unroll
-    for (int k = 0; k < PER; k++) {
-        cc += c[k];
-        cm += ms[k];
-        const double need = (top_p + (double)cc * 0x1p-24) * 0x1p40 + 1024.0;
-        if (best == INT_MAX && cc >= 1 && (double)cm >= need) { best = PER * tid + k; bestC = cc; }
-    }
-    atomicMin(&s_best, best);
-    __syncthreads();
-    if (best != INT_MAX && best == s_best) s_C = bestC;
+    const double need = (top_p + (double)cc * 0x1p-24) * 0x1p40 + 1024.0;
+    const uint64_t hit = __ballot(cc >= 1 && (double)cm >= need);
+    const int first = hit ? __ffsll((unsigned long long)hit) - 1 : 0;
+    const uint32_t fc = (uint32_t)__builtin_amdgcn_readlane((int)cc, first);
+    if (lane == 0) { hd[w] = hit ? w * WAVE + first : INT_MAX; hC[w] = fc; }
     __syncthreads();
     if (tid == 0) {
-        const int d = s_best;
+        int d = INT_MAX;
+        uint32_t C = (uint32_t)V;
+        for (int j = NW - 1; j >= 0; j--)
+            if (hd[j] != INT_MAX) { d = hd[j]; C = hC[j]; }
         ctl->bstar = d == INT_MAX ? 0 : SMP_BUCKETS - 1 - d;
-        ctl->C = d == INT_MAX ? (uint32_t)V : s_C;
+        ctl->C = C;
     }
 }
 
-// q = p / S; SELECT: also the histogram, and the candidate buckets from it
-template <bool SELECT>
 __global__ __launch_bounds__(SMP_T) void k_smp_norm(const float *__restrict__ p, int V,
-                                                    const float *__restrict__ sums, int nchunks, double top_p,
-                                                    SmpCtl *ctl, float *__restrict__ q, uint32_t *hcnt,
-                                                    unsigned long long *hmass) {
-    __shared__ uint32_t lc[SELECT ? SMP_BUCKETS : 1];
-    __shared__ unsigned long long lm[SELECT ? SMP_BUCKETS : 1];
-    __shared__ float s_S;
+                                                    const float *__restrict__ sums, int nchunks, SmpCtl *ctl,
+                                                    float *__restrict__ q) {
+    const float S = smp_total(sums, nchunks);
+    if (blockIdx.x == 0 && threadIdx.x == 0) ctl->S = S;
+    for (int i = blockIdx.x * SMP_T + threadIdx.x; i < V; i += gridDim.x * SMP_T) q[i] = p[i] / S;
+}
+
+// The same with the histogram; the last block to finish picks the candidate
+// buckets.  Bound by the device-scope atomics on the histogram: few blocks (8
+// values per thread of 1024) so that a bucket takes few of them, and no fence
+// (its write-back of the L2 cost 10 us): 8.3 us at 151,936 values, from 20.
+__global__ __launch_bounds__(SL_T) void k_smp_norm_select(const float *__restrict__ p, int V,
+                                                          const float *__restrict__ sums, int nchunks, double top_p,
+                                                          SmpCtl *ctl, float *__restrict__ q, uint32_t *hcnt,
+                                                          unsigned long long *hmass) {
+    __shared__ uint32_t lc[SMP_BUCKETS];
+    __shared__ unsigned long long lm[SMP_BUCKETS];
     __shared__ int s_last;
-    const int tid = threadIdx.x;
-    if constexpr (SELECT)
-        for (int b = tid; b < SMP_BUCKETS; b += SMP_T) { lc[b] = 0; lm[b] = 0; }
-    if (tid == 0) {
-        float S = 0.0f;
-        for (int c = 0; c < nchunks; c++) S = S + sums[c];
-        s_S = S;
-        if (blockIdx.x == 0) ctl->S = S;
-    }
+    const int tid = threadIdx.x, i0 = blockIdx.x * SL_T * SL_R + tid;
+    float x[SL_R];
+#pragma unroll
+    for (int r = 0; r < SL_R; r++) x[r] = p[min(i0 + r * SL_T, V - 1)];
+    lc[tid] = 0;
+    lm[tid] = 0;
+    const float S = smp_total(sums, nchunks);
+    if (blockIdx.x == 0 && tid == 0) ctl->S = S;
     __syncthreads();
-    const float S = s_S;
-    for (int i = blockIdx.x * SMP_T + tid; i < V; i += gridDim.x * SMP_T) {
-        const float v = p[i] / S;
-        q[i] = v;
-        if constexpr (SELECT) {
+#pragma unroll
+    for (int r = 0; r < SL_R; r++) {
+        const int i = i0 + r * SL_T;
+        if (i < V) {
+            const float v = x[r] / S;
+            q[i] = v;
             const uint32_t b = smp_bucket(v);
             atomicAdd(&lc[b], 1u);
             atomicAdd(&lm[b], smp_mass(v));
         }
     }
-    if constexpr (!SELECT) return;
     __syncthreads();
-    for (int b = tid; b < SMP_BUCKETS; b += SMP_T)
-        if (lc[b]) {
-            atomicAdd(&hcnt[b], lc[b]);
-            atomicAdd(&hmass[b], lm[b]);
-        }
-    // the last block to finish picks the candidate buckets
-    __threadfence();
+    if (lc[tid]) {
+        atomicAdd(&hcnt[tid], lc[tid]);
+        atomicAdd(&hmass[tid], lm[tid]);
+    }
+    // this thread's histogram atomics are done at device scope (a fence would
+    // also write the L2's q back); the last block reads them at device scope
+    __builtin_amdgcn_s_waitcnt(VMCNT0);
     __syncthreads();
-    if (tid == 0) s_last = atomicAdd(&ctl->done, 1u) == gridDim.x - 1;
+    if (tid == 0)
+        s_last = __hip_atomic_fetch_add(&ctl->done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
     __syncthreads();
-    if (s_last) {
-        __threadfence();
-        smp_select<SMP_T>(hcnt, hmass, V, top_p, ctl);
+    if (s_last) smp_select(hcnt, hmass, V, top_p, ctl);
+}
+
+// The candidates' keys (bucket >= ctl->bstar) into keys[0..C), in any order:
+// per block one global slot range.
+__global__ __launch_bounds__(SL_T) void k_smp_compact(const float *__restrict__ q, int V, SmpCtl *ctl,
+                                                      unsigned long long *__restrict__ keys) {
+    __shared__ uint32_t wc[SL_T / WAVE], s_base;
+    const uint32_t bstar = (uint32_t)ctl->bstar;
+    const int tid = threadIdx.x, lane = tid & (WAVE - 1), w = tid / WAVE, i0 = blockIdx.x * SL_T * SL_R + tid;
+    float v[SL_R];
+#pragma unroll
+    for (int r = 0; r < SL_R; r++) v[r] = q[min(i0 + r * SL_T, V - 1)];
+    uint64_t m[SL_R];
+    uint32_t n = 0;
+#pragma unroll
+    for (int r = 0; r < SL_R; r++) {
+        m[r] = __ballot(i0 + r * SL_T < V && smp_bucket(v[r]) >= bstar);
+        n += (uint32_t)__popcll(m[r]);
+    }
+    if (lane == 0) wc[w] = n;
+    __syncthreads();
+    if (tid == 0) {
+        uint32_t t = 0;
+        for (int j = 0; j < SL_T / WAVE; j++) t += wc[j];
+        s_base = t ? atomicAdd(&ctl->n, t) : 0u;
+    }
+    __syncthreads();
+    uint32_t at = s_base;
+    for (int j = 0; j < w; j++) at += wc[j];
+#pragma unroll
+    for (int r = 0; r < SL_R; r++) {
+        if ((m[r] >> lane) & 1)
+            keys[at + __popcll(m[r] & ((1ull << lane) - 1))] = smp_key(v[r], (uint32_t)(i0 + r * SL_T));
+        at += (uint32_t)__popcll(m[r]);
     }
 }
 
-// Bitonic network, 8 keys per thread: thread t holds keys 8t .. 8t+7 of a
-// run whose first key is key g0 of the whole network (g0 a multiple of 8192;
-// the direction of stage kk at key i is ascending when (i & kk) == 0).  One
-// step (kk, j): j < 8 in registers, 8 <= j < 512 with lane t ^ (j / 8) of the
-// same wave, larger through LDS (x, 8 keys per thread).  Every thread of the
-// block calls it; threads with 8t >= n hold no keys (n a power of two >= 8).
-template <int J>
-TG_DEV void bt_reg_step(unsigned long long (&k)[8], uint32_t g, int kk) {
+// At most SMP_SMALL candidates in order: a key's place is the number of
+// smaller keys (they are distinct).  A block places 64 keys, one per lane, its
+// 16 waves each counting over a sixteenth of all keys, read lane by lane: at
+// 1,400 candidates 22 blocks and 6 rounds of 16 keys a wave, 8.8 us, and the
+// scans after it 17 us; with a bitonic network of 66 dependent steps in one
+// block before the scans the two took 57 us.
+__global__ __launch_bounds__(1024) void k_smp_rank(const unsigned long long *__restrict__ keys,
+                                                   const SmpCtl *__restrict__ ctl, float *__restrict__ sq,
+                                                   uint32_t *__restrict__ sid) {
+    constexpr int NW = 1024 / WAVE;
+    __shared__ uint32_t cnt[WAVE];
+    const int tid = threadIdx.x, lane = tid & (WAVE - 1), w = tid / WAVE;
+    const int C = (int)ctl->C, k0 = blockIdx.x * WAVE;
+    if (ctl->bad || C > SMP_SMALL || k0 >= C) return;  // uniform
+    const unsigned long long mine = keys[min(k0 + lane, C - 1)];
+    if (tid < WAVE) cnt[tid] = 0;
+    const int per = (C + NW - 1) / NW, lo = min(w * per, C), hi = min(lo + per, C);
+    __syncthreads();
+    uint32_t n = 0;
+    for (int b = lo; b < hi; b += WAVE) {
+        const unsigned long long o = b + lane < hi ? keys[b + lane] : ~0ull;  // ~0: below no key
+        const int live = min(WAVE, hi - b);
+        for (int i = 0; i < live; i += 16) {  // (lanes past live hold ~0)
 #pragma unroll
-    for (int r = 0; r < 8; r++) {
-        const int l = r ^ J;
-        if (l > r) {
-            const bool asc = ((g + (uint32_t)r) & (uint32_t)kk) == 0;
-            const unsigned long long a = k[r], b = k[l];
-            if ((a > b) == asc) { k[r] = b; k[l] = a; }
-        }
-    }
-}
-
-TG_DEV unsigned long long shfl_xor_u64(unsigned long long v, int m) {
-    const uint32_t lo = (uint32_t)__shfl_xor((int)(uint32_t)v, m, WAVE);
-    const uint32_t hi = (uint32_t)__shfl_xor((int)(uint32_t)(v >> 32), m, WAVE);
-    return ((unsigned long long)hi << 32) | lo;
-}
-
-TG_DEV unsigned long long bt_pick(unsigned long long a, unsigned long long o, bool keep_min) {
-    return keep_min ? (a < o ? a : o) : (a > o ? a : o);
-}
-
-TG_DEV void bt_step(unsigned long long (&k)[8], int n, uint32_t g0, int kk, int j, unsigned long long *x) {
-    const int t = threadIdx.x;
-    const bool act = (t << 3) < n;
-    const uint32_t g = g0 + ((uint32_t)t << 3);
-    if (j >= 512) {
-        if (act) {
-#pragma unroll
-            for (int r = 0; r < 8; r++) x[(t << 3) + r] = k[r];
-        }
-        __syncthreads();
-        if (act) {
-#pragma unroll
-            for (int r = 0; r < 8; r++) {
-                const int i = (t << 3) + r;
-                const bool keep_min = (((g + (uint32_t)r) & (uint32_t)kk) == 0) == ((i & j) == 0);
-                k[r] = bt_pick(k[r], x[i ^ j], keep_min);
+            for (int j = 0; j < 16; j++) {
+                const uint32_t klo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)o, i + j);
+                const uint32_t khi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(o >> 32), i + j);
+                n += (((unsigned long long)khi << 32) | klo) < mine ? 1u : 0u;
             }
         }
-        __syncthreads();
-    } else if (j >= 8) {
-        const int m = j >> 3;  // partner lane t ^ m, in the same wave (m < 64)
-#pragma unroll
-        for (int r = 0; r < 8; r++) {
-            const unsigned long long o = shfl_xor_u64(k[r], m);
-            const bool keep_min = (((g + (uint32_t)r) & (uint32_t)kk) == 0) == ((t & m) == 0);
-            k[r] = bt_pick(k[r], o, keep_min);
-        }
-    } else if (j == 4) {
-        bt_reg_step<4>(k, g, kk);
-    } else if (j == 2) {
-        bt_reg_step<2>(k, g, kk);
-    } else {
-        bt_reg_step<1>(k, g, kk);
+    }
+    atomicAdd(&cnt[lane], n);
+    __syncthreads();
+    if (tid < WAVE && k0 + lane < C) {
+        sq[cnt[lane]] = smp_key_q(mine);
+        sid[cnt[lane]] = (uint32_t)mine;
     }
 }
 
-// Ascending sort of n keys (8 <= n <= 8192, a power of two) held 8 per thread.
-TG_DEV void bitonic_regs(unsigned long long (&k)[8], int n, unsigned long long *x) {
-    for (int kk = 2; kk <= n; kk <<= 1)
-        for (int j = kk >> 1; j > 0; j >>= 1) bt_step(k, n, 0, kk, j, x);
-}
-
-// The last launch of a call: at most 8192 candidates (keys[0..C) from
-// k_smp_compact) sorted in registers and LDS, then the scans by wave 0.
-// More candidates: ctl->large for the host.
-__global__ __launch_bounds__(1024) void k_smp_final(const unsigned long long *__restrict__ keys, int V,
-                                                    double top_p, double u, SmpCtl *ctl) {
-    extern __shared__ __align__(16) uint8_t smem[];
-    unsigned long long *sk = reinterpret_cast<unsigned long long *>(smem);
-    PwTree &t = *reinterpret_cast<PwTree *>(smem + sizeof(unsigned long long) * SMP_SMALL);
-    const int tid = threadIdx.x;
+// The last launch of a call with at most SMP_SMALL candidates: cutoff, the
+// candidates' sum and the draw.  More candidates: ctl->large for the host.
+__global__ __launch_bounds__(1024) void k_smp_final(const float *__restrict__ sq, const uint32_t *__restrict__ sid,
+                                                    int V, double top_p, double u, SmpCtl *ctl) {
+    __shared__ PwTree t;
+    __shared__ OrdLds ord;
+    const int tid = threadIdx.x, C = (int)ctl->C;
     if (ctl->bad) {
         if (tid == 0) ctl->status = SMP_ST_INPUT;
         return;
     }
-    const uint32_t C = ctl->C;
-    if (C > (uint32_t)SMP_SMALL) {
+    if (C > SMP_SMALL) {
         if (tid == 0) ctl->large = 1;
         return;
     }
-    int P = 8;
-    while (P < (int)C) P <<= 1;
-    unsigned long long k[8];
-#pragma unroll
-    for (int r = 0; r < 8; r++) {
-        const int i = (tid << 3) + r;
-        k[r] = i < (int)C ? keys[i] : ~0ull;
-    }
-    bitonic_regs(k, P, sk);
-    __syncthreads();
-    // sorted keys -> q (first half of the array) and ids (second half)
-    float *sq = reinterpret_cast<float *>(smem);
-    uint32_t *sid = reinterpret_cast<uint32_t *>(smem) + SMP_SMALL;
-#pragma unroll
-    for (int r = 0; r < 8; r++) {
-        const int i = (tid << 3) + r;
-        if (i < (int)C) {
-            sq[i] = smp_key_q(k[r]);
-            sid[i] = (uint32_t)k[r];
+    float s;
+    int cut = ord_block<float, false>(sq, 1.0f, C, s, [=](float r) { return (double)r >= top_p; }, ord, nullptr);
+    if (cut < 0) {
+        if (C != V) {  // the selection bound guarantees a crossing inside a strict prefix
+            if (tid == 0) ctl->status = SMP_ST_BOUND;
+            return;
         }
+        cut = V;  // searchsorted past the end: every token is a candidate
+    } else {
+        cut += 1;
     }
-    __syncthreads();
-    __shared__ OrdLds ord;
-    block_finish(sq, (int)C, V, top_p, u, t, ord, ctl, sid);
+    const float s2 = 0.0f + block_pw_sum(sq, cut, t);
+    const int pos = ord_draw(sq, cut, s2, u, ord);
+    if (tid == 0) {
+        ctl->cut = cut;
+        ctl->token = (int)sid[pos];
+        ctl->status = SMP_ST_OK;
+    }
 }
 
 // ------------------------------------------------ more than 8192 candidates
-// The candidates' keys (bucket >= ctl->bstar) into keys[0..C): per block a
-// count, one global slot range, then the keys.
-__global__ __launch_bounds__(SMP_T) void k_smp_compact(const float *__restrict__ q, int V, SmpCtl *ctl,
-                                                       unsigned long long *__restrict__ keys) {
-    __shared__ uint32_t s_cnt, s_base;
-    const uint32_t bstar = (uint32_t)ctl->bstar;
-    const int lane = __lane_id();
-    if (threadIdx.x == 0) s_cnt = 0;
-    __syncthreads();
-    for (int i = blockIdx.x * SMP_T + threadIdx.x; i < V; i += gridDim.x * SMP_T)
-        if (smp_bucket(q[i]) >= bstar) atomicAdd(&s_cnt, 1u);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        s_base = atomicAdd(&ctl->n, s_cnt);
-        s_cnt = 0;
-    }
-    __syncthreads();
-    for (int i0 = blockIdx.x * SMP_T; i0 < V; i0 += gridDim.x * SMP_T) {
-        const int i = i0 + threadIdx.x;
-        float v = 0.0f;
-        bool take = false;
-        if (i < V) {
-            v = q[i];
-            take = smp_bucket(v) >= bstar;
-        }
-        const uint64_t m = __ballot(take);
-        if (m) {
-            const int leader = __ffsll((long long)m) - 1;
-            uint32_t base = 0;
-            if (lane == leader) base = atomicAdd(&s_cnt, (uint32_t)__popcll(m));
-            base = (uint32_t)__shfl((int)base, leader, WAVE);
-            if (take) keys[s_base + base + __popcll(m & ((1ull << lane) - 1))] = smp_key(v, (uint32_t)i);
-        }
-    }
-}
-
 // All V probabilities in descending order, ties by ascending id: a stable
 // radix sort of 0x3F800000 - bits(q) (q <= 1: 30 bits) in three passes of 10
 // bits.  Per pass one launch counts each block's digits (table [block][digit])
@@ -850,8 +794,7 @@ __global__ __launch_bounds__(1024) void k_smp_draw(const float *__restrict__ sq,
     __shared__ OrdLds ord;
     if (ctl->status != SMP_ST_PENDING) return;
     const int cut = ctl->cut;
-    float s2 = 0.0f;
-    for (int c = 0; c * NP_BUFSIZE < cut; c++) s2 = s2 + sums[c];
+    const float s2 = smp_total(sums, (cut + NP_BUFSIZE - 1) / NP_BUFSIZE);
     const int pos = ord_draw(sq, cut, s2, u, ord);
     if (threadIdx.x == 0) {
         ctl->token = (int)sid[pos];
@@ -862,8 +805,6 @@ __global__ __launch_bounds__(1024) void k_smp_draw(const float *__restrict__ sq,
 // ------------------------------------------------ launchers
 static unsigned smp_grid(long n, long per) { return (unsigned)std::max<long>(1, std::min<long>(256, (n + per - 1) / per)); }
 
-size_t smp_small_lds() { return sizeof(unsigned long long) * SMP_SMALL + sizeof(PwTree); }
-
 // p and the buffer sums; then q with or without the candidate selection
 static void launch_probs(const SmpBufs &b, const float *logits, int V, float T, double top_p, bool select,
                          hipStream_t st) {
@@ -872,21 +813,23 @@ static void launch_probs(const SmpBufs &b, const float *logits, int V, float T, 
     TG_LAUNCH(k_smp_max, dim3(nb), dim3(SMP_T), 0, st, logits, V, b.pmax, b.pbad, b.hcnt, b.hmass, b.ctl);
     TG_LAUNCH(k_smp_exp, dim3(smp_grid(V, SMP_T * 2)), dim3(SMP_T), 0, st, logits, V, b.pmax, b.pbad, (int)nb, T,
               b.p, b.ctl);
-    TG_LAUNCH(k_smp_chunks, dim3(nchunks), dim3(WAVE), 0, st, b.p, V, 0, b.ctl, b.sums);
+    TG_LAUNCH(k_smp_chunks, dim3(nchunks), dim3(1024), 0, st, b.p, V, 0, b.ctl, b.sums);
     if (select)
-        TG_LAUNCH(k_smp_norm<true>, dim3(smp_grid(V, SMP_T * 8)), dim3(SMP_T), 0, st, b.p, V, b.sums, nchunks,
-                  top_p, b.ctl, b.q, b.hcnt, b.hmass);
+        TG_LAUNCH(k_smp_norm_select, dim3((unsigned)((V + SL_T * SL_R - 1) / (SL_T * SL_R))), dim3(SL_T), 0, st, b.p,
+                  V, b.sums, nchunks, top_p, b.ctl, b.q, b.hcnt, b.hmass);
     else
-        TG_LAUNCH(k_smp_norm<false>, dim3(smp_grid(V, SMP_T * 2)), dim3(SMP_T), 0, st, b.p, V, b.sums, nchunks,
-                  top_p, b.ctl, b.q, b.hcnt, b.hmass);
+        TG_LAUNCH(k_smp_norm, dim3(smp_grid(V, SMP_T * 2)), dim3(SMP_T), 0, st, b.p, V, b.sums, nchunks, b.ctl, b.q);
 }
 
 hipError_t launch_sample_main(const SmpBufs &b, const float *logits, int V, float T, double top_p, double u,
                               hipStream_t st) {
     if (V <= 0 || V > SMP_VMAX) return hipErrorInvalidValue;
     launch_probs(b, logits, V, T, top_p, true, st);
-    TG_LAUNCH(k_smp_compact, dim3(smp_grid(V, SMP_T * 8)), dim3(SMP_T), 0, st, b.q, V, b.ctl, b.keys);
-    TG_LAUNCH(k_smp_final, dim3(1), dim3(1024), smp_small_lds(), st, b.keys, V, top_p, u, b.ctl);
+    TG_LAUNCH(k_smp_compact, dim3((unsigned)((V + SL_T * SL_R - 1) / (SL_T * SL_R))), dim3(SL_T), 0, st, b.q, V,
+              b.ctl, b.keys);
+    TG_LAUNCH(k_smp_rank, dim3((unsigned)((std::min(V, SMP_SMALL) + WAVE - 1) / WAVE)), dim3(1024), 0, st, b.keys,
+              b.ctl, b.sq, b.sid);
+    TG_LAUNCH(k_smp_final, dim3(1), dim3(1024), 0, st, b.sq, b.sid, V, top_p, u, b.ctl);
     return hipGetLastError();
 }
 
@@ -901,7 +844,7 @@ hipError_t launch_sample_large(const SmpBufs &b, int V, double top_p, double u, 
     TG_LAUNCH(k_rs_place<2>, grid, block, 0, st, b.q, b.keys2, V, b.table, b.keys, b.sq, b.sid);
     const int nchunks = (V + NP_BUFSIZE - 1) / NP_BUFSIZE;
     TG_LAUNCH(k_smp_cut, dim3(1), dim3(1024), 0, st, b.sq, V, top_p, b.ctl);
-    TG_LAUNCH(k_smp_chunks, dim3(nchunks), dim3(WAVE), 0, st, b.sq, 0, 1, b.ctl, b.sums);
+    TG_LAUNCH(k_smp_chunks, dim3(nchunks), dim3(1024), 0, st, b.sq, 0, 1, b.ctl, b.sums);
     TG_LAUNCH(k_smp_draw, dim3(1), dim3(1024), 0, st, b.sq, b.sid, b.sums, u, b.ctl);
     return hipGetLastError();
 }
@@ -911,11 +854,6 @@ hipError_t launch_sample_all(const SmpBufs &b, const float *logits, int V, float
     if (V <= 0 || V > SMP_VMAX) return hipErrorInvalidValue;
     launch_probs(b, logits, V, T, top_p, false, st);
     return launch_sample_large(b, V, top_p, u, st);
-}
-
-hipError_t sample_prepare() {
-    return hipFuncSetAttribute((const void *)k_smp_final, hipFuncAttributeMaxDynamicSharedMemorySize,
-                               (int)smp_small_lds());
 }
 
 }  // namespace tg
