@@ -285,3 +285,23 @@ def test_fused_gate_up_down_across_calls(O, tglib, H, I, E, k, Ts):
             else:
                 os.environ[v] = val
         a.close()
+
+
+# mean entries per expert on both sides of the one-tile / 16 x 16 line (24), odd counts; experts over several
+# one-tile items (16 experts, mean 24) and a shape the fused launches do not take (I 160: the 32 x 32 kernels)
+@pytest.mark.parametrize("H,I,E,k,T", [(2048, 768, 128, 8, 333), (2048, 768, 128, 8, 384), (2048, 768, 128, 8, 385),
+                                       (512, 256, 16, 4, 96), (512, 256, 16, 4, 97), (512, 256, 32, 8, 131),
+                                       (256, 160, 16, 4, 150), (256, 160, 16, 4, 300)])
+def test_item_size_rule_edges(O, tglib, H, I, E, k, T):
+    gpu_note(f"grouped layer at the item size rule's edges H={H} I={I} E={E} T={T}")
+    from tinygiant_amd.moe import MoEBlock
+    a, layers, routers = make_arena(O, 1, H, I, E, k, seed=97)
+    try:
+        x = O.synth_normal(97, O.stream_id(0, T, 4), 1.0, T * H).reshape(T, H)
+        ref, ridx, _, _ = O.moe_layer(layers[0], routers[0], H, I, E, k, x)
+        out, idx, _ = MoEBlock(a).forward(0, dev(x), return_routing=True)
+        assert np.array_equal(host(idx), ridx)
+        assert np.array_equal(bits(host(out)), bits(ref))
+        assert tglib.tg_arena_status(a.handle) == 0
+    finally:
+        a.close()

@@ -1455,10 +1455,17 @@ int mfma_item_entries(const Shape &s, int mt) {
     return mt == 4 && x16_ok(s, true) && x16_ok(s, false) ? XT_CT * 16 : 32 * mt;
 }
 
+// Entries per expert in a work item, in M-tiles of 32, from the batch's mean
+// entries per expert.  Where both fused gate/up + down launches take the shape,
+// the one-tile kernel up to a mean of 24 and the 16 x 16 kernel above: at the
+// 30B shape (us a layer; one-tile, 16 x 16) 333 tokens 171, 182; 420 tokens
+// 186, 184; 512 tokens 219, 199; 1024 tokens 343, 256; at 235B 333 tokens 538,
+// 574; 420 tokens 599, 595; 512 tokens 673, 628.  The 32 x 32 kernels between
+// them (two launches, 247 us at 333 tokens, 382 at 1024, and 862, 1318 at
+// 235B) only take shapes that these do not.
 int mfma_tiles(const Shape &s, int T) {
-    // entries per expert in a work item: up to 4 M-tiles of 32; fewer when
-    // the batch is small or the LDS staging would not fit
     const int avg = (T * s.k + s.E - 1) / s.E;
+    if (mfma_item_entries(s, 4) > 128 && s.nbI % MF_KC == 0 && s.nbI <= MS_FC * MF_KC) return avg > 24 ? 4 : 1;
     return avg > 64 ? 4 : (avg > 16 ? 2 : 1);
 }
 
