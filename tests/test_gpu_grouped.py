@@ -305,3 +305,24 @@ def test_item_size_rule_edges(O, tglib, H, I, E, k, T):
         assert tglib.tg_arena_status(a.handle) == 0
     finally:
         a.close()
+
+
+# the one-tile kernels' staging rings: K of 1, 2, 3, 4, 5, 6, 9 and 12 chunks of 8 blocks (gate/up from H, down from I);
+# rows that fill no block (I 288: 9 tiles of 32, and not whole chunks); T gives items of 1 to 32 entries and split experts
+@pytest.mark.parametrize("H,I", [(256, 256), (512, 768), (768, 512), (1024, 1280), (1280, 1024), (1536, 256),
+                                 (2304, 1536), (3072, 288)])
+@pytest.mark.parametrize("T", [2, 9, 70])
+def test_one_tile_chunk_counts(O, tglib, H, I, T):
+    gpu_note(f"one-tile kernels H={H} I={I} T={T}")
+    from tinygiant_amd.moe import MoEBlock
+    E, k = 16, 4
+    a, layers, routers = make_arena(O, 1, H, I, E, k, seed=103)
+    try:
+        x = O.synth_normal(103, O.stream_id(0, T, 4), 1.0, T * H).reshape(T, H)
+        ref, ridx, _, _ = O.moe_layer(layers[0], routers[0], H, I, E, k, x)
+        out, idx, _ = MoEBlock(a).forward(0, dev(x), return_routing=True)
+        assert np.array_equal(host(idx), ridx)
+        assert np.array_equal(bits(host(out)), bits(ref))
+        assert tglib.tg_arena_status(a.handle) == 0
+    finally:
+        a.close()

@@ -428,43 +428,41 @@ TG_DEV void fused_combine(const FuseArgs &F, const Shape &s, const int32_t *__re
 
 // ================================================================ one M-tile
 // Work items of at most 32 entries (batched decode, a few entries per expert):
-// the operands swap roles, A = the item's Q8_0 activations (lane h*32+m:
-// entry m, elements 16h .. 16h+15 of the block) and B = the weight nibbles
-// (lane h*32+n: weight row n), so lane l, register r of the result holds
-// (entry 8 (r/4) + 4h + r%4, weight row l % 32).  The weight scale is then one
-// value per lane, and the epilogue runs only the register groups (8 entries
-// each) that hold entries of the item.  The weight bytes enter the MFMA as
-// 16 (q - 8) (as in the 16 x 16 kernel) against an inline zero accumulator,
-// so D = 16 S exactly; per block and entry group u16 = round(float(D) * dw)
-// = 16 round(S * dw) and acc = fma(u16, dx / 16, acc) = fma(round(S * dw),
-// dx, acc) bit for bit (powers of two scale exactly), blocks in ascending
-// order: the row-dot definition.  Gate/up: waves 2i / 2i+1
-// take gate / up of tile 2x + i, meet in LDS, and each applies SwiGLU and
-// Q8_0 to half of the entries, each entry's 32 rows (one per lane of a
-// half-wave: maximum and sum by row rotations and a swap of the rows).
-// Weights: per chunk of MF_KC = 8 blocks, lane (n, h) loads row n's blocks
-// 4h .. 4h+3 (64 contiguous bytes; the two lanes of a row cover its whole
-// 128-byte line) and, with nb % 8 == 0, the row's 8 scales in one 16-byte
-// load; the loads of the next two chunks are in flight while this one
-// computes.  Block bl's 16 bytes reach both lanes of the row through one
-// lane-half swap.
+// A = the item's Q8_0 activations (lane h*32+m: entry m, elements 16h .. 16h+15
+// of the block) and B = the weight nibbles (lane h*32+n: weight row n), so lane
+// l, register r of the result holds (entry 8 (r/4) + 4h + r%4, weight row
+// l % 32).  The weight scale is then one value per lane, and the epilogue runs
+// only the register groups (8 entries each) that hold entries of the item.  The
+// weight bytes enter the MFMA as 16 (q - 8) against an inline zero accumulator,
+// so D = 16 S exactly; per block and entry group u16 = round(float(D) * dw/16) =
+// round(S * dw) (powers of two scale exactly) and acc = fma(u16, dx, acc),
+// blocks in ascending order: the row-dot definition.  Gate/up: waves 2i / 2i+1
+// take gate / up of tile 2x + i, meet in LDS, and each applies SwiGLU and Q8_0 to
+// half of the entries, each entry's 32 rows (one per lane of a half-wave:
+// maximum and sum by row rotations and a swap of the rows).
+//
+// The weight stream bounds it.  Per chunk of MF_KC = 8 blocks a wave needs 128
+// bytes of each of its 32 rows.  Four loads of 8 rows x 128 bytes each (whole
+// lines), PF chunks ahead in registers, then through a wave-private LDS buffer
+// into the operand layout (row n's block in both half-waves): a CU streams 57
+// GB/s with this pattern and 34 with each lane loading 64 bytes of its own row
+// (32 half lines a load), which two resident blocks then shared.  The row
+// scales (contiguous over the 32 rows) go straight into LDS, 4 chunks at a
+// time; loaded per chunk, each scale line was fetched once a chunk again and
+// doubled the L1's fill traffic.  The activations of a pair of chunks are
+// staged in one of two LDS slots while the pair before is used; one barrier
+// per pair, none when K spans at most 4 chunks.  68 KB of LDS: two blocks per CU.
+// A layer (30B / 235B shape, weights from HBM), before and after: 5 tokens 75.9 ->
+// 60.7 / 122.9 -> 103 us, 64 tokens 108.5 -> 92.7 / 314 -> 260 us.
 constexpr int MS_NW = 4;    // waves per block
-constexpr int MS_PF = 2;    // weight chunks in flight per wave (down; gate/up one more)
-
-__host__ __device__ inline size_t ms_lds_bytes() { return 2 * 32 * (size_t)MF_TS + 2 * MF_KC * 32 * 4; }
-// Items whose K spans at most MS_FC chunks stage all of their activations
-// once, before the weight loop: [chunk][entry][256 bytes, 16-byte pieces
-// rotated by the entry] then [chunk][block][entry] activation scales.
-constexpr int MS_FC = 8;
-__host__ __device__ inline size_t ms_full_lds_bytes() { return (size_t)MS_FC * (32 * 256 + MF_KC * 32 * 4); }
-
-// one lane-half swap: lo takes half 0's value of v on every lane, hi half 1's
-// (lane i and lane i ^ 32 end with the same pair)
-TG_DEV void half_split(uint32_t v, uint32_t &lo, uint32_t &hi) {
-    const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
-    lo = r[0];
-    hi = r[1];
-}
+constexpr int MS_PF_GATE = 2, MS_PF_DOWN = 3;  // weight chunks in flight per wave (4 in gate/up measured the same)
+struct MsLds {
+    static constexpr int ACT = 0;                    // [4 chunks][32 entries][256 bytes, 16-byte pieces rotated by the entry]
+    static constexpr int DX = ACT + 4 * 32 * 256;    // [4 chunks][8 blocks][32 entries] activation scales
+    static constexpr int WB = DX + 4 * MF_KC * 32 * 4;  // [wave][32 rows][128 bytes, piece p of row r at p ^ (r & 7)]
+    static constexpr int WS = WB + MS_NW * 4096;     // [wave][2][32 rows][4 chunks' scales, chunk p at p ^ (r/2 & 3)]
+    static constexpr int BYTES = WS + MS_NW * 4096;
+};
 
 template <int CTRL>
 TG_DEV float dpp_f(float v) {
@@ -496,15 +494,15 @@ TG_DEV int half_sum(int v) {
     return v;
 }
 
-// One block of the one-tile kernels: item wi, row tile bx.  GD: gate/up and
-// down blocks of the same launch (k_mfma_small_gd): a gate/up block stores
-// h with agent-scope stores and, once they are acknowledged, counts itself in
-// at rdy[wi]; a down block waits (bounded) until all `need` gate/up blocks of
-// its item have, then stages h at agent scope.
-template <bool PAIR, bool SCV, bool FULL, bool GD>
+// One block of the one-tile kernels: item wi, row tile bx; K a whole number of
+// chunks.  GD: gate/up and down blocks of the same launch (k_mfma_small_gd): a
+// gate/up block stores h with agent-scope stores and, once they are
+// acknowledged, counts itself in at rdy[wi]; a down block waits (bounded)
+// until all `need` gate/up blocks of its item have, its first weights in
+// flight meanwhile, then stages h at agent scope.
+template <bool PAIR, bool GD>
 TG_DEV __attribute__((always_inline)) void ms_item(const uint8_t *__restrict__ layer_pl, const Shape s,
                                                    const int32_t *__restrict__ work,
-                                                   const int32_t *__restrict__ work_n,
                                                    const int32_t *__restrict__ entries,
                                                    const int8_t *__restrict__ aq, const float *__restrict__ ad,
                                                    int8_t *__restrict__ oq, float *__restrict__ od,
@@ -513,52 +511,65 @@ TG_DEV __attribute__((always_inline)) void ms_item(const uint8_t *__restrict__ l
     // the launch's dynamic LDS, named here so its addresses stay LDS
     // addresses (through a generic pointer each cast to LDS adds a null test)
     extern __shared__ __align__(16) uint8_t smem[];
-    constexpr int M = 32, NW = MS_NW, NT = NW * 64, TP = 2 * MF_KC;
-    constexpr int NTP = M * TP / NT, NDX = M * MF_KC / NT;
-    static_assert(NT % TP == 0 && NT % MF_KC == 0 && MF_KC == 8 && NTP >= 1 && NDX >= 1, "staging map");
-    static_assert(!GD || PAIR || FULL, "a waiting down block stages its activations once, at agent scope");
-    if (wi >= work_n[0]) return;  // uniform over the block
+    constexpr int M = 32, NW = MS_NW, NT = NW * 64, PF = PAIR ? MS_PF_GATE : MS_PF_DOWN;
+    constexpr int FA = M * 256, FD = MF_KC * M * 4;  // bytes of one chunk's rows, scales of one chunk
+    constexpr int JA = FA / (NT * 16);               // DMA rounds of a chunk's rows
+    static_assert(JA * NT * 16 == FA && NT * 4 == FD && MF_KC == 8, "staging map");
     const int e = work[3 * wi], o = work[3 * wi + 1], c = work[3 * wi + 2];
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, n = lane & 31, h = lane >> 5;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, n = lane & 31,
+              h = lane >> 5;
     const int K = PAIR ? s.H : s.I, nb = K / QK, rows = PAIR ? s.I : s.H, k = s.k;
-    const int nch = (nb + MF_KC - 1) / MF_KC;
+    const int nch = nb / MF_KC;
 
-    uint8_t *tokl = smem;                                                     // [2][M][MF_TS]
-    float *dxl = reinterpret_cast<float *>(smem + 2 * M * MF_TS);             // [2][MF_KC][M]
-
-    const int sp = tid % TP, sb = tid % MF_KC;
-    int toff[NTP], doff[NDX];
-#pragma unroll
-    for (int u = 0; u < NTP; u++) {
-        const int t = tid / TP + u * (NT / TP);
-        toff[u] = -1;
-        if (t < c) toff[u] = (PAIR ? entries[o + t] / k : entries[o + t]) * K;
-    }
-#pragma unroll
-    for (int u = 0; u < NDX; u++) {
-        const int t = tid / MF_KC + u * (NT / MF_KC);
-        doff[u] = -1;
-        if (t < c) doff[u] = (PAIR ? entries[o + t] / k : entries[o + t]) * nb;
-    }
-
+    // this wave's 32 weight rows; an out-of-range tile computes on the first
+    // and stores nothing
     const int mat = PAIR ? (wave & 1) : 0;  // 0 gate / down, 1 up
     const int nt = PAIR ? bx * (NW / 2) + (wave >> 1) : bx * NW + wave;
     const bool valid = nt * 32 < rows;
-    const int R = valid ? nt * 32 + n : n;
-    const uint8_t *ex = layer_pl + (size_t)e * s.EB;
-    const uint8_t *tb = PAIR ? ex + (size_t)mat * s.GB : ex + 2 * s.GB;
-    const size_t ntb = (size_t)rows * nb;
-    const uint4 *q0 = reinterpret_cast<const uint4 *>(tb) + (size_t)R * nb;
-    const uint16_t *s0 = reinterpret_cast<const uint16_t *>(tb + ntb * 16) + (size_t)R * nb;
+    const int r0 = valid ? nt * 32 : 0;
+    const uint8_t *tb = layer_pl + (size_t)e * s.EB + (PAIR ? (size_t)mat * s.GB : 2 * s.GB);
+    const uint8_t *wsc = tb + (size_t)rows * nb * 16 + (size_t)r0 * nb * 2;
+    // chunk ch of the rows: load i takes rows 8i .. 8i+7, lane l row l / 8,
+    // piece l % 8.  Chunks past the last are out of the buffer's range: such a
+    // load moves nothing, and every step issues the same number of loads, so
+    // the waits stay exact
+    const auto wrs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(tb + (size_t)r0 * nb * 16), 0, 32 * nb * 16,
+                                                       0x00020000);
+    const uint32_t wof = (uint32_t)((lane >> 3) * nb * 16 + (lane & 7) * 16);
+    auto wload = [&](int ch, v4i (&w)[4]) {
+        const uint32_t v = ch < nch ? wof + (uint32_t)ch * 128 : 0x40000000u;
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            w[i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wrs, (int)v, i * 8 * nb * 16, 0));
+    };
+    // the rows' scales of chunks 4g .. 4g+3 (past the last chunk: its again)
+    auto stage_ws = [&](int g) {
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const int r = j * 16 + (lane >> 2), p = (lane & 3) ^ ((r >> 1) & 3);
+            lds_dma16(wsc + (size_t)r * nb * 2 + min(4 * g + p, nch - 1) * 16,
+                      lds_addr(smem, MsLds::WS + wave * 4096 + (g & 1) * 2048 + j * 1024));
+        }
+    };
 
-    // (FULL) every chunk's activations and activation scales straight into
-    // LDS, issued before any weight load: the waits of the weight loop then
-    // count weight loads only.  Entries past the item stage the item's last
-    // entry's bytes (their sums are never stored).
-    // GD down block: every gate/up block of the item has counted in
-    // (bounded; when the wait runs out the rows are stored as NaN and *err set)
+    // The item's entries are looked up first and the first weights requested
+    // while they arrive; a down block requests PF chunks before it waits.
+    int ea[JA];
+#pragma unroll
+    for (int j = 0; j < JA; j++) ea[j] = entries[o + min(((j * NW + wave) * 64 + lane) >> 4, c - 1)];
+    const int ed = entries[o + min((wave * 64 + lane) % M, c - 1)];
+    __builtin_amdgcn_sched_barrier(0);
+    v4i w[PF][4];
     bool gd_bad = false;
+    stage_ws(0);
+    wload(0, w[0]);
     if constexpr (GD && !PAIR) {
+        if (nch > 4) stage_ws(1);
+#pragma unroll
+        for (int u = 1; u < PF; u++) wload(u, w[u]);
+        __builtin_amdgcn_sched_barrier(0);
+        // every gate/up block of the item has counted in (bounded; when the
+        // wait runs out the rows are stored as NaN and *err set)
         __shared__ int gd_flag;
         if (tid == 0) {
             uint32_t tries = 0;
@@ -573,219 +584,133 @@ TG_DEV __attribute__((always_inline)) void ms_item(const uint8_t *__restrict__ l
             gd_flag = bad;
             if (bad) __hip_atomic_store(G.err, 4u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
-        __syncthreads();
+        lds_barrier();  // the weight loads stay in flight
         gd_bad = gd_flag != 0;
     }
-
-    constexpr int FA = M * 256, FD = MF_KC * M;  // bytes of one chunk's rows, scales of one chunk
-    if constexpr (FULL) {
-        constexpr int JA = M * 256 / (NT * 16), JD = FD / NT;  // DMA rounds per chunk: rows, scales
-        static_assert(JA * NT * 16 == M * 256 && JD * NT == FD, "staging map");
-        // this lane's entries (looked up once): its row slots' and its scale slots'
-        const int8_t *asrc[JA];
-        const float *dsrc[JD];
+    // the activations and activation scales of chunks 2q, 2q+1 into slots
+    // ch % 4.  Groups of 4 rows without an entry of the item are left out
+    // (their sums are never stored).
+    const int8_t *asrc[JA];
 #pragma unroll
-        for (int j = 0; j < JA; j++) {
-            const int L = (j * NW + wave) * 64 + lane;  // 16-byte slot of a chunk's rows
-            const int t = L >> 4, pc = ((L & 15) - t) & 15;
-            const int et = entries[o + min(t, c - 1)];
-            asrc[j] = aq + (size_t)(PAIR ? et / k : et) * K + pc * 16;
-        }
+    for (int j = 0; j < JA; j++) {
+        const int L = (j * NW + wave) * 64 + lane;  // 16-byte slot of a chunk's rows
+        const int t = L >> 4, pc = ((L & 15) - t) & 15;
+        asrc[j] = aq + (size_t)(PAIR ? ea[j] / k : ea[j]) * K + pc * 16;
+    }
+    const float *dsrc = ad + (size_t)(PAIR ? ed / k : ed) * nb + (wave * 64 + lane) / M;
+    auto stage_act = [&](int q) {
 #pragma unroll
-        for (int j = 0; j < JD; j++) {
-            const int L = (j * NW + wave) * 64 + lane;  // scale slot: block L / M, entry L % M
-            const int et = entries[o + min(L % M, c - 1)];
-            dsrc[j] = ad + (size_t)(PAIR ? et / k : et) * nb + L / M;
-        }
-#pragma unroll
-        for (int ch = 0; ch < MS_FC; ch++) {
+        for (int cc = 0; cc < 2; cc++) {
+            const int ch = 2 * q + cc;
             if (ch < nch) {  // uniform
 #pragma unroll
                 for (int j = 0; j < JA; j++) {
-                    const uint32_t m0 = lds_addr(smem, ch * FA + (j * NW + wave) * 1024);
-                    if constexpr (GD && !PAIR)
-                        lds_dma16_coh(asrc[j] + ch * MF_KC * 32, m0);
-                    else
-                        lds_dma16(asrc[j] + ch * MF_KC * 32, m0);
+                    if (4 * (j * NW + wave) < c) {  // uniform
+                        const uint32_t m0 = lds_addr(smem, MsLds::ACT + (ch & 3) * FA + (j * NW + wave) * 1024);
+                        if constexpr (GD && !PAIR)
+                            lds_dma16_coh(asrc[j] + ch * MF_KC * 32, m0);
+                        else
+                            lds_dma16(asrc[j] + ch * MF_KC * 32, m0);
+                    }
                 }
-#pragma unroll
-                for (int j = 0; j < JD; j++) {
-                    const uint32_t m0 = lds_addr(smem, MS_FC * FA + (ch * FD + (j * NW + wave) * 64) * 4);
-                    if constexpr (GD && !PAIR)
-                        lds_dma4_coh(dsrc[j] + ch * MF_KC, m0);
-                    else
-                        lds_dma4(dsrc[j] + ch * MF_KC, m0);
-                }
+                const uint32_t m0 = lds_addr(smem, MsLds::DX + (ch & 3) * FD + wave * 256);
+                if constexpr (GD && !PAIR)
+                    lds_dma4_coh(dsrc + ch * MF_KC, m0);
+                else
+                    lds_dma4(dsrc + ch * MF_KC, m0);
             }
         }
-    }
-
-    // activation staging: unconditional loads from clamped, in-bounds
-    // addresses (entries past the item and blocks past K select zero when
-    // committed), so the waits before the commit count exactly the loads
-    // issued after them and leave the weight loads in flight
-    uint4 sv[NTP];
-    float sd[NDX];
-    auto stage = [&](int ch) {
-#pragma unroll
-        for (int u = 0; u < NTP; u++) {
-            const int kb = min(ch * MF_KC * 32 + sp * 16, K - 16);
-            sv[u] = *reinterpret_cast<const uint4 *>(aq + max(toff[u], 0) + kb);
-        }
-#pragma unroll
-        for (int u = 0; u < NDX; u++) sd[u] = ad[max(doff[u], 0) + min(ch * MF_KC + sb, nb - 1)];
     };
-    auto commit = [&](int q, int ch) {
-#pragma unroll
-        for (int u = 0; u < NTP; u++) {
-            const int t = tid / TP + u * (NT / TP);
-            const bool ok = toff[u] >= 0 && ch * MF_KC * 32 + sp * 16 < K;
-            *reinterpret_cast<uint4 *>(tokl + ((size_t)q * M + t) * MF_TS + sp * 16) =
-                ok ? sv[u] : make_uint4(0u, 0u, 0u, 0u);
-        }
-#pragma unroll
-        for (int u = 0; u < NDX; u++) {
-            const int t = tid / MF_KC + u * (NT / MF_KC);
-            const bool ok = doff[u] >= 0 && ch * MF_KC + sb < nb;
-            dxl[(q * MF_KC + sb) * M + t] = ok ? sd[u] * 0.0625f : 0.0f;  // dx / 16, exact
-        }
-    };
-    // row R's weights of chunk ch: blocks 8ch + 4h + i (clamped; blocks past
-    // nb are never used) and the chunk's 8 scales (packed halves); chunks
-    // past the last load the last one again (unconditional loads keep the
-    // waits exact)
-    auto wload = [&](int ch, uint4 (&w)[4], uint4 &sc) {
-#pragma unroll
-        for (int i = 0; i < 4; i++) w[i] = q0[min(ch * MF_KC + 4 * h + i, nb - 1)];
-        if (SCV) {
-            sc = *reinterpret_cast<const uint4 *>(s0 + min(ch, nch - 1) * MF_KC);
-        } else {
-            uint32_t hv[MF_KC];
-#pragma unroll
-            for (int j = 0; j < MF_KC; j++) hv[j] = s0[min(ch * MF_KC + j, nb - 1)];
-            sc = make_uint4(hv[0] | hv[1] << 16, hv[2] | hv[3] << 16, hv[4] | hv[5] << 16, hv[6] | hv[7] << 16);
-        }
-    };
-
-    float acc[16];
-#pragma unroll
-    for (int r = 0; r < 16; r++) acc[r] = 0.0f;
-
-    // weights run PF chunks ahead in PF + 1 register sets, each with a
-    // fixed role per unrolled step (a copy between sets would wait for the
-    // loads in flight); the activations one chunk ahead, issued before the
-    // newer weight loads so the wait before their commit leaves those in
-    // flight
-    // (gate / up with 16-byte scale loads: three chunks ahead in four sets,
-    // still two waves per SIMD; otherwise two ahead in three: the down
-    // launch measured slower with three, 80.5 -> 94.9 us at H 4096, I 1536)
-    constexpr int PF = PAIR && SCV ? MS_PF + 1 : MS_PF;
-    static_assert(MS_PF == 2, "three or four register sets");
-    uint4 wa[4], sa, wb[4], sbv, wcx[4], scx, wdx[4], sdx;
-    wload(0, wa, sa);
-    if constexpr (!FULL) stage(0);
-    wload(1, wb, sbv);
-    if constexpr (PF == 3) wload(2, wcx, scx);
-    if constexpr (FULL) {
-        // this wave's staging landed (it was issued before the 5 PF weight
-        // loads in flight); the barrier below makes every wave's visible
-        __builtin_amdgcn_s_waitcnt(VMCNT0 | (5 * PF));
+    stage_act(0);
+    stage_act(1);
+    if constexpr (GD && !PAIR) {
+        __builtin_amdgcn_s_waitcnt(VMCNT0);
     } else {
-        commit(0, 0);
+        if (nch > 4) stage_ws(1);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 1; u < PF; u++) wload(u, w[u]);
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt(VMCNT0 | (4 * (PF - 1)));  // everything staged before them landed
     }
     const v16i czero = {};  // the accumulator operand: an inline 0, no registers
     const int nsh = h ? 0 : 4;  // this half's nibble to the high half of each byte
     __syncthreads();
 
+    float acc[16];
+#pragma unroll
+    for (int r = 0; r < 16; r++) acc[r] = 0.0f;
+    uint8_t *wb = smem + MsLds::WB + wave * 4096;
+    uint8_t *wb_put = wb + (lane >> 3) * 128 + (((lane & 7) ^ (lane >> 3)) << 4);
+    const uint8_t *wb_row = wb + n * 128, *ws_row = smem + MsLds::WS + wave * 4096 + n * 64;
+
     // register groups holding entries of the item (8 entries per group)
     auto run = [&](auto ngc) {
         constexpr int NG = decltype(ngc)::value;
-        // chunk ch from set w (scales sc); chunk ch + PF loads into set wl
-        auto step = [&](int ch, uint4 (&w)[4], const uint4 &sc, uint4 (&wl)[4], uint4 &sl) {
-            const int q = ch & 1;
-            if constexpr (!FULL) {
-                stage(ch + 1);
-                __builtin_amdgcn_sched_barrier(0);  // activations issued before the weights
-            }
-            wload(ch + PF, wl, sl);
+        // chunk ch from set wl, which then takes chunk ch + PF
+        auto step = [&](int ch, v4i (&wl)[4]) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) *reinterpret_cast<v4i *>(wb_put + i * 1024) = wl[i];
+            __builtin_amdgcn_sched_barrier(0);
+            wload(ch + PF, wl);
+            __builtin_amdgcn_sched_barrier(0);
+            wave_lds_sync();
             if (ch < nch) {  // uniform
-                const uint8_t *tq = FULL ? smem + ch * FA + n * 256
-                                         : tokl + (size_t)q * M * MF_TS + (size_t)n * MF_TS + 16 * h;
-                const float *xq = FULL ? reinterpret_cast<const float *>(smem + MS_FC * FA) + ch * FD + 4 * h
-                                       : dxl + q * MF_KC * M + 4 * h;
+                const uint4 sc =
+                    *reinterpret_cast<const uint4 *>(ws_row + ((ch >> 2) & 1) * 2048 + (((ch & 3) ^ ((n >> 1) & 3)) << 4));
                 const uint32_t scw[4] = {sc.x, sc.y, sc.z, sc.w};
+                const uint8_t *tq = smem + MsLds::ACT + (ch & 3) * FA + n * 256;
+                const float *xq = reinterpret_cast<const float *>(smem + MsLds::DX + (ch & 3) * FD) + 4 * h;
 #pragma unroll
                 for (int bl = 0; bl < MF_KC; bl++) {
-                    const int b = ch * MF_KC + bl;
-                    // SCV: nb % MF_KC == 0, so every block of a chunk below nch
-                    // exists; without the test the chunk is one basic block and
-                    // the scheduler overlaps one block's epilogue with the next
-                    // block's swaps and MFMA (the guard cost 16 register moves
-                    // per chunk and 2-3 us of gate/up)
-                    if (SCV || b < nb) {
-                        // block bl sits in w[bl % 4] of the half bl / 4 lane: the swap
-                        // at bl < 4 yields block bl and keeps block bl + 4 in w[bl]
-                        uint4 blk;
-                        if (bl < 4) {
-                            uint4 &wr = w[bl];
-                            half_split(wr.x, blk.x, wr.x);
-                            half_split(wr.y, blk.y, wr.y);
-                            half_split(wr.z, blk.z, wr.z);
-                            half_split(wr.w, blk.w, wr.w);
-                        } else {
-                            blk = w[bl & 3];
-                        }
-                        // 16 (q - 8) per byte: ((q << 4) & 0xF0) ^ 0x80, exact in int8
-                        v4i wq;
-                        wq.x = (int)(((blk.x << nsh) & 0xF0F0F0F0u) ^ 0x80808080u);
-                        wq.y = (int)(((blk.y << nsh) & 0xF0F0F0F0u) ^ 0x80808080u);
-                        wq.z = (int)(((blk.z << nsh) & 0xF0F0F0F0u) ^ 0x80808080u);
-                        wq.w = (int)(((blk.w << nsh) & 0xF0F0F0F0u) ^ 0x80808080u);
-                        const v4i ta = FULL ? *reinterpret_cast<const v4i *>(tq + (((2 * bl + h + n) & 15) << 4))
-                                            : *reinterpret_cast<const v4i *>(tq + bl * 32);
-                        // (FULL: the staged scales are dx itself, so the 1/16 goes with dw;
-                        // both are exact: powers of two)
-                        const float dw = FULL ? h2f((uint16_t)(scw[bl >> 1] >> (16 * (bl & 1)))) * 0.0625f
-                                              : h2f((uint16_t)(scw[bl >> 1] >> (16 * (bl & 1))));
-                        float4 dx[NG];
+                    const uint4 blk = *reinterpret_cast<const uint4 *>(wb_row + ((bl ^ (n & 7)) << 4));
+                    // 16 (q - 8) per byte: ((q << 4) & 0xF0) ^ 0x80, exact in int8
+                    v4i wq;
+                    wq.x = (int)(((blk.x << nsh) & 0xF0F0F0F0u) ^ 0x80808080u);
+                    wq.y = (int)(((blk.y << nsh) & 0xF0F0F0F0u) ^ 0x80808080u);
+                    wq.z = (int)(((blk.z << nsh) & 0xF0F0F0F0u) ^ 0x80808080u);
+                    wq.w = (int)(((blk.w << nsh) & 0xF0F0F0F0u) ^ 0x80808080u);
+                    const v4i ta = *reinterpret_cast<const v4i *>(tq + (((2 * bl + h + n) & 15) << 4));
+                    const float dw = h2f((uint16_t)(scw[bl >> 1] >> (16 * (bl & 1)))) * 0.0625f;
+                    float4 dx[NG];
 #pragma unroll
-                        for (int g = 0; g < NG; g++) dx[g] = *reinterpret_cast<const float4 *>(xq + bl * M + 8 * g);
-                        // rc = 16 S exactly (|16 S| < 2^24): u16 = round(16 S * dw) =
-                        // 16 round(S * dw), and u16 * (dx / 16) = round(S * dw) * dx
-                        const v16i rc = __builtin_amdgcn_mfma_i32_32x32x32_i8(ta, wq, czero, 0, 0, 0);
+                    for (int g = 0; g < NG; g++) dx[g] = *reinterpret_cast<const float4 *>(xq + bl * M + 8 * g);
+                    // rc = 16 S exactly (|16 S| < 2^24)
+                    const v16i rc = __builtin_amdgcn_mfma_i32_32x32x32_i8(ta, wq, czero, 0, 0, 0);
 #pragma unroll
-                        for (int g = 0; g < NG; g++) {
-                            const float dxa[4] = {dx[g].x, dx[g].y, dx[g].z, dx[g].w};
+                    for (int g = 0; g < NG; g++) {
+                        const float dxa[4] = {dx[g].x, dx[g].y, dx[g].z, dx[g].w};
 #pragma unroll
-                            for (int rr = 0; rr < 4; rr++) {
-                                const int r = 4 * g + rr;
-                                const float u16 = (float)rc[r] * dw;
-                                acc[r] = __builtin_fmaf(u16, dxa[rr], acc[r]);
-                            }
+                        for (int rr = 0; rr < 4; rr++) {
+                            const int r = 4 * g + rr;
+                            const float u = (float)rc[r] * dw;
+                            acc[r] = __builtin_fmaf(u, dxa[rr], acc[r]);
                         }
                     }
                 }
-            }
-            // unconditional (zeros past the last chunk), so the activation
-            // loads stay ahead of the weight loads
-            if constexpr (!FULL) {
-                commit(q ^ 1, ch + 1);
-                __syncthreads();
+                // the sums formed here (sunk past the branches below, they would
+                // keep every block's MFMA result live and spill)
+#pragma unroll
+                for (int r = 0; r < 4 * NG; r++) asm volatile("" : "+v"(acc[r]));
+                wave_lds_sync();
+                // the pair's last chunk, more to come than the slots hold: the next
+                // pair's staging (issued one pair ago, before two steps' weight
+                // loads) landed on every wave, and this pair's slots take the one
+                // after it
+                if (nch > 4 && (ch & 1) && ch + 1 < nch) {
+                    __builtin_amdgcn_s_waitcnt(VMCNT0 | 8);
+                    if ((ch & 3) == 3 && ch + 5 < nch) stage_ws((ch >> 2) + 2);
+                    lds_barrier();
+                    if (ch + 3 < nch) stage_act((ch >> 1) + 2);
+                }
             }
         };
-        if constexpr (PF == 3) {
-            for (int ch = 0; ch < nch; ch += 4) {
-                step(ch, wa, sa, wdx, sdx);
-                step(ch + 1, wb, sbv, wa, sa);
-                step(ch + 2, wcx, scx, wb, sbv);
-                step(ch + 3, wdx, sdx, wcx, scx);
-            }
-        } else {
-            for (int ch = 0; ch < nch; ch += 3) {
-                step(ch, wa, sa, wcx, scx);
-                step(ch + 1, wb, sbv, wa, sa);
-                step(ch + 2, wcx, scx, wb, sbv);
-            }
+        static_assert(PF >= 2 && PF <= 4, "steps written out");
+        for (int ch = 0; ch < nch; ch += PF) {
+            step(ch, w[0]);
+            step(ch + 1, w[1]);
+            if constexpr (PF > 2) step(ch + 2, w[2]);
+            if constexpr (PF > 3) step(ch + 3, w[3]);
         }
     };
     const int ng = (c + 7) >> 3;
@@ -801,7 +726,7 @@ TG_DEV __attribute__((always_inline)) void ms_item(const uint8_t *__restrict__ l
         // its sums of the other half.  Register groups past the item's
         // entries are skipped (uniform).
         float *x = reinterpret_cast<float *>(smem) + (size_t)(wave >> 1) * 16 * 64;
-        if constexpr (FULL) __syncthreads();  // every wave is done with the staged activations
+        __syncthreads();  // every wave is done with the staged activations
 #pragma unroll
         for (int r = 0; r < 16; r++) {
             const bool give = r < 4 * ng && (mat == 0) == ((r & 2) != 0);  // uniform
@@ -868,42 +793,44 @@ TG_DEV __attribute__((always_inline)) void ms_item(const uint8_t *__restrict__ l
     }
 }
 
-template <bool PAIR, bool SCV, bool FULL>
-__global__ __launch_bounds__(MS_NW * 64) void k_mfma_small(const uint8_t *__restrict__ layer_pl, Shape s,
-                                                           const int32_t *__restrict__ work,
-                                                           const int32_t *__restrict__ work_n,
-                                                           const int32_t *__restrict__ entries,
-                                                           const int8_t *__restrict__ aq, const float *__restrict__ ad,
-                                                           int8_t *__restrict__ oq, float *__restrict__ od,
-                                                           int *__restrict__ os, float *__restrict__ D, FuseArgs F) {
-    ms_item<PAIR, SCV, FULL, false>(layer_pl, s, work, work_n, entries, aq, ad, oq, od, os, D, F, (int)blockIdx.y,
-                                    (int)blockIdx.x, GdArgs());
-}
-
-// Gate/up and down of the one-tile items in one launch: blocks [0, gxg wmax)
-// are the gate/up blocks (item b / gxg, row tile b % gxg), the rest the down
-// blocks.  Blocks are dispatched in order of their id on each XCD, so every
-// gate/up block has been dispatched (and runs without waiting) before a down
-// block of the same XCD takes a slot; a down block's wait ends once the
-// gate/up blocks of its item, on whichever XCD, have stored h.  The down
-// blocks then fill the slots the gate/up launch's last round leaves idle.
-template <bool SCVG, bool FULLG>
-__global__ __launch_bounds__(MS_NW * 64) void k_mfma_small_gd(const uint8_t *__restrict__ layer_pl, Shape s,
+template <bool PAIR>
+__global__ __launch_bounds__(MS_NW * 64, 2) void k_mfma_small(const uint8_t *__restrict__ layer_pl, Shape s,
                                                               const int32_t *__restrict__ work,
                                                               const int32_t *__restrict__ work_n,
                                                               const int32_t *__restrict__ entries,
-                                                              const int8_t *__restrict__ xq,
-                                                              const float *__restrict__ xd, int8_t *hq, float *hd,
-                                                              int *hs, float *__restrict__ D, GdArgs G, int gxg,
-                                                              int gxd, int wmax) {
-    const int b = (int)blockIdx.x, ng = gxg * wmax;
+                                                              const int8_t *__restrict__ aq,
+                                                              const float *__restrict__ ad, int8_t *__restrict__ oq,
+                                                              float *__restrict__ od, int *__restrict__ os,
+                                                              float *__restrict__ D, FuseArgs F) {
+    if ((int)blockIdx.y >= work_n[0]) return;  // uniform over the block
+    ms_item<PAIR, false>(layer_pl, s, work, entries, aq, ad, oq, od, os, D, F, (int)blockIdx.y, (int)blockIdx.x,
+                         GdArgs());
+}
+
+// Gate/up and down of the one-tile items in one launch: with n items (work_n,
+// at most the grid's) blocks [0, gxg n) are the gate/up blocks (item b / gxg, row
+// tile b % gxg), [gxg n, (gxg + gxd) n) the down blocks, and the rest have no
+// item: they come last, so none holds a slot that work waits for.  Blocks are
+// dispatched in order of their id on each XCD, so every gate/up block has been
+// dispatched (and runs without waiting) before a down block of the same XCD
+// takes a slot; a down block's wait ends once the gate/up blocks of its item, on
+// whichever XCD, have stored h.  The down blocks then fill the slots the
+// gate/up launch's last round leaves idle.
+__global__ __launch_bounds__(MS_NW * 64, 2) void k_mfma_small_gd(const uint8_t *__restrict__ layer_pl, Shape s,
+                                                                 const int32_t *__restrict__ work,
+                                                                 const int32_t *__restrict__ work_n,
+                                                                 const int32_t *__restrict__ entries,
+                                                                 const int8_t *__restrict__ xq,
+                                                                 const float *__restrict__ xd, int8_t *hq, float *hd,
+                                                                 int *hs, float *__restrict__ D, GdArgs G, int gxg,
+                                                                 int gxd) {
+    const int b = (int)blockIdx.x, n = work_n[0], ng = gxg * n;
     if (b < ng) {
-        ms_item<true, SCVG, FULLG, true>(layer_pl, s, work, work_n, entries, xq, xd, hq, hd, hs, nullptr, FuseArgs(),
-                                         b / gxg, b % gxg, G);
-    } else {
+        ms_item<true, true>(layer_pl, s, work, entries, xq, xd, hq, hd, hs, nullptr, FuseArgs(), b / gxg, b % gxg, G);
+    } else if (b < ng + gxd * n) {
         const int d = b - ng;
-        ms_item<false, true, true, true>(layer_pl, s, work, work_n, entries, hq, hd, nullptr, nullptr, nullptr, D,
-                                         FuseArgs(), d / gxd, d % gxd, G);
+        ms_item<false, true>(layer_pl, s, work, entries, hq, hd, nullptr, nullptr, nullptr, D, FuseArgs(), d / gxd,
+                             d % gxd, G);
     }
 }
 
@@ -981,7 +908,6 @@ TG_DEV long xt_unpack(uint2 w, int sh) {
 template <bool PAIR, bool GD>
 TG_DEV __attribute__((always_inline)) void x16_item(const uint8_t *__restrict__ layer_pl, const Shape s,
                                                     const int32_t *__restrict__ work,
-                                                    const int32_t *__restrict__ work_n,
                                                     const int32_t *__restrict__ entries,
                                                     const int8_t *__restrict__ aq, const float *__restrict__ ad,
                                                     int8_t *__restrict__ oq, float *__restrict__ od,
@@ -994,7 +920,6 @@ TG_DEV __attribute__((always_inline)) void x16_item(const uint8_t *__restrict__ 
     constexpr int NACT = ROWS * XT_NP / 64;          // activation load instructions per chunk (full item)
     constexpr int NAXS = XT_KC * 16 * XT_CS / 64;    // activation-scale load instructions per chunk
     static_assert(NACT % NW == 0 && NAXS % NW == 0, "staging split");
-    if (wi >= work_n[0]) return;  // uniform over the block
     const int e = work[3 * wi], o = work[3 * wi + 1], c = work[3 * wi + 2];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, g = lane >> 4, cl = lane & 15;
     const int K = PAIR ? s.H : s.I, nb = K / QK, k = s.k;
@@ -1366,30 +1291,34 @@ __global__ __launch_bounds__(XT_NW * 64) void k_mfma16(const uint8_t *__restrict
     const int gx = PAIR ? s.I / (32 * (XT_NW / 2)) : s.H / (32 * XT_NW);
     int wi, bx;
     x16_place((int)blockIdx.x, gx, wi, bx);
-    x16_item<PAIR, false>(layer_pl, s, work, work_n, entries, aq, ad, oq, od, os, D, F, wi, bx, GdArgs());
+    if (wi >= work_n[0]) return;  // uniform over the block
+    x16_item<PAIR, false>(layer_pl, s, work, entries, aq, ad, oq, od, os, D, F, wi, bx, GdArgs());
 }
 
-// Gate/up and down of the 16 x 16 items in one launch: blocks [0, gxg wm8)
-// are the gate/up blocks, the rest the down blocks (each part placed as in
-// k_mfma16).  Blocks are dispatched in id order on each XCD and gate/up
-// blocks never wait, so the down blocks' waits end (as in k_mfma_small_gd);
-// the down blocks of the items done first fill the gate/up launch's tail.
+// Gate/up and down of the 16 x 16 items in one launch: with n8 = the item
+// count rounded up to 8, blocks [0, gxg n8) are the gate/up blocks, the next
+// gxd n8 the down blocks (each part placed as in k_mfma16), and the rest have no
+// item.  Blocks are dispatched in id order on each XCD and gate/up blocks never
+// wait, so the down blocks' waits end (as in k_mfma_small_gd); the down blocks
+// of the items done first fill the gate/up launch's tail.
 __global__ __launch_bounds__(XT_NW * 64) void k_mfma16_gd(const uint8_t *__restrict__ layer_pl, Shape s,
                                                           const int32_t *__restrict__ work,
                                                           const int32_t *__restrict__ work_n,
                                                           const int32_t *__restrict__ entries,
                                                           const int8_t *__restrict__ xq, const float *__restrict__ xd,
                                                           int8_t *hq, float *hd, int *hs, float *__restrict__ D,
-                                                          GdArgs G, int gxg, int gxd, int wm8) {
-    const int b = (int)blockIdx.x, ng = gxg * wm8;
+                                                          GdArgs G, int gxg, int gxd) {
+    const int b = (int)blockIdx.x, n = work_n[0], n8 = (n + 7) & ~7, ng = gxg * n8;
     int wi, bx;
     if (b < ng) {
         x16_place(b, gxg, wi, bx);
-        x16_item<true, true>(layer_pl, s, work, work_n, entries, xq, xd, hq, hd, hs, nullptr, FuseArgs(), wi, bx, G);
+        if (wi < n)
+            x16_item<true, true>(layer_pl, s, work, entries, xq, xd, hq, hd, hs, nullptr, FuseArgs(), wi, bx, G);
     } else {
         x16_place(b - ng, gxd, wi, bx);
-        x16_item<false, true>(layer_pl, s, work, work_n, entries, hq, hd, nullptr, nullptr, nullptr, D, FuseArgs(),
-                              wi, bx, G);
+        if (wi < n)
+            x16_item<false, true>(layer_pl, s, work, entries, hq, hd, nullptr, nullptr, nullptr, D, FuseArgs(), wi,
+                                  bx, G);
     }
 }
 
@@ -1465,7 +1394,7 @@ int mfma_item_entries(const Shape &s, int mt) {
 // 235B) only take shapes that these do not.
 int mfma_tiles(const Shape &s, int T) {
     const int avg = (T * s.k + s.E - 1) / s.E;
-    if (mfma_item_entries(s, 4) > 128 && s.nbI % MF_KC == 0 && s.nbI <= MS_FC * MF_KC) return avg > 24 ? 4 : 1;
+    if (mfma_item_entries(s, 4) > 128 && s.nbI % MF_KC == 0) return avg > 24 ? 4 : 1;
     return avg > 64 ? 4 : (avg > 16 ? 2 : 1);
 }
 
@@ -1497,29 +1426,17 @@ static hipError_t ms_go(const uint8_t *layer_pl, const Shape &s, int wmax, const
                         float *D, const FuseArgs &F, hipStream_t st) {
     static_assert(MS_NW * 32 == FC_ROWS && XT_NW * 32 == FC_ROWS, "one down block per output tile");
     const int rows = PAIR ? s.I : s.H, nb = (PAIR ? s.H : s.I) / QK;
-    const unsigned gx = PAIR ? mf_cdiv((size_t)rows, 32 * (MS_NW / 2)) : mf_cdiv((size_t)rows, 32 * MS_NW);
-    // whole chunks, at most MS_FC of them: the activations staged once (TG_MS_FULL=0: per chunk)
-    static const bool full_on = [] {
-        const char *v = getenv("TG_MS_FULL");
-        return !(v && v[0] == '0');
-    }();
-    if (full_on && nb % MF_KC == 0 && nb <= MS_FC * MF_KC) {
-        const size_t lds = ms_full_lds_bytes();
-        static std::atomic<uint64_t> attr{0};
-        hipError_t e = lds_attr(reinterpret_cast<const void *>(&k_mfma_small<PAIR, true, true>), lds, attr);
-        if (e != hipSuccess) return e;
-        TG_LAUNCH((k_mfma_small<PAIR, true, true>), dim3(gx, wmax), dim3(MS_NW * 64), lds, st, layer_pl, s, work,
-                  work_n, entries, aq, ad, oq, od, os, D, F);
-        return hipGetLastError();
+    // whole chunks of K (the row scales are staged in 16-byte pieces); other shapes take the 32 x 32 kernel's one tile
+    if (nb % MF_KC != 0) {
+        if (F.cnt) return hipErrorInvalidValue;
+        return mf_go<1, PAIR>(layer_pl, s, wmax, work, work_n, entries, aq, ad, oq, od, os, D, st);
     }
-    const size_t lds = ms_lds_bytes();
-    // 16-byte scale loads need every row's scales 16-byte aligned (nb % 8 == 0)
-    if (nb % MF_KC == 0)
-        TG_LAUNCH((k_mfma_small<PAIR, true, false>), dim3(gx, wmax), dim3(MS_NW * 64), lds, st, layer_pl, s, work,
-                           work_n, entries, aq, ad, oq, od, os, D, F);
-    else
-        TG_LAUNCH((k_mfma_small<PAIR, false, false>), dim3(gx, wmax), dim3(MS_NW * 64), lds, st, layer_pl, s, work,
-                           work_n, entries, aq, ad, oq, od, os, D, F);
+    const unsigned gx = PAIR ? mf_cdiv((size_t)rows, 32 * (MS_NW / 2)) : mf_cdiv((size_t)rows, 32 * MS_NW);
+    static std::atomic<uint64_t> attr{0};
+    hipError_t e = lds_attr(reinterpret_cast<const void *>(&k_mfma_small<PAIR>), MsLds::BYTES, attr);
+    if (e != hipSuccess) return e;
+    TG_LAUNCH((k_mfma_small<PAIR>), dim3(gx, wmax), dim3(MS_NW * 64), MsLds::BYTES, st, layer_pl, s, work, work_n,
+              entries, aq, ad, oq, od, os, D, F);
     return hipGetLastError();
 }
 
@@ -1569,7 +1486,7 @@ hipError_t launch_gateup_mfma(const uint8_t *layer_pl, const Shape &s, int mt, i
 bool down_fuses(const Shape &s, int mt, int T) {
     const char *v = getenv("TG_FUSE_COMBINE");
     const bool on = v && v[0] == '1';
-    const bool kern = mt == 1 || (mt == 4 && mfma_item_entries(s, mt) > 128);
+    const bool kern = (mt == 1 && s.nbI % MF_KC == 0) || (mt == 4 && mfma_item_entries(s, mt) > 128);
     return on && kern && s.H % FC_ROWS == 0 && (size_t)T * s.k * s.H < ((size_t)1 << 31);
 }
 
@@ -1592,7 +1509,7 @@ hipError_t launch_down_mfma(const uint8_t *layer_pl, const Shape &s, int mt, int
 bool gd_fuses(const Shape &s, int mt) {
     const char *v = getenv("TG_FUSE_GD");
     const bool on = !(v && v[0] == '0');
-    return on && mt == 1 && mfma_shape_ok(s) && s.nbI % MF_KC == 0 && s.nbI <= MS_FC * MF_KC;
+    return on && mt == 1 && mfma_shape_ok(s) && s.nbH % MF_KC == 0 && s.nbI % MF_KC == 0;
 }
 
 bool gd16_fuses(const Shape &s, int mt) {
@@ -1614,20 +1531,7 @@ hipError_t launch_gu_down_x16(const uint8_t *layer_pl, const Shape &s, int wmax,
     hipError_t e = lds_attr(reinterpret_cast<const void *>(&k_mfma16_gd), XtLds::BYTES, attr);
     if (e != hipSuccess) return e;
     TG_LAUNCH(k_mfma16_gd, dim3((unsigned)((gxg + gxd) * wm8)), dim3(XT_NW * 64), XtLds::BYTES, st, layer_pl, s,
-              work, work_n, entries, xq, xd, hq, hd, hs, D, G, gxg, gxd, wm8);
-    return hipGetLastError();
-}
-
-template <bool SCVG, bool FULLG>
-static hipError_t gd_go(const uint8_t *layer_pl, const Shape &s, int wmax, const int32_t *work,
-                        const int32_t *work_n, const int32_t *entries, const int8_t *xq, const float *xd, int8_t *hq,
-                        float *hd, int *hs, float *D, const GdArgs &G, int gxg, int gxd, hipStream_t st) {
-    const size_t lds = ms_full_lds_bytes();
-    static std::atomic<uint64_t> attr{0};
-    hipError_t e = lds_attr(reinterpret_cast<const void *>(&k_mfma_small_gd<SCVG, FULLG>), lds, attr);
-    if (e != hipSuccess) return e;
-    TG_LAUNCH((k_mfma_small_gd<SCVG, FULLG>), dim3((unsigned)((gxg + gxd) * wmax)), dim3(MS_NW * 64), lds, st,
-              layer_pl, s, work, work_n, entries, xq, xd, hq, hd, hs, D, G, gxg, gxd, wmax);
+              work, work_n, entries, xq, xd, hq, hd, hs, D, G, gxg, gxd);
     return hipGetLastError();
 }
 
@@ -1639,12 +1543,12 @@ hipError_t launch_gu_down_ms(const uint8_t *layer_pl, const Shape &s, int wmax, 
     if ((size_t)(gxg + gxd) * (size_t)wmax >= ((size_t)1 << 31)) return hipErrorInvalidValue;
     GdArgs G = G0;
     G.need = gxg;
-    const int nbH = s.nbH;
-    if (nbH % MF_KC == 0 && nbH <= MS_FC * MF_KC)
-        return gd_go<true, true>(layer_pl, s, wmax, work, work_n, entries, xq, xd, hq, hd, hs, D, G, gxg, gxd, st);
-    if (nbH % MF_KC == 0)
-        return gd_go<true, false>(layer_pl, s, wmax, work, work_n, entries, xq, xd, hq, hd, hs, D, G, gxg, gxd, st);
-    return gd_go<false, false>(layer_pl, s, wmax, work, work_n, entries, xq, xd, hq, hd, hs, D, G, gxg, gxd, st);
+    static std::atomic<uint64_t> attr{0};
+    hipError_t e = lds_attr(reinterpret_cast<const void *>(&k_mfma_small_gd), MsLds::BYTES, attr);
+    if (e != hipSuccess) return e;
+    TG_LAUNCH(k_mfma_small_gd, dim3((unsigned)((gxg + gxd) * wmax)), dim3(MS_NW * 64), MsLds::BYTES, st, layer_pl, s,
+              work, work_n, entries, xq, xd, hq, hd, hs, D, G, gxg, gxd);
+    return hipGetLastError();
 }
 
 }  // namespace tg

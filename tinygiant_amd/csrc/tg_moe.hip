@@ -3046,7 +3046,9 @@ hipError_t launch_route_chains(const float *Wr, const float *x, int T, int E, in
 int group_chunk_gateup(const Shape &s) { return gu_chunk(s.nbH); }
 int group_chunk_down(const Shape &s) { return dn_chunk(s.nbI, s.I); }
 
-int group_work_max(const Shape &s, int n, int ch) { return s.E + (n + ch - 1) / ch; }
+// items of n entries at ch per item: each of at most min(E, n) experts adds at
+// most one item that is not full
+int group_work_max(const Shape &s, int n, int ch) { return std::min(s.E, n) + (n + ch - 1) / ch; }
 
 int group_work_max(const Shape &s, int n) {
     const int ch = gu_chunk(s.nbH) < dn_chunk(s.nbI, s.I) ? gu_chunk(s.nbH) : dn_chunk(s.nbI, s.I);
