@@ -617,7 +617,7 @@ static int layer_kernels_grouped(tg_arena *a, const Scratch &c, int layer, const
             G.drop = tg::poll_drop();
             if (gd)
                 PROFILED("gu_down_mfma", st,
-                         tg::launch_gu_down_ms(lp, s, wmax, c.work, c.work_n, ent, c.xq, c.xd, c.hq, c.hd, c.hs, c.D,
+                         tg::launch_gu_down_ms(lp, s, mt, wmax, c.work, c.work_n, ent, c.xq, c.xd, c.hq, c.hd, c.hs, c.D,
                                                G, st));
             else
                 PROFILED("gu_down_mfma", st,

@@ -341,7 +341,7 @@ struct GdArgs {
 // the fused launch applies: one-tile items (mt == 1), the down K at most 8
 // chunks of 8 blocks, and TG_FUSE_GD not 0 (read per call)
 bool gd_fuses(const Shape &s, int mt);
-hipError_t launch_gu_down_ms(const uint8_t *layer_pl, const Shape &s, int wmax, const int32_t *work,
+hipError_t launch_gu_down_ms(const uint8_t *layer_pl, const Shape &s, int mt, int wmax, const int32_t *work,
                              const int32_t *work_n, const int32_t *entries, const int8_t *xq, const float *xd,
                              int8_t *hq, float *hd, int *hs, float *D, const GdArgs &G, hipStream_t st);
 // The same for the 16 x 16 items (mt == 4 with items of more than 128

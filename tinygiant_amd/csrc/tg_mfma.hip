@@ -31,6 +31,7 @@
 // of one entry sit in lanes n and n + 32, 16 registers each.  Down writes
 // fp32 rows per entry for the combine.
 #include <atomic>
+#include <cmath>
 
 #include "tg_device.h"
 #include "tg_internal.h"
@@ -455,14 +456,20 @@ TG_DEV void fused_combine(const FuseArgs &F, const Shape &s, const int32_t *__re
 // A layer (30B / 235B shape, weights from HBM), before and after: 5 tokens 75.9 ->
 // 60.7 / 122.9 -> 103 us, 64 tokens 108.5 -> 92.7 / 314 -> 260 us.
 constexpr int MS_NW = 4;    // waves per block
-constexpr int MS_PF_GATE = 2, MS_PF_DOWN = 3;  // weight chunks in flight per wave (4 in gate/up measured the same)
-struct MsLds {
-    static constexpr int ACT = 0;                    // [4 chunks][32 entries][256 bytes, 16-byte pieces rotated by the entry]
-    static constexpr int DX = ACT + 4 * 32 * 256;    // [4 chunks][8 blocks][32 entries] activation scales
-    static constexpr int WB = DX + 4 * MF_KC * 32 * 4;  // [wave][32 rows][128 bytes, piece p of row r at p ^ (r & 7)]
+// weight chunks in flight per wave (with four or with the LDS reads and MFMAs of
+// the next blocks issued ahead of a block's epilogue, 16-entry items took the
+// same time and spilled)
+constexpr int ms_pf(int m, bool pair) { return m == 16 ? 2 : pair ? 4 : 3; }
+template <int M> struct MsLds {
+    static constexpr int ACT = 0;                    // [4 chunks][M entries][256 bytes, 16-byte pieces rotated by the entry]
+    static constexpr int DX = ACT + 4 * M * 256;     // [4 chunks][8 blocks][M entries] activation scales
+    static constexpr int WB = DX + 4 * MF_KC * M * 4;  // [wave][32 rows][128 bytes, piece p of row r at p ^ (r & 7)]
     static constexpr int WS = WB + MS_NW * 4096;     // [wave][2][32 rows][4 chunks' scales, chunk p at p ^ (r/2 & 3)]
     static constexpr int BYTES = WS + MS_NW * 4096;
 };
+// blocks per CU (the LDS allows no more; 168 or 256 VGPRs)
+constexpr int ms_blocks(int m) { return m == 16 ? 3 : 2; }
+static_assert((MsLds<16>::BYTES + 1280) * 3 <= 160 * 1024 && (MsLds<32>::BYTES + 1280) * 2 <= 160 * 1024, "LDS per CU");
 
 template <int CTRL>
 TG_DEV float dpp_f(float v) {
@@ -500,7 +507,7 @@ TG_DEV int half_sum(int v) {
 // acknowledged, counts itself in at rdy[wi]; a down block waits (bounded)
 // until all `need` gate/up blocks of its item have, its first weights in
 // flight meanwhile, then stages h at agent scope.
-template <bool PAIR, bool GD>
+template <int M, bool PAIR, bool GD>
 TG_DEV __attribute__((always_inline)) void ms_item(const uint8_t *__restrict__ layer_pl, const Shape s,
                                                    const int32_t *__restrict__ work,
                                                    const int32_t *__restrict__ entries,
@@ -511,10 +518,12 @@ TG_DEV __attribute__((always_inline)) void ms_item(const uint8_t *__restrict__ l
     // the launch's dynamic LDS, named here so its addresses stay LDS
     // addresses (through a generic pointer each cast to LDS adds a null test)
     extern __shared__ __align__(16) uint8_t smem[];
-    constexpr int M = 32, NW = MS_NW, NT = NW * 64, PF = PAIR ? MS_PF_GATE : MS_PF_DOWN;
+    using Lds = MsLds<M>;
+    constexpr int NW = MS_NW, NT = NW * 64, PF = ms_pf(M, PAIR);
     constexpr int FA = M * 256, FD = MF_KC * M * 4;  // bytes of one chunk's rows, scales of one chunk
     constexpr int JA = FA / (NT * 16);               // DMA rounds of a chunk's rows
-    static_assert(JA * NT * 16 == FA && NT * 4 == FD && MF_KC == 8, "staging map");
+    constexpr int ND = FD / 256;                     // waves that stage a chunk's scales
+    static_assert((M == 16 || M == 32) && JA * NT * 16 == FA && MF_KC == 8, "staging map");
     const int e = work[3 * wi], o = work[3 * wi + 1], c = work[3 * wi + 2];
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, n = lane & 31,
               h = lane >> 5;
@@ -548,7 +557,7 @@ TG_DEV __attribute__((always_inline)) void ms_item(const uint8_t *__restrict__ l
         for (int j = 0; j < 2; j++) {
             const int r = j * 16 + (lane >> 2), p = (lane & 3) ^ ((r >> 1) & 3);
             lds_dma16(wsc + (size_t)r * nb * 2 + min(4 * g + p, nch - 1) * 16,
-                      lds_addr(smem, MsLds::WS + wave * 4096 + (g & 1) * 2048 + j * 1024));
+                      lds_addr(smem, Lds::WS + wave * 4096 + (g & 1) * 2048 + j * 1024));
         }
     };
 
@@ -606,18 +615,20 @@ TG_DEV __attribute__((always_inline)) void ms_item(const uint8_t *__restrict__ l
 #pragma unroll
                 for (int j = 0; j < JA; j++) {
                     if (4 * (j * NW + wave) < c) {  // uniform
-                        const uint32_t m0 = lds_addr(smem, MsLds::ACT + (ch & 3) * FA + (j * NW + wave) * 1024);
+                        const uint32_t m0 = lds_addr(smem, Lds::ACT + (ch & 3) * FA + (j * NW + wave) * 1024);
                         if constexpr (GD && !PAIR)
                             lds_dma16_coh(asrc[j] + ch * MF_KC * 32, m0);
                         else
                             lds_dma16(asrc[j] + ch * MF_KC * 32, m0);
                     }
                 }
-                const uint32_t m0 = lds_addr(smem, MsLds::DX + (ch & 3) * FD + wave * 256);
-                if constexpr (GD && !PAIR)
-                    lds_dma4_coh(dsrc + ch * MF_KC, m0);
-                else
-                    lds_dma4(dsrc + ch * MF_KC, m0);
+                if (wave < ND) {  // uniform
+                    const uint32_t m0 = lds_addr(smem, Lds::DX + (ch & 3) * FD + wave * 256);
+                    if constexpr (GD && !PAIR)
+                        lds_dma4_coh(dsrc + ch * MF_KC, m0);
+                    else
+                        lds_dma4(dsrc + ch * MF_KC, m0);
+                }
             }
         }
     };
@@ -640,9 +651,9 @@ TG_DEV __attribute__((always_inline)) void ms_item(const uint8_t *__restrict__ l
     float acc[16];
 #pragma unroll
     for (int r = 0; r < 16; r++) acc[r] = 0.0f;
-    uint8_t *wb = smem + MsLds::WB + wave * 4096;
+    uint8_t *wb = smem + Lds::WB + wave * 4096;
     uint8_t *wb_put = wb + (lane >> 3) * 128 + (((lane & 7) ^ (lane >> 3)) << 4);
-    const uint8_t *wb_row = wb + n * 128, *ws_row = smem + MsLds::WS + wave * 4096 + n * 64;
+    const uint8_t *wb_row = wb + n * 128, *ws_row = smem + Lds::WS + wave * 4096 + n * 64;
 
     // register groups holding entries of the item (8 entries per group)
     auto run = [&](auto ngc) {
@@ -659,8 +670,8 @@ TG_DEV __attribute__((always_inline)) void ms_item(const uint8_t *__restrict__ l
                 const uint4 sc =
                     *reinterpret_cast<const uint4 *>(ws_row + ((ch >> 2) & 1) * 2048 + (((ch & 3) ^ ((n >> 1) & 3)) << 4));
                 const uint32_t scw[4] = {sc.x, sc.y, sc.z, sc.w};
-                const uint8_t *tq = smem + MsLds::ACT + (ch & 3) * FA + n * 256;
-                const float *xq = reinterpret_cast<const float *>(smem + MsLds::DX + (ch & 3) * FD) + 4 * h;
+                const uint8_t *tq = smem + Lds::ACT + (ch & 3) * FA + (n & (M - 1)) * 256;
+                const float *xq = reinterpret_cast<const float *>(smem + Lds::DX + (ch & 3) * FD) + 4 * h;
 #pragma unroll
                 for (int bl = 0; bl < MF_KC; bl++) {
                     const uint4 blk = *reinterpret_cast<const uint4 *>(wb_row + ((bl ^ (n & 7)) << 4));
@@ -714,10 +725,15 @@ TG_DEV __attribute__((always_inline)) void ms_item(const uint8_t *__restrict__ l
         }
     };
     const int ng = (c + 7) >> 3;
-    if (ng >= 4) run(Tiles<4>{});
-    else if (ng == 3) run(Tiles<3>{});
-    else if (ng == 2) run(Tiles<2>{});
-    else run(Tiles<1>{});
+    if constexpr (M == 32) {
+        if (ng >= 4) run(Tiles<4>{});
+        else if (ng == 3) run(Tiles<3>{});
+        else if (ng == 2) run(Tiles<2>{});
+        else run(Tiles<1>{});
+    } else {
+        if (ng >= 2) run(Tiles<2>{});
+        else run(Tiles<1>{});
+    }
 
     if (PAIR) {
         // the pair's sums meet in LDS (over the activation buffers) and each
@@ -793,8 +809,8 @@ TG_DEV __attribute__((always_inline)) void ms_item(const uint8_t *__restrict__ l
     }
 }
 
-template <bool PAIR>
-__global__ __launch_bounds__(MS_NW * 64, 2) void k_mfma_small(const uint8_t *__restrict__ layer_pl, Shape s,
+template <int M, bool PAIR>
+__global__ __launch_bounds__(MS_NW * 64, ms_blocks(M)) void k_mfma_small(const uint8_t *__restrict__ layer_pl, Shape s,
                                                               const int32_t *__restrict__ work,
                                                               const int32_t *__restrict__ work_n,
                                                               const int32_t *__restrict__ entries,
@@ -803,7 +819,7 @@ __global__ __launch_bounds__(MS_NW * 64, 2) void k_mfma_small(const uint8_t *__r
                                                               float *__restrict__ od, int *__restrict__ os,
                                                               float *__restrict__ D, FuseArgs F) {
     if ((int)blockIdx.y >= work_n[0]) return;  // uniform over the block
-    ms_item<PAIR, false>(layer_pl, s, work, entries, aq, ad, oq, od, os, D, F, (int)blockIdx.y, (int)blockIdx.x,
+    ms_item<M, PAIR, false>(layer_pl, s, work, entries, aq, ad, oq, od, os, D, F, (int)blockIdx.y, (int)blockIdx.x,
                          GdArgs());
 }
 
@@ -816,7 +832,8 @@ __global__ __launch_bounds__(MS_NW * 64, 2) void k_mfma_small(const uint8_t *__r
 // takes a slot; a down block's wait ends once the gate/up blocks of its item, on
 // whichever XCD, have stored h.  The down blocks then fill the slots the
 // gate/up launch's last round leaves idle.
-__global__ __launch_bounds__(MS_NW * 64, 2) void k_mfma_small_gd(const uint8_t *__restrict__ layer_pl, Shape s,
+template <int M>
+__global__ __launch_bounds__(MS_NW * 64, ms_blocks(M)) void k_mfma_small_gd(const uint8_t *__restrict__ layer_pl, Shape s,
                                                                  const int32_t *__restrict__ work,
                                                                  const int32_t *__restrict__ work_n,
                                                                  const int32_t *__restrict__ entries,
@@ -826,10 +843,10 @@ __global__ __launch_bounds__(MS_NW * 64, 2) void k_mfma_small_gd(const uint8_t *
                                                                  int gxd) {
     const int b = (int)blockIdx.x, n = work_n[0], ng = gxg * n;
     if (b < ng) {
-        ms_item<true, true>(layer_pl, s, work, entries, xq, xd, hq, hd, hs, nullptr, FuseArgs(), b / gxg, b % gxg, G);
+        ms_item<M, true, true>(layer_pl, s, work, entries, xq, xd, hq, hd, hs, nullptr, FuseArgs(), b / gxg, b % gxg, G);
     } else if (b < ng + gxd * n) {
         const int d = b - ng;
-        ms_item<false, true>(layer_pl, s, work, entries, hq, hd, nullptr, nullptr, nullptr, D, FuseArgs(), d / gxd,
+        ms_item<M, false, true>(layer_pl, s, work, entries, hq, hd, nullptr, nullptr, nullptr, D, FuseArgs(), d / gxd,
                              d % gxd, G);
     }
 }
@@ -1381,20 +1398,29 @@ hipError_t launch_clock_mfma(unsigned long long *out, int blocks, int iters, hip
 }
 
 int mfma_item_entries(const Shape &s, int mt) {
-    return mt == 4 && x16_ok(s, true) && x16_ok(s, false) ? XT_CT * 16 : 32 * mt;
+    return mt == 4 && x16_ok(s, true) && x16_ok(s, false) ? XT_CT * 16 : mt == 0 ? 16 : 32 * mt;
 }
 
-// Entries per expert in a work item, in M-tiles of 32, from the batch's mean
-// entries per expert.  Where both fused gate/up + down launches take the shape,
-// the one-tile kernel up to a mean of 24 and the 16 x 16 kernel above: at the
-// 30B shape (us a layer; one-tile, 16 x 16) 333 tokens 171, 182; 420 tokens
-// 186, 184; 512 tokens 219, 199; 1024 tokens 343, 256; at 235B 333 tokens 538,
-// 574; 420 tokens 599, 595; 512 tokens 673, 628.  The 32 x 32 kernels between
-// them (two launches, 247 us at 333 tokens, 382 at 1024, and 862, 1318 at
-// 235B) only take shapes that these do not.
+// Entries per expert in a work item, in M-tiles of 32 (0: 16 entries), from the
+// batch's mean entries per expert.  Where both fused gate/up + down launches take
+// the shape, the one-tile kernel up to a mean of 24 and the 16 x 16 kernel above
+// (30B shape, us a layer at 420 tokens 186, 184; 512 tokens 219, 199; 235B 420
+// tokens 599, 595).  Items of 16 entries let three blocks share a CU instead of
+// two: they pay once the gate/up blocks fill five a CU (30B 16 tokens 69 us, 73
+// with 16-entry items; 32 tokens 77, 75; 64 tokens 93, 84; 235B 8 tokens 122, 128;
+// 16 tokens 164, 152) and until experts with more than 16 entries, whose weights
+// they read twice, weigh more: a mean of 8, or 12 where K is at most 8 chunks (30B
+// 192 tokens 135, 130; 235B 160 tokens 356, 365).  Other shapes keep the 32 x 32
+// kernels (two launches).
 int mfma_tiles(const Shape &s, int T) {
     const int avg = (T * s.k + s.E - 1) / s.E;
-    if (mfma_item_entries(s, 4) > 128 && s.nbI % MF_KC == 0) return avg > 24 ? 4 : 1;
+    if (mfma_item_entries(s, 4) > 128 && s.nbI % MF_KC == 0) {
+        if (avg > 24) return 4;
+        // experts that T tokens select, each missed by a token with chance 1 - k / E
+        const double distinct = s.E * (1.0 - std::pow(1.0 - (double)s.k / s.E, T));
+        const int gxg = (s.I + 63) / 64;
+        return avg <= (s.nbH <= 8 * MF_KC ? 12 : 8) && distinct * gxg >= 1280.0 ? 0 : 1;
+    }
     return avg > 64 ? 4 : (avg > 16 ? 2 : 1);
 }
 
@@ -1420,7 +1446,7 @@ static hipError_t mf_go(const uint8_t *layer_pl, const Shape &s, int wmax, const
     return hipGetLastError();
 }
 
-template <bool PAIR>
+template <int M, bool PAIR>
 static hipError_t ms_go(const uint8_t *layer_pl, const Shape &s, int wmax, const int32_t *work, const int32_t *work_n,
                         const int32_t *entries, const int8_t *aq, const float *ad, int8_t *oq, float *od, int *os,
                         float *D, const FuseArgs &F, hipStream_t st) {
@@ -1433,9 +1459,9 @@ static hipError_t ms_go(const uint8_t *layer_pl, const Shape &s, int wmax, const
     }
     const unsigned gx = PAIR ? mf_cdiv((size_t)rows, 32 * (MS_NW / 2)) : mf_cdiv((size_t)rows, 32 * MS_NW);
     static std::atomic<uint64_t> attr{0};
-    hipError_t e = lds_attr(reinterpret_cast<const void *>(&k_mfma_small<PAIR>), MsLds::BYTES, attr);
+    hipError_t e = lds_attr(reinterpret_cast<const void *>(&k_mfma_small<M, PAIR>), MsLds<M>::BYTES, attr);
     if (e != hipSuccess) return e;
-    TG_LAUNCH((k_mfma_small<PAIR>), dim3(gx, wmax), dim3(MS_NW * 64), MsLds::BYTES, st, layer_pl, s, work, work_n,
+    TG_LAUNCH((k_mfma_small<M, PAIR>), dim3(gx, wmax), dim3(MS_NW * 64), MsLds<M>::BYTES, st, layer_pl, s, work, work_n,
               entries, aq, ad, oq, od, os, D, F);
     return hipGetLastError();
 }
@@ -1471,7 +1497,8 @@ hipError_t launch_gateup_mfma(const uint8_t *layer_pl, const Shape &s, int mt, i
     if (!mfma_shape_ok(s)) return hipErrorInvalidValue;
     (void)xs;
     const FuseArgs none;
-    if (mt == 1) return ms_go<true>(layer_pl, s, wmax, work, work_n, entries, xq, xd, hq, hd, hs, nullptr, none, st);
+    if (mt == 0) return ms_go<16, true>(layer_pl, s, wmax, work, work_n, entries, xq, xd, hq, hd, hs, nullptr, none, st);
+    if (mt == 1) return ms_go<32, true>(layer_pl, s, wmax, work, work_n, entries, xq, xd, hq, hd, hs, nullptr, none, st);
     if (mt == 2) return mf_go<2, true>(layer_pl, s, wmax, work, work_n, entries, xq, xd, hq, hd, hs, nullptr, st);
     if (mfma_item_entries(s, mt) > 128)
         return x16_go<true>(layer_pl, s, wmax, work, work_n, entries, xq, xd, hq, hd, hs, nullptr, none, st);
@@ -1486,7 +1513,7 @@ hipError_t launch_gateup_mfma(const uint8_t *layer_pl, const Shape &s, int mt, i
 bool down_fuses(const Shape &s, int mt, int T) {
     const char *v = getenv("TG_FUSE_COMBINE");
     const bool on = v && v[0] == '1';
-    const bool kern = (mt == 1 && s.nbI % MF_KC == 0) || (mt == 4 && mfma_item_entries(s, mt) > 128);
+    const bool kern = (mt <= 1 && s.nbI % MF_KC == 0) || (mt == 4 && mfma_item_entries(s, mt) > 128);
     return on && kern && s.H % FC_ROWS == 0 && (size_t)T * s.k * s.H < ((size_t)1 << 31);
 }
 
@@ -1495,8 +1522,10 @@ hipError_t launch_down_mfma(const uint8_t *layer_pl, const Shape &s, int mt, int
                             const int *hs, float *D, const FuseArgs &F, hipStream_t st) {
     if (!mfma_shape_ok(s)) return hipErrorInvalidValue;
     (void)hs;
-    if (mt == 1) return ms_go<false>(layer_pl, s, wmax, work, work_n, entries, hq, hd, nullptr, nullptr, nullptr,
-                                     D, F, st);
+    if (mt == 0) return ms_go<16, false>(layer_pl, s, wmax, work, work_n, entries, hq, hd, nullptr, nullptr, nullptr,
+                                         D, F, st);
+    if (mt == 1) return ms_go<32, false>(layer_pl, s, wmax, work, work_n, entries, hq, hd, nullptr, nullptr, nullptr,
+                                         D, F, st);
     if (mt == 4 && mfma_item_entries(s, mt) > 128)
         return x16_go<false>(layer_pl, s, wmax, work, work_n, entries, hq, hd, nullptr, nullptr, nullptr, D, F,
                              st);
@@ -1509,7 +1538,7 @@ hipError_t launch_down_mfma(const uint8_t *layer_pl, const Shape &s, int mt, int
 bool gd_fuses(const Shape &s, int mt) {
     const char *v = getenv("TG_FUSE_GD");
     const bool on = !(v && v[0] == '0');
-    return on && mt == 1 && mfma_shape_ok(s) && s.nbH % MF_KC == 0 && s.nbI % MF_KC == 0;
+    return on && mt <= 1 && mfma_shape_ok(s) && s.nbH % MF_KC == 0 && s.nbI % MF_KC == 0;
 }
 
 bool gd16_fuses(const Shape &s, int mt) {
@@ -1535,20 +1564,29 @@ hipError_t launch_gu_down_x16(const uint8_t *layer_pl, const Shape &s, int wmax,
     return hipGetLastError();
 }
 
-hipError_t launch_gu_down_ms(const uint8_t *layer_pl, const Shape &s, int wmax, const int32_t *work,
+template <int M>
+static hipError_t gd_go(const uint8_t *layer_pl, const Shape &s, int wmax, const int32_t *work,
+                        const int32_t *work_n, const int32_t *entries, const int8_t *xq, const float *xd, int8_t *hq,
+                        float *hd, int *hs, float *D, const GdArgs &G, int gxg, int gxd, hipStream_t st) {
+    static std::atomic<uint64_t> attr{0};
+    hipError_t e = lds_attr(reinterpret_cast<const void *>(&k_mfma_small_gd<M>), MsLds<M>::BYTES, attr);
+    if (e != hipSuccess) return e;
+    TG_LAUNCH((k_mfma_small_gd<M>), dim3((unsigned)((gxg + gxd) * wmax)), dim3(MS_NW * 64), MsLds<M>::BYTES, st,
+              layer_pl, s, work, work_n, entries, xq, xd, hq, hd, hs, D, G, gxg, gxd);
+    return hipGetLastError();
+}
+
+hipError_t launch_gu_down_ms(const uint8_t *layer_pl, const Shape &s, int mt, int wmax, const int32_t *work,
                              const int32_t *work_n, const int32_t *entries, const int8_t *xq, const float *xd,
                              int8_t *hq, float *hd, int *hs, float *D, const GdArgs &G0, hipStream_t st) {
-    if (!gd_fuses(s, 1) || !G0.rdy || !G0.err || G0.spin == 0) return hipErrorInvalidValue;
+    if (!gd_fuses(s, mt) || !G0.rdy || !G0.err || G0.spin == 0) return hipErrorInvalidValue;
     const int gxg = (int)mf_cdiv((size_t)s.I, 32 * (MS_NW / 2)), gxd = (int)mf_cdiv((size_t)s.H, 32 * MS_NW);
     if ((size_t)(gxg + gxd) * (size_t)wmax >= ((size_t)1 << 31)) return hipErrorInvalidValue;
     GdArgs G = G0;
     G.need = gxg;
-    static std::atomic<uint64_t> attr{0};
-    hipError_t e = lds_attr(reinterpret_cast<const void *>(&k_mfma_small_gd), MsLds::BYTES, attr);
-    if (e != hipSuccess) return e;
-    TG_LAUNCH(k_mfma_small_gd, dim3((unsigned)((gxg + gxd) * wmax)), dim3(MS_NW * 64), MsLds::BYTES, st, layer_pl, s,
-              work, work_n, entries, xq, xd, hq, hd, hs, D, G, gxg, gxd);
-    return hipGetLastError();
+    if (mt == 0)
+        return gd_go<16>(layer_pl, s, wmax, work, work_n, entries, xq, xd, hq, hd, hs, D, G, gxg, gxd, st);
+    return gd_go<32>(layer_pl, s, wmax, work, work_n, entries, xq, xd, hq, hd, hs, D, G, gxg, gxd, st);
 }
 
 }  // namespace tg
