@@ -219,3 +219,44 @@ def test_235b_shape_stack(O, tglib):
         a.status()
     finally:
         a.close()
+
+
+@pytest.mark.parametrize("T", [2, 3])
+@pytest.mark.parametrize("H,I,E,k", [(2048, 768, 128, 8), (512, 256, 32, 8)])
+def test_few_tokens_match_oracle(O, tglib, H, I, E, k, T):
+    """Two and three tokens: one layer (routed launches after one prologue for both; the grouped path from three) with
+    and without routing outputs, a stack of three layers token by token, and the batch paths chosen by hand."""
+    from tinygiant_amd.arena import HBMExpertArena
+    from tinygiant_amd.moe import MoEBlock
+    gpu_note(f"few tokens H={H} I={I} E={E} T={T}")
+    L = 3
+    a = HBMExpertArena(L, E, H, I, k)
+    try:
+        layers = []
+        for l in range(L):
+            lb, r = O.synth_layer(113, l, H, I, E)
+            a.load_layer(l, lb)
+            a.load_router(l, r)
+            layers.append((lb, r))
+        x = O.synth_normal(113, O.stream_id(0, T, 4), 1.0, T * H).reshape(T, H)
+        blk = MoEBlock(a)
+        ref, ridx, rw, _ = O.moe_layer(*layers[1], H, I, E, k, x)
+        for path in (a.BATCH_AUTO, a.BATCH_GROUPED, a.BATCH_PER_TOKEN, a.BATCH_AUTO):
+            a.set_batch_path(path)
+            out, idx, w = blk.forward(1, torch.from_numpy(x).cuda(), return_routing=True)
+            torch.cuda.synchronize()
+            assert np.array_equal(idx.cpu().numpy(), ridx)
+            assert np.array_equal(w.cpu().numpy().view(np.uint32), rw.view(np.uint32))
+            assert np.array_equal(out.cpu().numpy().view(np.uint32), ref.view(np.uint32))
+        out, idx, w = blk.forward_host(1, x)
+        assert np.array_equal(idx, ridx) and np.array_equal(w.view(np.uint32), rw.view(np.uint32))
+        assert np.array_equal(out.view(np.uint32), ref.view(np.uint32))
+        y = x
+        for lb, r in layers:
+            y = y + O.moe_layer(lb, r, H, I, E, k, y)[0]
+        got = blk.step(torch.from_numpy(x).cuda())
+        torch.cuda.synchronize()
+        assert np.array_equal(got.cpu().numpy().view(np.uint32), y.astype(np.float32).view(np.uint32))
+        assert tglib.tg_arena_status(a.handle) == 0
+    finally:
+        a.close()

@@ -237,7 +237,8 @@ hipError_t launch_sample_all(const SmpBufs &b, const float *logits, int V, float
 bool layer_dec_ok(const Shape &s, int n_cu);
 size_t dec_part_floats(const Shape &s);
 size_t dec_ow_words(const Shape &s);
-hipError_t launch_dec_part(const float *Wr, const float *x, const Shape &s, float *part, uint32_t *ctl, int n_layers,
+// (one or two tokens; the generation advances by n_gen)
+hipError_t launch_dec_part(const float *Wr, const float *x, const Shape &s, int tokens, float *part, uint32_t *ctl, int n_gen,
                            hipStream_t st);
 hipError_t launch_layer_dec(const uint8_t *layer_pl, const Shape &s, int n_cu, const float *x, const float *gn,
                             const float *part_in, const float *wr_next, float *part_out, uint64_t *hw, uint64_t *ow,
@@ -278,7 +279,8 @@ struct RouteGroup {
 };
 hipError_t launch_route_q8(const float *raw, const float *chains, const float *x, const float *gn, int T, int E,
                            int H, int k, float eps, int32_t *idx, float *w, int8_t *xq, float *xd, int *xs,
-                           int32_t *ecnt, int32_t *ent_cap, const RouteGroup &G, hipStream_t st);
+                           int32_t *ecnt, int32_t *ent_cap, const RouteGroup &G, int32_t *idx_out, float *w_out,
+                           hipStream_t st);
 // TG_ROUTE_GROUP not 0 (read per call): route_q8 builds the placed lists'
 // one-tile work items itself
 bool route_groups_on();

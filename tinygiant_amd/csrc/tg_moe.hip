@@ -2041,9 +2041,13 @@ __global__ __launch_bounds__(FX_THREADS) void k_layer_dec(const float *__restric
 // call's first layer (block g: group g; thread e < E the chain of expert e,
 // thread E the chain of squares), and block 0 advances the generation word
 // by n_layers (one generation per layer launch of the call).
+// grid (H/32, tokens): token t's partials at part + t * half
 __global__ __launch_bounds__(256) void k_dec_part(const float *__restrict__ Wr, const float *__restrict__ x, int E,
-                                                  int H, float *__restrict__ part, uint32_t *ctl, int n_layers) {
+                                                  int H, float *__restrict__ part, uint32_t *ctl, int n_gen,
+                                                  size_t half) {
     const int g = blockIdx.x, tid = threadIdx.x, G = H / RG;
+    x += (size_t)blockIdx.y * H;
+    part += blockIdx.y * half;
     const float4 *x4 = reinterpret_cast<const float4 *>(x + (size_t)g * RG);
     float4 xv[RG / 4];
 #pragma unroll
@@ -2073,9 +2077,9 @@ __global__ __launch_bounds__(256) void k_dec_part(const float *__restrict__ Wr, 
         }
         part[(size_t)E * G + g] = aq;
     }
-    if (g == 0 && tid == 0) {
+    if (g == 0 && blockIdx.y == 0 && tid == 0) {
         uint32_t v = __hip_atomic_load(ctl + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        for (int i = 0; i < n_layers; i++) v = next_gen(v);
+        for (int i = 0; i < n_gen; i++) v = next_gen(v);
         __hip_atomic_store(ctl + 1, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 }
@@ -2155,7 +2159,7 @@ __global__ __launch_bounds__(RO_THREADS) void k_route_q8(const float *__restrict
                                                          float *__restrict__ w, int8_t *__restrict__ xq,
                                                          float *__restrict__ xd, int *__restrict__ xs,
                                                          int32_t *__restrict__ ecnt, int32_t *__restrict__ ent_cap,
-                                                         RouteGroup G) {
+                                                         RouteGroup G, int32_t *idx_out, float *w_out) {
     extern __shared__ __align__(16) uint8_t smem[];
     __shared__ float rsum[RO_THREADS];
     RouteLds L = route_lds(smem, H);
@@ -2191,6 +2195,9 @@ __global__ __launch_bounds__(RO_THREADS) void k_route_q8(const float *__restrict
             const int j = k - 1 - tid;
             idx[(size_t)t * k + j] = L.sidx[j];
             w[(size_t)t * k + j] = wj;
+            // the caller's copies (two device copies after the layer's launches took about 5 us)
+            if (idx_out) idx_out[(size_t)t * k + j] = L.sidx[j];
+            if (w_out) w_out[(size_t)t * k + j] = wj;
             if (ent_cap) {  // entry t k + j into its expert's list of capacity T, in arrival order
                 const int e = L.sidx[j];
                 const int pos = atomicAdd(ecnt + e, 1);
@@ -2933,9 +2940,11 @@ bool layer_dec_ok(const Shape &s, int n_cu) {
            RG - rd <= FX_THREADS && lds <= 160 * 1024;
 }
 
-hipError_t launch_dec_part(const float *Wr, const float *x, const Shape &s, float *part, uint32_t *ctl, int n_layers,
-                           hipStream_t st) {
-    TG_LAUNCH(k_dec_part, dim3(s.H / RG), dim3(256), 0, st, Wr, x, s.E, s.H, part, ctl, n_layers);
+hipError_t launch_dec_part(const float *Wr, const float *x, const Shape &s, int tokens, float *part, uint32_t *ctl,
+                           int n_gen, hipStream_t st) {
+    if (tokens < 1 || tokens > 2) return hipErrorInvalidValue;  // part holds two buffers
+    TG_LAUNCH(k_dec_part, dim3(s.H / RG, tokens), dim3(256), 0, st, Wr, x, s.E, s.H, part, ctl, n_gen,
+              dec_part_floats(s) / 2);
     return hipGetLastError();
 }
 
@@ -3000,7 +3009,8 @@ bool grouped_shape_ok(const Shape &s) {
 
 hipError_t launch_route_q8(const float *raw, const float *chains, const float *x, const float *gn, int T, int E,
                            int H, int k, float eps, int32_t *idx, float *w, int8_t *xq, float *xd, int *xs,
-                           int32_t *ecnt, int32_t *ent_cap, const RouteGroup &G, hipStream_t st) {
+                           int32_t *ecnt, int32_t *ent_cap, const RouteGroup &G, int32_t *idx_out, float *w_out,
+                           hipStream_t st) {
     if (G.arrive && (!ent_cap || !ecnt || G.ch <= 0 || G.wmax <= 0 || E > RO_THREADS || !G.counts || !G.offsets ||
                      !G.work || !G.work_n))
         return hipErrorInvalidValue;
@@ -3016,7 +3026,7 @@ hipError_t launch_route_q8(const float *raw, const float *chains, const float *x
         hipError_t e = allow_lds((const void *)kern, lds);
         if (e != hipSuccess) return e;
         TG_LAUNCH(kern, dim3(T), dim3(RO_THREADS), lds, st, raw, chains, T, x, gn, E, H, k, eps, idx, w, xq, xd, xs,
-                  ecnt, ent_cap, G);
+                  ecnt, ent_cap, G, idx_out, w_out);
         return hipGetLastError();
     };
     if (chains) return go(k_route_q8<true, RO_MAXPASS>);
