@@ -1270,6 +1270,9 @@ struct LgCarve {
     }
 };
 
+static hipStream_t g_lg_kv_st = nullptr;  // the KV cache's copy (lg_kv_in) and its end
+static hipEvent_t g_lg_kv_ev = nullptr;
+static bool g_lg_kv_busy = false;         // copies issued on it that g_lg_st does not wait for
 static size_t g_lg_pin_off = 0;  // bounce bytes handed out since the last wait (pinned buffer below)
 static int lg_sync();
 
@@ -1282,12 +1285,17 @@ static int lg_reserve(size_t bytes) {
         HIP_TRY(hipSetDevice(g_lg_dev));
         (void)hipFree(g_lg_buf);
         if (g_lg_st) (void)hipStreamDestroy(g_lg_st);
+        if (g_lg_kv_st) (void)hipStreamDestroy(g_lg_kv_st);
+        if (g_lg_kv_ev) (void)hipEventDestroy(g_lg_kv_ev);
         g_lg_buf = nullptr; g_lg_cap = 0; g_lg_st = nullptr;
+        g_lg_kv_st = nullptr; g_lg_kv_ev = nullptr; g_lg_kv_busy = false;
         HIP_TRY(hipSetDevice(dev));
     }
     g_lg_dev = dev;
     if (!g_lg_st) HIP_TRY(hipStreamCreateWithFlags(&g_lg_st, hipStreamNonBlocking));
-    if (g_lg_pin_off) {  // a call that failed before its closing wait left bounce slots taken
+    if (!g_lg_kv_st) HIP_TRY(hipStreamCreateWithFlags(&g_lg_kv_st, hipStreamNonBlocking));
+    if (!g_lg_kv_ev) HIP_TRY(hipEventCreateWithFlags(&g_lg_kv_ev, hipEventDisableTiming));
+    if (g_lg_pin_off || g_lg_kv_busy) {  // a call that failed before its closing wait left bounce slots taken
         int rc2 = lg_sync();
         if (rc2) return rc2;
     }
@@ -1342,6 +1350,8 @@ static int lg_h2d(void *dst, const void *src, size_t n) {
 // again afterwards.
 static int lg_sync() {
     HIP_TRY(hipStreamSynchronize(g_lg_st));
+    if (g_lg_kv_busy) HIP_TRY(hipStreamSynchronize(g_lg_kv_st));  // a call failed on the way
+    g_lg_kv_busy = false;
     g_lg_pin_off = 0;  // every copy issued so far has completed
     return TG_OK;
 }
@@ -1604,7 +1614,7 @@ static int lg_expert(const uint8_t *gate, const uint8_t *up, const void *down, i
         P.w[0] = weight;
         PROFILED("lg_moe_gateup", st, tg::launch_moe_gateup_q4k(P, 1, x, b.g, embed, inter, st));
         PROFILED("lg_moe_silu", st, tg::launch_moe_silu_q8k(b.g, b.hq, 1, inter, st));
-        PROFILED("lg_moe_down", st, tg::launch_moe_down_acc_q4k(P, 1, b.hq, out, embed, inter, true, st));
+        PROFILED("lg_moe_down", st, tg::launch_moe_down_acc_q4k(P, 1, b.hq, out, embed, inter, tg::LG_DOWN_ACC, st));
         return TG_OK;
     }
     PROFILED("lg_quant", st, tg::launch_quantize_q8k(x, b.xq, gbpr, st));
@@ -1710,11 +1720,11 @@ static int lg_moe_ops(int n, const uint8_t *const *gp, const uint8_t *const *up,
 // out = sum over the experts in order of weight * down(SiLU(gate x) * up x),
 // x the device input (its Q8 blocks formed inside the gate / up launch)
 static int lg_moe_run(const tg::LgMoeOps &P, int n, const float *x, float *out, int embed, int inter,
-                      const LgExpertBufs &b, const LgMoeAllBufs &m) {
+                      const LgExpertBufs &b, const LgMoeAllBufs &m, tg::LgDownOut mode = tg::LG_DOWN_SET) {
     hipStream_t st = g_lg_st;
     PROFILED("lg_moe_gateup", st, tg::launch_moe_gateup_q4k(P, n, x, m.gu, embed, inter, st));
     PROFILED("lg_moe_silu", st, tg::launch_moe_silu_q8k(m.gu, m.hq, n, inter, st));
-    PROFILED("lg_moe_down", st, tg::launch_moe_down_acc_q4k(P, n, m.hq, out, embed, inter, false, st));
+    PROFILED("lg_moe_down", st, tg::launch_moe_down_acc_q4k(P, n, m.hq, out, embed, inter, mode, st));
     return TG_OK;
 }
 
@@ -1922,7 +1932,8 @@ struct LgAttn {
 
 // Device buffers of one attention step (weights excluded).
 struct LgAttnBufs {
-    float *x, *q, *k, *v, *qn, *kn, *ao, *out, *kc, *vc, *scr, *cs, *sn;
+    float *x, *q, *k, *v, *qn, *ao, *out, *kc, *vc, *scr, *cs, *sn;
+    float *ret;  // what goes back to the host in one copy: embed outputs, the new keys, the new values
     void *xq, *aq;
 };
 
@@ -1934,12 +1945,12 @@ static LgAttnBufs lg_attn_bufs(LgCarve &c, const LgAttn &g) {
     b.k = c.take<float>(4 * (size_t)g.kv_dim());
     b.v = c.take<float>(4 * (size_t)g.kv_dim());
     b.qn = c.take<float>(4 * (size_t)g.q_dim());
-    b.kn = c.take<float>(4 * (size_t)g.kv_dim());
     b.ao = c.take<float>(4 * (size_t)g.q_dim());
     b.out = c.take<float>(4 * (size_t)g.embed);
     b.kc = c.take<float>(cache);
     b.vc = c.take<float>(cache);
     b.scr = c.take<float>(sizeof(float) * tg::attn_scratch_floats(g.n_heads, g.seq()));
+    b.ret = c.take<float>(4 * ((size_t)g.embed + 2 * (size_t)g.kv_dim()));
     b.cs = c.take<float>(4 * (size_t)(g.hd / 2));
     b.sn = c.take<float>(4 * (size_t)(g.hd / 2));
     b.xq = c.take<uint8_t>((size_t)(g.embed / tg::LG_QK) * tg::LG_Q8K_BYTES);
@@ -1949,38 +1960,57 @@ static LgAttnBufs lg_attn_bufs(LgCarve &c, const LgAttn &g) {
 
 // Host cache rows 0 .. kv_len-1 of every kv head into the device caches
 // [n_kv][seq][hd], and this position's RoPE table rows.
-static int lg_attn_in(const LgAttn &g, const LgAttnBufs &b, const float *kv_k, const float *kv_v,
-                      const float *rope_cos, const float *rope_sin) {
-    const size_t row = 4 * (size_t)g.hd, half = 4 * (size_t)(g.hd / 2);
-    if (g.kv_len > 0) {
-        HIP_TRY(hipMemcpy2DAsync(b.kc, row * g.seq(), kv_k, row * g.kv_max, row * g.kv_len, g.n_kv,
-                                 hipMemcpyHostToDevice, g_lg_st));
-        HIP_TRY(hipMemcpy2DAsync(b.vc, row * g.seq(), kv_v, row * g.kv_max, row * g.kv_len, g.n_kv,
-                                 hipMemcpyHostToDevice, g_lg_st));
-    }
-    int rc;
-    if ((rc = lg_h2d(b.cs, rope_cos + (size_t)g.pos * (g.hd / 2), half)) ||
-        (rc = lg_h2d(b.sn, rope_sin + (size_t)g.pos * (g.hd / 2), half)))
-        return rc;
-    return TG_OK;
+static int lg_rope_in(const LgAttn &g, const LgAttnBufs &b, const float *rope_cos, const float *rope_sin) {
+    const size_t half = 4 * (size_t)(g.hd / 2);
+    int rc = lg_h2d(b.cs, rope_cos + (size_t)g.pos * (g.hd / 2), half);
+    return rc ? rc : lg_h2d(b.sn, rope_sin + (size_t)g.pos * (g.hd / 2), half);
 }
 
-// The new cache rows (row kv_len of every kv head) back to the host caches.
-static int lg_attn_out(const LgAttn &g, const LgAttnBufs &b, float *kv_k, float *kv_v) {
+// The cached rows on a stream of their own: the host copies them out of pageable
+// memory while the projections run (4.2 MB at 1024 positions of 4 x 128: 80-100
+// us on the host either way), and the attention waits for them.
+static int lg_kv_in(const LgAttn &g, const LgAttnBufs &b, const float *kv_k, const float *kv_v) {
     const size_t row = 4 * (size_t)g.hd;
-    HIP_TRY(hipMemcpy2DAsync(kv_k + (size_t)g.kv_len * g.hd, row * g.kv_max, b.kc + (size_t)g.kv_len * g.hd,
-                             row * g.seq(), row, g.n_kv, hipMemcpyDeviceToHost, g_lg_st));
-    HIP_TRY(hipMemcpy2DAsync(kv_v + (size_t)g.kv_len * g.hd, row * g.kv_max, b.vc + (size_t)g.kv_len * g.hd,
-                             row * g.seq(), row, g.n_kv, hipMemcpyDeviceToHost, g_lg_st));
+    if (g.kv_len <= 0) return TG_OK;
+    g_lg_kv_busy = true;
+    HIP_TRY(hipMemcpy2DAsync(b.kc, row * g.seq(), kv_k, row * g.kv_max, row * g.kv_len, g.n_kv, hipMemcpyHostToDevice,
+                             g_lg_kv_st));
+    HIP_TRY(hipMemcpy2DAsync(b.vc, row * g.seq(), kv_v, row * g.kv_max, row * g.kv_len, g.n_kv, hipMemcpyHostToDevice,
+                             g_lg_kv_st));
+    HIP_TRY(hipEventRecord(g_lg_kv_ev, g_lg_kv_st));
+    HIP_TRY(hipStreamWaitEvent(g_lg_st, g_lg_kv_ev, 0));
+    g_lg_kv_busy = false;
     return TG_OK;
 }
 
-// The attention step on device operands (input b.x, output b.out): q/k/v
-// projections (q4: Q4_K q, k, o and f16 v; else f32), per-head RMS norms of
-// q and k (eps 1e-6), RoPE, the new rows into the caches, GQA attention,
-// output projection.
+// b.ret back: the outputs to `output`, the new key and value rows into the
+// caller's caches.
+static int lg_attn_finish(const LgAttn &g, const LgAttnBufs &b, float *output, float *kv_k, float *kv_v) {
+    const size_t ev = 4 * (size_t)g.embed, row = 4 * (size_t)g.hd, kvb = 4 * (size_t)g.kv_dim();
+    const float *kvn = b.ret + g.embed;
+    if (auto *p = static_cast<uint8_t *>(lg_pin_take(ev + 2 * kvb))) {
+        HIP_TRY(hipMemcpyAsync(p, b.ret, ev + 2 * kvb, hipMemcpyDeviceToHost, g_lg_st));
+        int rc = lg_sync();
+        if (rc) return rc;
+        memcpy(output, p, ev);
+        for (int h = 0; h < g.n_kv; h++) {
+            const size_t at = ((size_t)h * g.kv_max + g.kv_len) * g.hd;
+            memcpy(kv_k + at, p + ev + h * row, row);
+            memcpy(kv_v + at, p + ev + kvb + h * row, row);
+        }
+        return TG_OK;
+    }
+    const size_t at = (size_t)g.kv_len * g.hd;
+    HIP_TRY(hipMemcpy2DAsync(kv_k + at, row * g.kv_max, kvn, row, row, g.n_kv, hipMemcpyDeviceToHost, g_lg_st));
+    HIP_TRY(hipMemcpy2DAsync(kv_v + at, row * g.kv_max, kvn + g.kv_dim(), row, row, g.n_kv, hipMemcpyDeviceToHost,
+                             g_lg_st));
+    return lg_finish(output, b.ret, ev);
+}
+
+// b.x (normed) through the attention into out; the new key and value rows to b.ret
 static int lg_attn_core(bool q4, const void *wq, const void *wk, const void *wv, const void *wo, const float *qnw,
-                        const float *knw, const LgAttn &g, const LgAttnBufs &b) {
+                        const float *knw, const LgAttn &g, const LgAttnBufs &b, const float *kv_k, const float *kv_v,
+                        float *out) {
     hipStream_t st = g_lg_st;
     const int ebpr = g.embed / tg::LG_QK;
     if (q4) {
@@ -1991,15 +2021,17 @@ static int lg_attn_core(bool q4, const void *wq, const void *wk, const void *wv,
                  tg::launch_matmul_q4k(static_cast<const uint8_t *>(wk), b.xq, b.k, g.kv_dim(), ebpr, st));
         PROFILED("lg_f16", st, tg::launch_matvec_two_acc(wv, true, b.x, b.v, g.kv_dim(), g.embed, st));
     } else {
-        PROFILED("lg_f32", st, tg::launch_matvec_two_acc(wq, false, b.x, b.q, g.q_dim(), g.embed, st));
-        PROFILED("lg_f32", st, tg::launch_matvec_two_acc(wk, false, b.x, b.k, g.kv_dim(), g.embed, st));
-        PROFILED("lg_f32", st, tg::launch_matvec_two_acc(wv, false, b.x, b.v, g.kv_dim(), g.embed, st));
+        const float *const A[3] = {static_cast<const float *>(wq), static_cast<const float *>(wk),
+                                   static_cast<const float *>(wv)};
+        float *const y[3] = {b.q, b.k, b.v};
+        const int rows[3] = {g.q_dim(), g.kv_dim(), g.kv_dim()};
+        PROFILED("lg_f32", st, tg::launch_matvec3_f32(A, y, rows, b.x, g.embed, st));
     }
-    PROFILED("lg_rms", st, tg::launch_rms_norm_rows(b.q, qnw, b.qn, g.hd, g.n_heads, 1e-6f, st));
-    PROFILED("lg_rms", st, tg::launch_rms_norm_rows(b.k, knw, b.kn, g.hd, g.n_kv, 1e-6f, st));
-    PROFILED("lg_rope", st, tg::launch_rope(b.qn, g.n_heads, g.hd, b.cs, b.sn, st));
-    PROFILED("lg_rope", st, tg::launch_rope(b.kn, g.n_kv, g.hd, b.cs, b.sn, st));
-    PROFILED("lg_kv", st, tg::launch_kv_append(b.kn, b.v, b.kc, b.vc, g.n_kv, g.seq(), g.hd, g.kv_len, st));
+    PROFILED("lg_heads", st,
+             tg::launch_head_prep(b.q, b.k, b.v, qnw, knw, b.cs, b.sn, b.qn, b.kc, b.vc, b.ret + g.embed, g.n_heads,
+                                  g.n_kv, g.seq(), g.hd, g.kv_len, 1e-6f, st));
+    int rc = lg_kv_in(g, b, kv_k, kv_v);
+    if (rc) return rc;
     const float inv_sqrt = 1.0f / sqrtf((float)g.hd);
     PROFILED("lg_attn_sc", st,
              tg::launch_attn_scores(b.qn, b.kc, b.scr, g.n_heads, g.seq(), g.hd, g.n_heads / g.n_kv, inv_sqrt, st));
@@ -2009,9 +2041,9 @@ static int lg_attn_core(bool q4, const void *wq, const void *wk, const void *wv,
         const int abpr = g.q_dim() / tg::LG_QK;
         PROFILED("lg_quant", st, tg::launch_quantize_q8k(b.ao, b.aq, abpr, st));
         PROFILED("lg_q4k_attn", st,
-                 tg::launch_matmul_q4k(static_cast<const uint8_t *>(wo), b.aq, b.out, g.embed, abpr, st));
+                 tg::launch_matmul_q4k(static_cast<const uint8_t *>(wo), b.aq, out, g.embed, abpr, st));
     } else {
-        PROFILED("lg_f32", st, tg::launch_matvec_two_acc(wo, false, b.ao, b.out, g.embed, g.q_dim(), st));
+        PROFILED("lg_f32", st, tg::launch_matvec_two_acc(wo, false, b.ao, out, g.embed, g.q_dim(), st));
     }
     return TG_OK;
 }
@@ -2053,10 +2085,10 @@ static int lg_attention(bool q4, const void *wq, const void *wk, const void *wv,
         const float *pqn, *pkn;
         if ((rc = lg_in(wq, bq, dq, &pq)) || (rc = lg_in(wk, bk, dk, &pk)) || (rc = lg_in(wv, bv, dv, &pv)) ||
             (rc = lg_in(wo, bo, dwo, &po)) || (rc = lg_in(qnw, nb, dqn, &pqn)) || (rc = lg_in(knw, nb, dkn, &pkn)) ||
-            (rc = lg_h2d(b.x, input, 4 * (size_t)g.embed)) || (rc = lg_attn_in(g, b, kv_k, kv_v, rope_cos, rope_sin)) ||
-            (rc = lg_attn_core(q4, pq, pk, pv, po, pqn, pkn, g, b)) || (rc = lg_attn_out(g, b, kv_k, kv_v)))
+            (rc = lg_h2d(b.x, input, 4 * (size_t)g.embed)) || (rc = lg_rope_in(g, b, rope_cos, rope_sin)) ||
+            (rc = lg_attn_core(q4, pq, pk, pv, po, pqn, pkn, g, b, kv_k, kv_v, b.ret)))
             return rc;
-        return lg_finish(output, b.out, 4 * (size_t)g.embed);
+        return lg_attn_finish(g, b, output, kv_k, kv_v);
     }
     return TG_OK;
 }
@@ -2118,7 +2150,7 @@ static int lg_transformer_layer(const float *wq, const float *wk, const float *w
         uint8_t *dq = c.take<uint8_t>(bq), *dk = c.take<uint8_t>(bk), *dv = c.take<uint8_t>(bv);
         uint8_t *dwo = c.take<uint8_t>(bo);
         float *dqn = c.take<float>(nb), *dkn = c.take<float>(nb), *dan = c.take<float>(ev), *dfn = c.take<float>(ev);
-        float *dx = c.take<float>(ev), *dmo = c.take<float>(ev);
+        float *dmo = c.take<float>(moe_all ? 0 : ev);
         // one expert's staging (the per-expert loop)
         uint8_t *dg = c.take<uint8_t>(moe_all ? 0 : gb), *du = c.take<uint8_t>(moe_all ? 0 : gb);
         uint8_t *dd = c.take<uint8_t>(moe_all ? 0 : dbmax);
@@ -2132,6 +2164,7 @@ static int lg_transformer_layer(const float *wq, const float *wk, const float *w
             continue;
         }
         hipStream_t st = g_lg_st;
+        float *dx = b.ret;  // x, updated in place
         int rc;
         const uint8_t *pq, *pk, *pv, *po;
         const float *pqn, *pkn, *pan, *pfn;
@@ -2139,17 +2172,16 @@ static int lg_transformer_layer(const float *wq, const float *wk, const float *w
             (rc = lg_in(wo, bo, dwo, &po)) || (rc = lg_in(q_norm_w, nb, dqn, &pqn)) ||
             (rc = lg_in(k_norm_w, nb, dkn, &pkn)) || (rc = lg_in(attn_norm_w, ev, dan, &pan)) ||
             (rc = lg_in(ffn_norm_w, ev, dfn, &pfn)) || (rc = lg_h2d(dx, x, ev)) ||
-            (rc = lg_attn_in(g, b, kv_k, kv_v, rope_cos, rope_sin)))
+            (rc = lg_rope_in(g, b, rope_cos, rope_sin)))
             return rc;
         PROFILED("lg_rms", st, tg::launch_rms_norm(dx, pan, b.x, embed, 1e-6f, st));
-        if ((rc = lg_attn_core(false, pq, pk, pv, po, pqn, pkn, g, b))) return rc;
-        PROFILED("lg_add", st, tg::launch_add_vec(dx, b.out, embed, st));
-        PROFILED("lg_rms", st, tg::launch_rms_norm(dx, pfn, b.x, embed, 1e-6f, st));
+        if ((rc = lg_attn_core(false, pq, pk, pv, po, pqn, pkn, g, b, kv_k, kv_v, b.out))) return rc;
+        PROFILED("lg_rms", st, tg::launch_add_rms_norm(dx, b.out, pfn, b.x, embed, 1e-6f, st));
         if (moe_all) {
             tg::LgMoeOps P;
             if ((rc = lg_moe_ops(n_active, gate_ptrs, up_ptrs, down_ptrs, expert_weights, gb, down_bytes(0, embed, inter),
                                  mb.stage, P)) ||
-                (rc = lg_moe_run(P, n_active, b.x, dmo, embed, inter, eb, mb)))
+                (rc = lg_moe_run(P, n_active, b.x, dx, embed, inter, eb, mb, tg::LG_DOWN_ADD)))
                 return rc;
         } else {
             HIP_TRY(hipMemsetAsync(dmo, 0, ev, st));  // moe_out starts at zero
@@ -2162,10 +2194,9 @@ static int lg_transformer_layer(const float *wq, const float *wk, const float *w
                     (rc = lg_expert(pg, pu, pd, fmt, b.x, dmo, expert_weights[e], embed, inter, eb)))
                     return rc;
             }
+            PROFILED("lg_add", st, tg::launch_add_vec(dx, dmo, embed, st));
         }
-        PROFILED("lg_add", st, tg::launch_add_vec(dx, dmo, embed, st));
-        if ((rc = lg_attn_out(g, b, kv_k, kv_v))) return rc;
-        return lg_finish(x, dx, ev);
+        return lg_attn_finish(g, b, x, kv_k, kv_v);
     }
     return TG_OK;
 }

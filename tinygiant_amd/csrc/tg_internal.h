@@ -155,14 +155,26 @@ bool moe_q4k_ok(int n_exp, int embed, int inter);
 hipError_t launch_moe_gateup_q4k(const LgMoeOps &P, int n_exp, const float *x, float *gu, int embed, int inter,
                                  hipStream_t st);
 hipError_t launch_moe_silu_q8k(const float *gu, void *hq, int n_exp, int inter, hipStream_t st);
+// out = sum over the experts (SET), out + each expert in turn (ACC), or out + the
+// finished sum (ADD)
+enum LgDownOut { LG_DOWN_SET, LG_DOWN_ACC, LG_DOWN_ADD };
 hipError_t launch_moe_down_acc_q4k(const LgMoeOps &P, int n_exp, const void *hq, float *out, int embed, int inter,
-                                   bool add_to_out,
-                                   hipStream_t st);
-hipError_t launch_rms_norm_rows(const float *x, const float *w, float *out, int dim, int rows, float eps,
-                                hipStream_t st);
-hipError_t launch_rope(float *x, int n_heads, int hd, const float *c, const float *sn, hipStream_t st);
-hipError_t launch_kv_append(const float *kn, const float *v, float *kc, float *vc, int n_kv, int seq, int hd, int row,
-                            hipStream_t st);
+                                   LgDownOut mode, hipStream_t st);
+// x += add, then the norm of x
+hipError_t launch_add_rms_norm(float *x, const float *add, const float *w, float *out, int dim, float eps,
+                               hipStream_t st);
+// the matrices of one k_matvec_two_acc launch; b0[m]: the first block of matrix m
+struct MvMats {
+    const void *A[3];
+    float *y[3];
+    int rows[3], b0[3];
+};
+hipError_t launch_matvec3_f32(const float *const (&A)[3], float *const (&y)[3], const int (&rows)[3], const float *x,
+                              int ncols, hipStream_t st);
+// norm, rotation and cache rows of the new position; kvn: 2 * n_kv * hd floats, the new keys then values
+hipError_t launch_head_prep(const float *q, const float *k, const float *v, const float *qw, const float *kw,
+                            const float *cs, const float *sn, float *qn, float *kc, float *vc, float *kvn, int n_heads,
+                            int n_kv, int seq, int hd, int row, float eps, hipStream_t st);
 // Attention of n_heads query heads over seq cached positions, caches
 // [n_kv][seq][hd] (ratio = n_heads / n_kv query heads per kv head), hd <= 512,
 // in three launches: scores and per-block maxima, the softmax weights of each

@@ -312,10 +312,11 @@ TG_DEV const uint8_t *pick_expert(const uint8_t *const (&t)[LG_MOE_MAX], int n, 
 // one output row per wave: the sequence of its n_exp * dbpr blocks (expert
 // by expert), each expert's row value added as acc + w * value when its last
 // block is in
-// (acc starts at out[r] when add_to_out: expert_forward's out += w * down)
+// (acc starts at out[r] when add_to_out: expert_forward's out += w * down; from
+// zero and added to out[r] at the end when add_last: the layer's x += moe)
 __global__ __launch_bounds__(256) void k_moe_down_acc_q4k(const LgMoeOps P, const Q8K *__restrict__ hq,
                                                           float *__restrict__ out, int n_exp, int embed, int dbpr,
-                                                          int add_to_out) {
+                                                          int add_to_out, int add_last) {
     const int lane = threadIdx.x & 63, r = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
     if (r >= embed) return;  // uniform over the wave
     const int j4 = lane >> 2, g = lane & 3, nblk = n_exp * dbpr;
@@ -346,7 +347,7 @@ __global__ __launch_bounds__(256) void k_moe_down_acc_q4k(const LgMoeOps P, cons
             }
         }
     }
-    if (lane == 0) out[r] = acc;
+    if (lane == 0) out[r] = add_last ? out[r] + acc : acc;
 }
 
 // --------------------------------------------------------------- Q6_K dot
@@ -464,11 +465,17 @@ __global__ __launch_bounds__(256) void k_matmul_q6k(const uint8_t *__restrict__ 
 // load makes the compiler wait for it in place); clamped steps are not added.
 constexpr int MV_D = 16, MV_XS = 8192;
 
+// Up to three matrices of the same ncols times the same x in one launch (q, k
+// and v: two 512-row launches of 7.9 us each join the 4096-row one); matrix m's
+// blocks start at M.b0[m].
 template <bool HALF>
-__global__ __launch_bounds__(256) void k_matvec_two_acc(const void *__restrict__ A, const float *__restrict__ x,
-                                                        float *__restrict__ y, int nrows, int ncols) {
+__global__ __launch_bounds__(256) void k_matvec_two_acc(const MvMats M, const float *__restrict__ x, int ncols) {
     __shared__ float xs[MV_XS];
-    const int tid = threadIdx.x, c = tid & 7, row = (blockIdx.x * 256 + tid) >> 3;
+    const int m = (int)blockIdx.x < M.b0[1] ? 0 : (int)blockIdx.x < M.b0[2] ? 1 : 2;  // uniform
+    const void *__restrict__ A = M.A[m];
+    float *__restrict__ y = M.y[m];
+    const int nrows = M.rows[m];
+    const int tid = threadIdx.x, c = tid & 7, row = (((int)blockIdx.x - M.b0[m]) * 256 + tid) >> 3;
     const bool on = row < nrows;
     const int n8 = ncols & ~7;
     auto wat = [&](size_t i) -> float {
@@ -535,21 +542,24 @@ __global__ __launch_bounds__(256) void k_matvec_two_acc(const void *__restrict__
 // --------------------------------------------------------------- RMS norm
 // tg_rms_norm, libtinygiant.c:322-340: four fma chains of squares over
 // steps of 4, ss = (v0 + v1) + (v2 + v3), the tail one product and add at a
-// time, scale = 1 / sqrt(ss / dim + eps), out = (x * scale) * w.  One block
-// per row (row b at x + b * dim, the same weight w).  The row passes
+// time, scale = 1 / sqrt(ss / dim + eps), out = (x * scale) * w.  One block.
+// The row passes
 // through LDS in chunks of 4096 values, loaded by all threads with their
 // loads in flight together, so the four chains (threads 0-3) read LDS
 // rather than wait on a global load per step.
 constexpr int RMS_CH = 4096;
 
-__global__ __launch_bounds__(256) void k_rms_norm(const float *__restrict__ x, const float *__restrict__ w,
+// add: first x[i] += add[i] (the residual, libtinygiant.c:682), written back.
+__global__ __launch_bounds__(256) void k_rms_norm(float *x, const float *__restrict__ add, const float *__restrict__ w,
                                                   float *__restrict__ out, int dim, float eps) {
     __shared__ float xs[RMS_CH];
     __shared__ float v[4];
     __shared__ float scale;
     const int tid = threadIdx.x, n4 = dim & ~3;
-    x += (size_t)blockIdx.x * dim;
-    out += (size_t)blockIdx.x * dim;
+    if (add) {  // (one row; every thread reads below what it wrote or, past a barrier, LDS)
+        for (int i = tid; i < dim; i += 256) x[i] = x[i] + add[i];
+        __syncthreads();
+    }
     float a = 0.0f;
     for (int c0 = 0; c0 < n4; c0 += RMS_CH) {
         const int n = min(RMS_CH, n4 - c0);
@@ -624,32 +634,67 @@ __global__ __launch_bounds__(256) void k_acc_scaled(float *__restrict__ out, con
 }
 
 // -------------------------------------------------------------- attention
-// apply_rope_inplace, libtinygiant.c:344-361, at one position (c, s: the
-// tables' row): x1' = x1 c - x2 s (products rounded, then the difference:
-// vmlsq_f32), x2' = fma(x1, s, x2 c) (vfmaq_f32 on the rounded x2 c).  One
-// thread per pair (head h, i < half).
-__global__ __launch_bounds__(256) void k_rope(float *__restrict__ x, int n_heads, int hd, const float *__restrict__ c,
-                                              const float *__restrict__ sn) {
-    const int half = hd / 2, p = blockIdx.x * 256 + threadIdx.x;
-    if (p >= n_heads * half) return;
-    const int h = p / half, i = p - h * half;
-    float *xh = x + (size_t)h * hd;
-    const float x1 = xh[i], x2 = xh[half + i];
-    const float a = x1 * c[i], b = x2 * sn[i];
-    xh[i] = a - b;
-    xh[half + i] = __builtin_fmaf(x1, sn[i], x2 * c[i]);
-}
-
-// The new key and value rows into the caches [n_kv][seq][hd] at row `row`
-// (libtinygiant.c:395-401).
-__global__ __launch_bounds__(256) void k_kv_append(const float *__restrict__ kn, const float *__restrict__ v,
-                                                   float *__restrict__ kc, float *__restrict__ vc, int n_kv, int seq,
-                                                   int hd, int row) {
-    const int p = blockIdx.x * 256 + threadIdx.x;
-    if (p >= n_kv * hd) return;
-    const int h = p / hd, d = p - h * hd;
-    kc[((size_t)h * seq + row) * hd + d] = kn[p];
-    vc[((size_t)h * seq + row) * hd + d] = v[p];
+// The new position's heads before the attention, one block each: a query head
+// (blocks [0, n_heads)) or key head (the next n_kv) is RMS-normalised in
+// tg_rms_norm's order (four fma chains, :322-340) and rotated in pairs
+// (apply_rope_inplace, libtinygiant.c:344-361, at one position): x1 c - x2 s
+// (products rounded, then the difference), fma(x1, s, x2 c) on the rounded x2 c; keys and values (the
+// last n_kv blocks) go into the caches [n_kv][seq][hd] at row `row` (:395-401)
+// and, packed, to kvn (keys, then values) for the caller.  hd even, at most 512.
+// Five launches of 2.9-4.5 us each before.
+__global__ __launch_bounds__(128) void k_head_prep(const float *__restrict__ q, const float *__restrict__ k,
+                                                   const float *__restrict__ v, const float *__restrict__ qw,
+                                                   const float *__restrict__ kw, const float *__restrict__ cs,
+                                                   const float *__restrict__ sn, float *__restrict__ qn,
+                                                   float *__restrict__ kc, float *__restrict__ vc,
+                                                   float *__restrict__ kvn, int n_heads, int n_kv, int seq, int hd,
+                                                   int row, float eps) {
+    __shared__ float xs[512];
+    __shared__ float ch[4];
+    __shared__ float scale;
+    const int b = blockIdx.x, tid = threadIdx.x, n4 = hd & ~3, half = hd / 2;
+    if (b >= n_heads + n_kv) {
+        const int h = b - n_heads - n_kv;
+        for (int i = tid; i < hd; i += 128) {
+            const float f = v[(size_t)h * hd + i];
+            vc[((size_t)h * seq + row) * hd + i] = f;
+            kvn[(size_t)(n_kv + h) * hd + i] = f;
+        }
+        return;
+    }
+    const bool isq = b < n_heads;
+    const int h = isq ? b : b - n_heads;
+    const float *x = (isq ? q : k) + (size_t)h * hd, *w = isq ? qw : kw;
+    for (int i = tid; i < hd; i += 128) xs[i] = x[i];
+    __syncthreads();
+    if (tid < 4) {
+        float a = 0.0f;
+#pragma unroll 8
+        for (int i = tid; i < n4; i += 4) a = __builtin_fmaf(xs[i], xs[i], a);
+        ch[tid] = a;
+    }
+    __syncthreads();
+    if (tid == 0) {
+        float ss = (ch[0] + ch[1]) + (ch[2] + ch[3]);
+        for (int i = n4; i < hd; i++) ss = ss + xs[i] * xs[i];
+        scale = 1.0f / __builtin_sqrtf(ss / (float)hd + eps);
+    }
+    __syncthreads();
+    const float sc = scale;
+    for (int i = tid; i < half; i += 128) {
+        const float x1 = (xs[i] * sc) * w[i], x2 = (xs[half + i] * sc) * w[half + i];
+        const float a1 = x1 * cs[i], b1 = x2 * sn[i];
+        const float o1 = a1 - b1, o2 = __builtin_fmaf(x1, sn[i], x2 * cs[i]);
+        if (isq) {
+            qn[(size_t)h * hd + i] = o1;
+            qn[(size_t)h * hd + half + i] = o2;
+        } else {
+            kc[((size_t)h * seq + row) * hd + i] = o1;
+            kc[((size_t)h * seq + row) * hd + half + i] = o2;
+            kvn[(size_t)h * hd + i] = o1;
+            kvn[(size_t)h * hd + half + i] = o2;
+        }
+    }
 }
 
 // Attention over seq cached positions (libtinygiant.c:405-446), the head's
@@ -1081,22 +1126,41 @@ hipError_t launch_matmul_q6k(const uint8_t *W, const void *xq, float *y, int nro
 hipError_t launch_matvec_two_acc(const void *A, bool half, const float *x, float *y, int nrows, int ncols,
                                  hipStream_t st) {
     if (nrows <= 0) return hipSuccess;
+    const MvMats M = {{A, A, A}, {y, y, y}, {nrows, 0, 0}, {0, INT_MAX, INT_MAX}};
     const dim3 grid(lg_cdiv(nrows, 32));
     if (half)
-        TG_LAUNCH(k_matvec_two_acc<true>, grid, dim3(256), 0, st, A, x, y, nrows, ncols);
+        TG_LAUNCH(k_matvec_two_acc<true>, grid, dim3(256), 0, st, M, x, ncols);
     else
-        TG_LAUNCH(k_matvec_two_acc<false>, grid, dim3(256), 0, st, A, x, y, nrows, ncols);
+        TG_LAUNCH(k_matvec_two_acc<false>, grid, dim3(256), 0, st, M, x, ncols);
+    return hipGetLastError();
+}
+
+hipError_t launch_matvec3_f32(const float *const (&A)[3], float *const (&y)[3], const int (&rows)[3], const float *x,
+                              int ncols, hipStream_t st) {
+    if (rows[0] <= 0 || rows[1] <= 0 || rows[2] <= 0) return hipErrorInvalidValue;
+    MvMats M;
+    int b = 0;
+    for (int m = 0; m < 3; m++) {
+        M.A[m] = A[m];
+        M.y[m] = y[m];
+        M.rows[m] = rows[m];
+        M.b0[m] = b;
+        b += (int)lg_cdiv(rows[m], 32);
+    }
+    TG_LAUNCH(k_matvec_two_acc<false>, dim3(b), dim3(256), 0, st, M, x, ncols);
     return hipGetLastError();
 }
 
 hipError_t launch_rms_norm(const float *x, const float *w, float *out, int dim, float eps, hipStream_t st) {
-    return launch_rms_norm_rows(x, w, out, dim, 1, eps, st);
+    if (dim <= 0) return hipSuccess;
+    TG_LAUNCH(k_rms_norm, dim3(1), dim3(256), 0, st, const_cast<float *>(x), (const float *)nullptr, w, out, dim, eps);
+    return hipGetLastError();
 }
 
-hipError_t launch_rms_norm_rows(const float *x, const float *w, float *out, int dim, int rows, float eps,
-                                hipStream_t st) {
-    if (dim <= 0 || rows <= 0) return hipSuccess;
-    TG_LAUNCH(k_rms_norm, dim3(rows), dim3(256), 0, st, x, w, out, dim, eps);
+hipError_t launch_add_rms_norm(float *x, const float *add, const float *w, float *out, int dim, float eps,
+                               hipStream_t st) {
+    if (dim <= 0) return hipSuccess;
+    TG_LAUNCH(k_rms_norm, dim3(1), dim3(256), 0, st, x, add, w, out, dim, eps);
     return hipGetLastError();
 }
 
@@ -1112,17 +1176,12 @@ hipError_t launch_silu_mul_vec(const float *g, const float *u, float *h, int n, 
     return hipGetLastError();
 }
 
-hipError_t launch_rope(float *x, int n_heads, int hd, const float *c, const float *sn, hipStream_t st) {
-    const int n = n_heads * (hd / 2);
-    if (n <= 0) return hipSuccess;
-    TG_LAUNCH(k_rope, dim3(lg_cdiv(n, 256)), dim3(256), 0, st, x, n_heads, hd, c, sn);
-    return hipGetLastError();
-}
-
-hipError_t launch_kv_append(const float *kn, const float *v, float *kc, float *vc, int n_kv, int seq, int hd, int row,
-                            hipStream_t st) {
-    if (n_kv * hd <= 0) return hipSuccess;
-    TG_LAUNCH(k_kv_append, dim3(lg_cdiv((long)n_kv * hd, 256)), dim3(256), 0, st, kn, v, kc, vc, n_kv, seq, hd, row);
+hipError_t launch_head_prep(const float *q, const float *k, const float *v, const float *qw, const float *kw,
+                            const float *cs, const float *sn, float *qn, float *kc, float *vc, float *kvn, int n_heads,
+                            int n_kv, int seq, int hd, int row, float eps, hipStream_t st) {
+    if (n_heads <= 0 || n_kv <= 0 || hd <= 0 || hd % 2 || hd > 512) return hipErrorInvalidValue;
+    TG_LAUNCH(k_head_prep, dim3(n_heads + 2 * n_kv), dim3(128), 0, st, q, k, v, qw, kw, cs, sn, qn, kc, vc, kvn,
+              n_heads, n_kv, seq, hd, row, eps);
     return hipGetLastError();
 }
 
@@ -1198,10 +1257,10 @@ hipError_t launch_moe_silu_q8k(const float *gu, void *hq, int n_exp, int inter, 
 }
 
 hipError_t launch_moe_down_acc_q4k(const LgMoeOps &P, int n_exp, const void *hq, float *out, int embed, int inter,
-                                   bool add_to_out, hipStream_t st) {
+                                   LgDownOut mode, hipStream_t st) {
     if (!moe_q4k_ok(n_exp, embed, inter)) return hipErrorInvalidValue;
     TG_LAUNCH(k_moe_down_acc_q4k, dim3(lg_cdiv(embed, 4)), dim3(256), 0, st, P, static_cast<const Q8K *>(hq), out,
-              n_exp, embed, inter / LG_QK, add_to_out ? 1 : 0);
+              n_exp, embed, inter / LG_QK, mode == LG_DOWN_ACC ? 1 : 0, mode == LG_DOWN_ADD ? 1 : 0);
     return hipGetLastError();
 }
 
