@@ -196,7 +196,7 @@ def test_head_sample(O, tglib):
 
 @pytest.mark.parametrize("V", [1023, 1024, 1025, 1032, 8191, 9215, 9216, 9217, 12288, 12289, 17408, 17409])
 def test_sample_ordered_sum_edges(tglib, sampler_factory, V):
-    """The parallel ordered sums at the edges of the one-wave head (1024 values) and of the block tiles (8192 after
+    """The parallel ordered sums at the edges of the one-wave head (1024 values) and of the block tiles (16384 after
     it): every token a candidate, tied values (ties to even on half ulps), spread and nearly equal ones."""
     gpu_note(f"tg_sampler_run ordered sums V={V}")
     s = sampler_factory(V)

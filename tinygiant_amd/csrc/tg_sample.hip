@@ -183,10 +183,10 @@ TG_DEV float block_pw_sum(const float *v, int n, PwTree &t) {
 // first lane whose sum reaches 2^(e+1) still ends on the true sum (it made
 // every addition itself); the lanes after it are scanned again from that sum,
 // once per binade.  v_k <= v_0 <= s throughout; pairs past a crossing may be
-// inexact and are not used.  The same 151,936 values now take 36 us (fp32 cut)
-// and 72 us (float64 draw): one block, bound by its additions and 19 tiles of
-// two barriers each.  (Values loaded one dword at a time instead of two float4
-// per lane: 95 and 113 us.  Ulps counted as 64-bit integers: 166 and 192 us.)
+// inexact and are not used.  The same 151,936 values now take 25 us (fp32 cut)
+// and 56 us (float64 draw): one block, bound by its additions and 10 tiles of
+// two barriers each.  (With 8 values per lane 36 and 72 us, loaded one dword at a
+// time instead of by float4 95 and 113 us.  Ulps counted as 64-bit integers: 166 and 192 us.)
 template <class F> struct Grid;  // the sum's binade as 2^e, its ulp, a value's parity in ulps
 template <> struct Grid<float> {
     TG_DEV static float binade(float s) { return __uint_as_float(__float_as_uint(s) & 0x7F800000u); }
@@ -234,7 +234,9 @@ template <class F> TG_DEV Hop<F> hop_scan(F c, Hop<F> v) {
     return v;
 }
 
-constexpr int ORD_R = 8;        // values per lane and scan
+// values per lane and scan: by a block (8: cut 36, draw 72 us instead of 25 and
+// 56 at 151,936 values), by one wave (which scans its values once per binade)
+constexpr int ORD_R = 16, ORD_R1 = 8;
 constexpr int ORD_NW = 16;      // waves of a block scan
 constexpr int ORD_HEAD = 1024;  // values summed by one wave first (most of the binades lie there)
 constexpr int ORD_TILE = ORD_NW * WAVE * ORD_R;
@@ -250,43 +252,45 @@ struct OrdLds {
     double log[ORD_LOG];    // the sum before each tile
 };
 
-// Continues the running sum s of the values before pos (a multiple of 8; at 0,
+// Continues the running sum s of the values before pos (a multiple of 16; at 0,
 // s = v[0] and the sum goes on from v[1]) over v[pos..n) (each divided by div
 // when DIV), by NW waves (NW == 1: any one wave; else the whole block of ORD_NW
-// waves).  v is 16-byte aligned and readable to the next multiple of 8 values.
+// waves).  v is 16-byte aligned and readable to the next multiple of 16 values.
 // Returns the first index whose running sum satisfies pred (monotone), or -1
 // with s the sum of all.  log: the sum before each tile.
 template <class F, int NW, bool DIV, class Pred>
 TG_DEV int ord_run(const float *v, float div, int n, int pos, F &s, Pred pred, OrdLds &L, double *log) {
-    constexpr int TILE = NW * WAVE * ORD_R;
-    const int lane = __lane_id(), w = NW == 1 ? 0 : (int)threadIdx.x / WAVE, slot = (w * WAVE + lane) * ORD_R;
-    float raw[ORD_R];
-    F x[ORD_R];
-    // two 16-byte loads, unconditional (at the last group of 8 past the end,
-    // whose values are not used), so that they stay in flight during a scan
+    constexpr int R = NW == 1 ? ORD_R1 : ORD_R, TILE = NW * WAVE * R;
+    const int lane = __lane_id(), w = NW == 1 ? 0 : (int)threadIdx.x / WAVE, slot = (w * WAVE + lane) * R;
+    float raw[R];
+    F x[R];
+    // 16-byte loads, unconditional (at the last group past the end, whose
+    // values are not used), so that they stay in flight during a scan
     auto load = [&](int p0) {
-        const float4 *g = reinterpret_cast<const float4 *>(v + min(p0 + slot, (n - 1) & ~(ORD_R - 1)));
-        const float4 a = g[0], b = g[1];
-        raw[0] = a.x; raw[1] = a.y; raw[2] = a.z; raw[3] = a.w;
-        raw[4] = b.x; raw[5] = b.y; raw[6] = b.z; raw[7] = b.w;
+        const float4 *g = reinterpret_cast<const float4 *>(v + min(p0 + slot, (n - 1) & ~(R - 1)));
+#pragma unroll
+        for (int q = 0; q < R / 4; q++) {
+            const float4 f = g[q];
+            raw[4 * q] = f.x; raw[4 * q + 1] = f.y; raw[4 * q + 2] = f.z; raw[4 * q + 3] = f.w;
+        }
     };
     load(pos);
     for (; pos < n; pos += TILE) {
 #pragma unroll
-        for (int j = 0; j < ORD_R; j++) {
+        for (int j = 0; j < R; j++) {
             const int i = pos + slot + j;
             const float q = DIV ? raw[j] / div : raw[j];
             x[j] = i > 0 && i < n ? (F)q : (F)0;
         }
         load(pos + TILE);
         if (NW > 1 && log && threadIdx.x == 0) *log++ = (double)s;
-        const int end = min(pos + slot + ORD_R, n);  // of this lane's run
+        const int end = min(pos + slot + R, n);  // of this lane's run
         for (;;) {
             // x: this tile's values not yet in s (those that are, and past n: 0)
             const F c = Grid<F>::binade(s), c1 = c + c * Grid<F>::ULP;
             F a0 = c, a1 = c1;
 #pragma unroll
-            for (int j = 0; j < ORD_R; j++) {
+            for (int j = 0; j < R; j++) {
                 a0 = a0 + x[j];
                 a1 = a1 + x[j];
             }
@@ -302,7 +306,7 @@ TG_DEV int ord_run(const float *v, float div, int n, int pos, F &s, Pred pred, O
             const F sl = s + (Grid<F>::odd(s) ? ex.d1 : ex.d0);
             F se = sl;
 #pragma unroll
-            for (int j = 0; j < ORD_R; j++) se = se + x[j];
+            for (int j = 0; j < R; j++) se = se + x[j];
             const uint64_t m = __ballot(se >= c + c || pred(se));
             int first = WAVE - 1, at = INT_MAX, hit = -1;
             if (m) {
@@ -311,12 +315,12 @@ TG_DEV int ord_run(const float *v, float div, int n, int pos, F &s, Pred pred, O
                 F r = sl;
                 int k = 0;
 #pragma unroll
-                for (int j = 0; j < ORD_R; j++) {
+                for (int j = 0; j < R; j++) {
                     r = r + x[j];
                     k += pred(r) ? 0 : 1;
                 }
                 k = __builtin_amdgcn_readlane(k, first);
-                if (k < ORD_R) hit = pos + (w * WAVE + first) * ORD_R + k;
+                if (k < R) hit = pos + (w * WAVE + first) * R + k;
             }
             F sn = rdl(se, first);
             if (NW > 1) {
@@ -332,7 +336,7 @@ TG_DEV int ord_run(const float *v, float div, int n, int pos, F &s, Pred pred, O
             if (at == INT_MAX) break;  // the whole tile is in s
             if (hit >= 0) return hit;
 #pragma unroll
-            for (int j = 0; j < ORD_R; j++)
+            for (int j = 0; j < R; j++)
                 if (end <= at) x[j] = (F)0;
         }
     }
