@@ -319,7 +319,7 @@ hipError_t launch_place(const int32_t *idx, int n, int E, int cap, int32_t *ecnt
 // clears ecnt for the next call
 hipError_t launch_group_placed(const Shape &s, int n, int ch, int cap, int32_t *ecnt, int32_t *counts,
                                int32_t *offsets, int32_t *work, int32_t *work_n, int32_t *rdy, hipStream_t st);
-// int8-MFMA grouped gate/up and down (mt = M-tiles of 32 entries per item)
+// int8-MFMA grouped gate/up and down (mt = M-tiles of 32 entries per item; 0: items of 16)
 bool mfma_shape_ok(const Shape &s);
 int mfma_tiles(const Shape &s, int T);
 // entries per work item for the MFMA launches at mt M-tiles
