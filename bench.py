@@ -1180,15 +1180,15 @@ def run_legacy_layer(args, torch, call):
     for _ in range(4):
         step()
     call("tg_prof_enable", 0)
-    kern = kernel_times(call, ("lg_f32", "lg_rms", "lg_rope", "lg_kv", "lg_attn_sc", "lg_attn_sm", "lg_attn", "lg_add",
+    kern = kernel_times(call, ("lg_f32", "lg_rms", "lg_heads", "lg_attn_sc", "lg_attn_sm", "lg_attn", "lg_add",
                                "lg_quant", "lg_q4k", "lg_silu", "lg_q4k_down", "lg_acc", "lg_moe_gateup",
                                "lg_moe_silu", "lg_moe_down"))
     kern_us = {k: round(v[1] / max(v[0], 1) * 1e3, 3) for k, v in kern.items()}
     # dominant kernel: the f32 q / k / v / o projections (k_matvec_two_acc),
-    # bytes per launch = weights + input averaged over the four launches
+    # bytes per launch = weights + input averaged over its two launches (q, k and v; o)
     n_f, ms_f = kern["lg_f32"]
     proj_shapes = ((Hh * hd, H), (KV * hd, H), (KV * hd, H), (H, Hh * hd))
-    proj_bytes = sum(4 * (r * c + c + r) for r, c in proj_shapes) / len(proj_shapes)
+    proj_bytes = sum(4 * (r * c + c + r) for r, c in proj_shapes) / 2
     achieved = proj_bytes / (ms_f / n_f * 1e-3)
     # attention proper: scores, softmax weights, weighted sum of V
     attn_bytes = 2 * KV * (kv_len + 1) * hd * 4  # the K and V cache rows, each read once
