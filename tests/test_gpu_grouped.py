@@ -287,10 +287,10 @@ def test_fused_gate_up_down_across_calls(O, tglib, H, I, E, k, Ts):
         a.close()
 
 
-# mean entries per expert on both sides of the one-tile / 16 x 16 line (24) and of 16-entry items (12), odd counts; experts over several
-# one-tile items (16 experts, mean 24) and a shape the fused launches do not take (I 160: the 32 x 32 kernels)
-@pytest.mark.parametrize("H,I,E,k,T", [(2048, 768, 128, 8, 333), (2048, 768, 128, 8, 384), (2048, 768, 128, 8, 385), (2048, 768, 128, 8, 192), (2048, 768, 128, 8, 193),
-                                       (512, 256, 16, 4, 96), (512, 256, 16, 4, 97), (512, 256, 32, 8, 131),
+# mean entries per expert on both sides of the one-tile / 16 x 16 line (32) and of 16-entry items (12), odd counts; experts over several
+# one-tile items (16 experts, mean 32) and a shape the fused launches do not take (I 160: the 32 x 32 kernels)
+@pytest.mark.parametrize("H,I,E,k,T", [(2048, 768, 128, 8, 333), (2048, 768, 128, 8, 512), (2048, 768, 128, 8, 513), (2048, 768, 128, 8, 192), (2048, 768, 128, 8, 193),
+                                       (512, 256, 16, 4, 128), (512, 256, 16, 4, 129), (512, 256, 32, 8, 131),
                                        (256, 160, 16, 4, 150), (256, 160, 16, 4, 300)])
 def test_item_size_rule_edges(O, tglib, H, I, E, k, T):
     gpu_note(f"grouped layer at the item size rule's edges H={H} I={I} E={E} T={T}")

@@ -1403,10 +1403,10 @@ int mfma_item_entries(const Shape &s, int mt) {
 
 // Entries per expert in a work item, in M-tiles of 32 (0: 16 entries), from the
 // batch's mean entries per expert.  Where both fused gate/up + down launches take
-// the shape, the one-tile kernel up to a mean of 24 and the 16 x 16 kernel above
-// (30B shape, us a layer at 420 tokens 186, 184; 512 tokens 219, 199; 235B 420
-// tokens 599, 595).  Items of 16 entries let three blocks share a CU instead of
-// two: they pay once the gate/up blocks fill five a CU (30B 16 tokens 69 us, 73
+// the shape, the one-tile kernel up to a mean of 32 and the 16 x 16 kernel above
+// (us a layer, 30B shape: 420 tokens 173, 181; 512 tokens 201, 199; 640 tokens 236,
+// 211; 235B: 420 tokens 539, 611; 512 tokens 616, 648; 640 tokens 703, 701).
+// Items of 16 entries let three blocks share a CU instead of two: they pay once the gate/up blocks fill five a CU (30B 16 tokens 69 us, 73
 // with 16-entry items; 32 tokens 77, 75; 64 tokens 93, 84; 235B 8 tokens 122, 128;
 // 16 tokens 164, 152) and until experts with more than 16 entries, whose weights
 // they read twice, weigh more: a mean of 8, or 12 where K is at most 8 chunks (30B
@@ -1415,7 +1415,7 @@ int mfma_item_entries(const Shape &s, int mt) {
 int mfma_tiles(const Shape &s, int T) {
     const int avg = (T * s.k + s.E - 1) / s.E;
     if (mfma_item_entries(s, 4) > 128 && s.nbI % MF_KC == 0) {
-        if (avg > 24) return 4;
+        if (avg > 32) return 4;
         // experts that T tokens select, each missed by a token with chance 1 - k / E
         const double distinct = s.E * (1.0 - std::pow(1.0 - (double)s.k / s.E, T));
         const int gxg = (s.I + 63) / 64;
