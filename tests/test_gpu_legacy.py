@@ -330,3 +330,34 @@ def test_output_head(O, L, vocab, embed, case):
         assert ref_tok == 3
     if case == "nan":
         assert ref_tok == vocab // 2
+
+
+@pytest.mark.parametrize("embed,n_heads,n_kv,hd,kv_max,kv_len,inter,n",
+                         [(2048, 32, 4, 128, 64, 40, 768, 8), (256, 4, 2, 64, 8, 0, 256, 1),
+                          (768, 12, 4, 64, 20, 19, 512, 3)])
+def test_transformer_layer_q4k(O, L, embed, n_heads, n_kv, hd, kv_max, kv_len, inter, n):
+    """tg_transformer_layer with Q4_K experts only: all experts in one group of launches, the finished sum added to x."""
+    gpu_note(f"tg_transformer_layer, Q4_K experts, E={embed} I={inter} n={n} kv_len={kv_len}")
+    rng = np.random.default_rng(embed + n)
+    run_transformer_layer(O, L, rng, embed, n_heads, n_kv, hd, kv_max, kv_len, inter, [0] * n)
+
+
+def run_transformer_layer(O, L, rng, embed, n_heads, n_kv, hd, kv_max, kv_len, inter, fmts):
+    """One layer call on random operands against the oracle, x and both caches bit for bit."""
+    wq, wk, wv, wo, qn, kn, c, s, kv_k, kv_v, x = attn_case(rng, False, embed, n_heads, n_kv, hd, kv_max)
+    an, fn = (rng.normal(1.0, 0.1, embed).astype(np.float32) for _ in range(2))
+    n = len(fmts)
+    ex = [expert_operands(rng, embed, inter, f) for f in fmts]
+    ew = rng.dirichlet(np.ones(n)).astype(np.float32)
+    gx, gk, gv = x.copy(), kv_k.copy(), kv_v.copy()
+    arr = [(ctypes.c_void_p * n)(*[e[t].ctypes.data for e in ex]) for t in range(3)]
+    dif = np.array(fmts, np.int32)
+    L.tg_transformer_layer(ptr(wq), ptr(wk), ptr(wv), ptr(wo), ptr(an), ptr(qn), ptr(kn), ptr(fn), ptr(gk), ptr(gv),
+                           kv_len, kv_max, ptr(c), ptr(s), *arr, ptr(dif), ptr(ew), n, ptr(gx), embed, inter, n_heads,
+                           n_kv, hd, kv_len)
+    rx, rk, rv = x.copy(), kv_k.copy(), kv_v.copy()
+    O.transformer_layer(wq, wk, wv, wo, an, qn, kn, fn, rk, rv, kv_len, kv_max, c, s,
+                        *([e[t] for e in ex] for t in range(3)), fmts, ew, rx, embed, inter, n_heads, n_kv, hd, kv_len)
+    assert_exact(gx, rx, "transformer layer x")
+    assert np.array_equal(gk.view(np.uint32), rk.view(np.uint32)), "key cache"
+    assert np.array_equal(gv.view(np.uint32), rv.view(np.uint32)), "value cache"

@@ -312,15 +312,17 @@ TG_DEV const uint8_t *pick_expert(const uint8_t *const (&t)[LG_MOE_MAX], int n, 
 // one output row per wave: the sequence of its n_exp * dbpr blocks (expert
 // by expert), each expert's row value added as acc + w * value when its last
 // block is in
-// (acc starts at out[r] when add_to_out: expert_forward's out += w * down; from
-// zero and added to out[r] at the end when add_last: the layer's x += moe)
+// (acc starts at out[r] for LG_DOWN_ACC: expert_forward's out += w * down; from
+// zero and added to out[r] at the end for LG_DOWN_ADD: the layer's x += moe).
+// MODE is a template argument: with it and the reload of out[r] decided at run
+// time the eight-expert launch took 5.87 us instead of 5.65.
+template <LgDownOut MODE>
 __global__ __launch_bounds__(256) void k_moe_down_acc_q4k(const LgMoeOps P, const Q8K *__restrict__ hq,
-                                                          float *__restrict__ out, int n_exp, int embed, int dbpr,
-                                                          int add_to_out, int add_last) {
+                                                          float *__restrict__ out, int n_exp, int embed, int dbpr) {
     const int lane = threadIdx.x & 63, r = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
     if (r >= embed) return;  // uniform over the wave
     const int j4 = lane >> 2, g = lane & 3, nblk = n_exp * dbpr;
-    float acc = add_to_out ? out[r] : 0.0f, cur = 0.0f;
+    float acc = MODE == LG_DOWN_ACC ? out[r] : 0.0f, cur = 0.0f;
     int b = 0, e = 0;  // wave-uniform: the block within the expert's row, the expert
     for (int p0 = 0; p0 < nblk; p0 += 32) {
         Q4kGrp W[2];
@@ -347,7 +349,7 @@ __global__ __launch_bounds__(256) void k_moe_down_acc_q4k(const LgMoeOps P, cons
             }
         }
     }
-    if (lane == 0) out[r] = add_last ? out[r] + acc : acc;
+    if (lane == 0) out[r] = MODE == LG_DOWN_ADD ? out[r] + acc : acc;
 }
 
 // --------------------------------------------------------------- Q6_K dot
@@ -1259,8 +1261,15 @@ hipError_t launch_moe_silu_q8k(const float *gu, void *hq, int n_exp, int inter, 
 hipError_t launch_moe_down_acc_q4k(const LgMoeOps &P, int n_exp, const void *hq, float *out, int embed, int inter,
                                    LgDownOut mode, hipStream_t st) {
     if (!moe_q4k_ok(n_exp, embed, inter)) return hipErrorInvalidValue;
-    TG_LAUNCH(k_moe_down_acc_q4k, dim3(lg_cdiv(embed, 4)), dim3(256), 0, st, P, static_cast<const Q8K *>(hq), out,
-              n_exp, embed, inter / LG_QK, mode == LG_DOWN_ACC ? 1 : 0, mode == LG_DOWN_ADD ? 1 : 0);
+    const dim3 grid(lg_cdiv(embed, 4)), block(256);
+    const Q8K *h = static_cast<const Q8K *>(hq);
+    const int dbpr = inter / LG_QK;
+    if (mode == LG_DOWN_SET)
+        TG_LAUNCH(k_moe_down_acc_q4k<LG_DOWN_SET>, grid, block, 0, st, P, h, out, n_exp, embed, dbpr);
+    else if (mode == LG_DOWN_ACC)
+        TG_LAUNCH(k_moe_down_acc_q4k<LG_DOWN_ACC>, grid, block, 0, st, P, h, out, n_exp, embed, dbpr);
+    else
+        TG_LAUNCH(k_moe_down_acc_q4k<LG_DOWN_ADD>, grid, block, 0, st, P, h, out, n_exp, embed, dbpr);
     return hipGetLastError();
 }
 
