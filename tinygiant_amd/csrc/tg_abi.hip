@@ -1293,8 +1293,6 @@ static int lg_reserve(size_t bytes) {
     }
     g_lg_dev = dev;
     if (!g_lg_st) HIP_TRY(hipStreamCreateWithFlags(&g_lg_st, hipStreamNonBlocking));
-    if (!g_lg_kv_st) HIP_TRY(hipStreamCreateWithFlags(&g_lg_kv_st, hipStreamNonBlocking));
-    if (!g_lg_kv_ev) HIP_TRY(hipEventCreateWithFlags(&g_lg_kv_ev, hipEventDisableTiming));
     if (g_lg_pin_off || g_lg_kv_busy) {  // a call that failed before its closing wait left bounce slots taken
         int rc2 = lg_sync();
         if (rc2) return rc2;
@@ -1972,6 +1970,8 @@ static int lg_rope_in(const LgAttn &g, const LgAttnBufs &b, const float *rope_co
 static int lg_kv_in(const LgAttn &g, const LgAttnBufs &b, const float *kv_k, const float *kv_v) {
     const size_t row = 4 * (size_t)g.hd;
     if (g.kv_len <= 0) return TG_OK;
+    if (!g_lg_kv_st) HIP_TRY(hipStreamCreateWithFlags(&g_lg_kv_st, hipStreamNonBlocking));
+    if (!g_lg_kv_ev) HIP_TRY(hipEventCreateWithFlags(&g_lg_kv_ev, hipEventDisableTiming));
     g_lg_kv_busy = true;
     HIP_TRY(hipMemcpy2DAsync(b.kc, row * g.seq(), kv_k, row * g.kv_max, row * g.kv_len, g.n_kv, hipMemcpyHostToDevice,
                              g_lg_kv_st));
