@@ -293,8 +293,9 @@ int tg_arena_set_decode_path(tg_arena *a, int path);
  * GROUPED (the (token, slot) pairs grouped by expert, each selected
  * expert's weights read once per layer; int8 MFMA tiles), GROUPED_DOT (the
  * same grouping on packed int8 dot instructions), PER_TOKEN (every token
- * reads its own k experts), AUTO (GROUPED for n_tokens >= 2).  GROUPED and
- * GROUPED_DOT also serve a single token when asked for explicitly.  Every
+ * reads its own k experts), AUTO (PER_TOKEN for 2 and 3 tokens, GROUPED
+ * above).  GROUPED and GROUPED_DOT also serve a single token when asked for
+ * explicitly.  None of them needs a launch's blocks resident at once.  Every
  * path gives the same bytes. */
 #define TG_BATCH_AUTO 0
 #define TG_BATCH_GROUPED 1

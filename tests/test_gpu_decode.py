@@ -6,6 +6,8 @@ All must equal the oracle bit for bit, layer by layer and through a stack
 (with the routing of every layer), and must agree with each other when
 calls alternate on one arena (the tag generations of the exchange words
 carry over between paths)."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -224,8 +226,8 @@ def test_235b_shape_stack(O, tglib):
 @pytest.mark.parametrize("T", [2, 3])
 @pytest.mark.parametrize("H,I,E,k", [(2048, 768, 128, 8), (512, 256, 32, 8)])
 def test_few_tokens_match_oracle(O, tglib, H, I, E, k, T):
-    """Two and three tokens: one layer (routed launches after one prologue for both; the grouped path from three) with
-    and without routing outputs, a stack of three layers token by token, and the batch paths chosen by hand."""
+    """Two and three tokens: one layer with and without routing outputs, a stack of three layers, and the batch paths
+    chosen by hand."""
     from tinygiant_amd.arena import HBMExpertArena
     from tinygiant_amd.moe import MoEBlock
     gpu_note(f"few tokens H={H} I={I} E={E} T={T}")
@@ -258,5 +260,44 @@ def test_few_tokens_match_oracle(O, tglib, H, I, E, k, T):
         torch.cuda.synchronize()
         assert np.array_equal(got.cpu().numpy().view(np.uint32), y.astype(np.float32).view(np.uint32))
         assert tglib.tg_arena_status(a.handle) == 0
+    finally:
+        a.close()
+
+
+def launches(L, role):
+    n, ms = ctypes.c_int(0), ctypes.c_double(0.0)
+    assert L.tg_prof_read(role.encode(), ctypes.byref(n), ctypes.byref(ms)) == 0
+    return n.value
+
+
+@pytest.mark.parametrize("T", [2, 3])
+def test_few_tokens_need_no_resident_launch(O, tglib, T):
+    """Two and three tokens (layer and stack) run beside other work: no launch whose blocks must all be resident.  The
+    output may lie over input rows of later tokens, which are read before any is written."""
+    from tinygiant_amd.arena import HBMExpertArena
+    from tinygiant_amd.moe import MoEBlock
+    H, I, E, k, L = 512, 256, 32, 8, 2
+    gpu_note(f"few tokens, launches and overlapping output T={T}")
+    a = HBMExpertArena(L, E, H, I, k)
+    try:
+        layers = [O.synth_layer(127, l, H, I, E) for l in range(L)]
+        for l, (lb, r) in enumerate(layers):
+            a.load_layer(l, lb)
+            a.load_router(l, r)
+        x = O.synth_normal(127, O.stream_id(0, T, 4), 1.0, T * H).reshape(T, H)
+        ref = O.moe_layer(*layers[0], H, I, E, k, x)[0]
+        buf = torch.zeros(T + 1, H, device="cuda")
+        buf[:T] = torch.from_numpy(x).cuda()
+        assert tglib.tg_prof_enable(1) == 0
+        try:
+            assert tglib.tg_moe_layer_q40_dev(a.handle, 0, buf.data_ptr(), buf.data_ptr() + 4 * H, T, None, None, 1e-6,
+                                              torch.cuda.current_stream().cuda_stream) == 0
+            MoEBlock(a).step(torch.from_numpy(x).cuda())
+            torch.cuda.synchronize()
+            assert launches(tglib, "route") == 1 + L
+            assert launches(tglib, "layer") == 0 and launches(tglib, "dec_part") == 0
+        finally:
+            tglib.tg_prof_enable(0)
+        assert np.array_equal(buf[1:].cpu().numpy().view(np.uint32), ref.view(np.uint32))
     finally:
         a.close()

@@ -90,7 +90,7 @@ class HBMExpertArena:
         """GROUPED: tokens grouped by expert, each selected expert read once
         per layer, on int8 MFMA tiles; GROUPED_DOT: the same grouping on
         packed int8 dot instructions; PER_TOKEN: every token reads its own
-        experts; AUTO: GROUPED for two or more tokens."""
+        experts; AUTO: PER_TOKEN for two and three tokens, GROUPED for more."""
         call("tg_arena_set_batch_path", self.handle, int(path))
 
     def status(self) -> None:

@@ -526,10 +526,18 @@ static const float *router_of(tg_arena *a, int layer) {
 
 // One MoE block: raw router dots, gate/up (norm, routing and Q8_0 fused),
 // down + combine.  out = moe_out (resid NULL) or resid + moe_out.
+//
+// Two and three tokens read their own experts (routing, gate/up and down, three
+// launches for all of them) rather than grouped (four): us a layer of a stack,
+// 30B shape two tokens 24, grouped 47; three 31, 51; 235B 55, 76 and 77, 82; the
+// same order on 24 other shapes of 0.7 to 71 MB of experts a token.  From four
+// tokens it depends on the shape (235B five 109, 107).  The one-token launch, token
+// by token, takes 26 and 40, 57 and 85, and needs every one of its blocks resident.
+constexpr int PER_TOKEN_MAX = 3;
 static bool grouped_usable(tg_arena *a, int T) {
     if (a->batch_path == TG_BATCH_PER_TOKEN) return false;
     if (a->batch_path == TG_BATCH_GROUPED || a->batch_path == TG_BATCH_GROUPED_DOT) return tg::grouped_shape_ok(a->s);
-    return T >= 2 && tg::grouped_shape_ok(a->s);
+    return T > PER_TOKEN_MAX && tg::grouped_shape_ok(a->s);
 }
 
 // The MFMA kernels address activation rows with 32-bit offsets.
@@ -654,13 +662,11 @@ static int layer_kernels_grouped(tg_arena *a, const Scratch &c, int layer, const
     return TG_OK;
 }
 
-// Few tokens, one launch per token and layer that also routes (the default path
-// of one token where the shape allows it; of up to ROUTED_TOKENS unless a batch
-// path was chosen).
-constexpr int ROUTED_TOKENS = 3;
+// One token, one launch per layer that also routes (the default one-token
+// path where the shape allows it).
 static bool routed_usable(tg_arena *a, int T) {
-    return (T == 1 || (T <= ROUTED_TOKENS && a->batch_path == TG_BATCH_AUTO)) &&
-           (a->decode_path == TG_DECODE_AUTO || a->decode_path == TG_DECODE_ROUTED) && tg::layer_dec_ok(a->s, a->n_cu);
+    return T == 1 && (a->decode_path == TG_DECODE_AUTO || a->decode_path == TG_DECODE_ROUTED) &&
+           tg::layer_dec_ok(a->s, a->n_cu);
 }
 
 // One token, gate/up and down in one launch after a routing kernel.
@@ -674,74 +680,52 @@ static bool fused_usable(tg_arena *a, int T) {
 // j reads the partials buffer j % 2 and leaves the next layer's in the
 // other.  Layer j's top-k ids / weights go to idx + j * k_step (k_step 0:
 // every layer overwrites the same k entries).
-static int routed_layer_at(tg_arena *a, const Scratch &c, int l, int buf, const float *wr_next, int back,
-                           const float *x, float *out, const float *resid, float eps, int32_t *idx, float *w,
-                           hipStream_t st) {
-    const Shape &s = a->s;
-    const size_t half = tg::dec_part_floats(s) / 2;
-    PROFILED("layer", st,
-             tg::launch_layer_dec(a->experts + (size_t)l * s.LB, s, a->n_cu, x, norm_of(a, l),
-                                  c.dec_part + (size_t)buf * half, wr_next, c.dec_part + (size_t)(1 - buf) * half,
-                                  c.dec_hw, c.dec_ow, c.dec_ctl, (uint32_t)back, c.dec_err, resid, out, idx, w, eps,
-                                  st));
-    return TG_OK;
-}
-
 static int routed_layers(tg_arena *a, const Scratch &c, int l0, int n, const float *x, float *out, const float *resid, float eps,
                          int32_t *idx, float *w, int k_step, hipStream_t st) {
     const Shape &s = a->s;
-    PROFILED("dec_part", st, tg::launch_dec_part(router_of(a, l0), x, s, 1, c.dec_part, c.dec_ctl, n, st));
+    const size_t half = tg::dec_part_floats(s) / 2;
+    PROFILED("dec_part", st, tg::launch_dec_part(router_of(a, l0), x, s, c.dec_part, c.dec_ctl, n, st));
     for (int j = 0; j < n; j++) {
-        int rc = routed_layer_at(a, c, l0 + j, j & 1, j + 1 < n ? router_of(a, l0 + j + 1) : nullptr, n - 1 - j,
-                                 j == 0 ? x : out, out, j == 0 ? resid : out, eps, idx + (size_t)j * k_step,
-                                 w + (size_t)j * k_step, st);
-        if (rc) return rc;
+        const int l = l0 + j;
+        const float *wr_next = j + 1 < n ? router_of(a, l + 1) : nullptr;
+        PROFILED("layer", st,
+                 tg::launch_layer_dec(a->experts + (size_t)l * s.LB, s, a->n_cu, j == 0 ? x : out, norm_of(a, l),
+                                      c.dec_part + (size_t)(j & 1) * half, wr_next,
+                                      c.dec_part + (size_t)((j + 1) & 1) * half, c.dec_hw, c.dec_ow, c.dec_ctl,
+                                      (uint32_t)(n - 1 - j), c.dec_err, j == 0 ? resid : out, out,
+                                      idx + (size_t)j * k_step, w + (size_t)j * k_step, eps, st));
     }
     return TG_OK;
 }
 
-// One or two tokens through one layer on the routed path, one launch each after
-// one prologue for both (token t's partials in buffer t).  The grouped path's
-// four launches only pay from three tokens (30B / 235B shape, us a layer: two
-// tokens 47 / 80 grouped, 27 / 59 routed; three 50 / 83 grouped).
-static int routed_tokens(tg_arena *a, const Scratch &c, int layer, const float *x, float *out, const float *resid,
-                         int T, float eps, int32_t *idx, float *w, hipStream_t st) {
-    const Shape &s = a->s;
-    PROFILED("dec_part", st, tg::launch_dec_part(router_of(a, layer), x, s, T, c.dec_part, c.dec_ctl, T, st));
-    for (int t = 0; t < T; t++) {
-        const size_t o = (size_t)t * s.H, ko = (size_t)t * s.k;
-        int rc = routed_layer_at(a, c, layer, t, nullptr, T - 1 - t, x + o, out + o, resid ? resid + o : nullptr, eps,
-                                 idx + ko, w + ko, st);
-        if (rc) return rc;
-    }
-    return TG_OK;
-}
-
-// idx_out / w_out: the caller's copies of the routing, or null
+// idx_out / w_out: where the caller wants the routing, or null
 static int layer_kernels(tg_arena *a, const Scratch &c, int layer, const float *x, float *out, const float *resid, int T, float eps,
                          int32_t *idx_out, float *w_out, hipStream_t st) {
-    if (routed_usable(a, T) && T <= 2 && !(T == 1 && grouped_usable(a, T))) {
-        // the routing goes to the caller's arrays, or to the scratch the host entry points read
-        const bool own = idx_out && w_out;
-        int rc = routed_tokens(a, c, layer, x, out, resid, T, eps, own ? idx_out : c.idx, own ? w_out : c.w, st);
-        if (rc || own) return rc;
-    } else if (grouped_usable(a, T)) {
-        return layer_kernels_grouped(a, c, layer, x, out, resid, T, eps, idx_out, w_out, st);
+    if (grouped_usable(a, T)) return layer_kernels_grouped(a, c, layer, x, out, resid, T, eps, idx_out, w_out, st);
+    // the routing goes to the caller's arrays, or to the scratch that the host entry points read (the
+    // kernels after it read it there; two copies behind them took about 5 us)
+    const bool own = idx_out && w_out;
+    int32_t *idx = own ? idx_out : c.idx;
+    float *w = own ? w_out : c.w;
+    if (routed_usable(a, T)) {
+        int rc = routed_layers(a, c, layer, 1, x, out, resid, eps, idx, w, 0, st);
+        if (rc) return rc;
     } else {
         const Shape &s = a->s;
         const uint8_t *lp = a->experts + (size_t)layer * s.LB;
         PROFILED("route", st,
                  tg::launch_route_dec(router_of(a, layer), x, norm_of(a, layer), T, s, eps, c.dec_lw, c.dec_ctl,
-                                      c.dec_err, c.idx, c.w, c.xq, c.xd, c.xs, st));
+                                      c.dec_err, idx, w, c.xq, c.xd, c.xs, st));
         if (fused_usable(a, T)) {
             PROFILED("experts", st,
-                     tg::launch_experts_fused(lp, s, a->n_cu, c.idx, c.w, c.xq, c.xd, c.xs, c.dec_hw, c.dec_ctl,
+                     tg::launch_experts_fused(lp, s, a->n_cu, idx, w, c.xq, c.xd, c.xs, c.dec_hw, c.dec_ctl,
                                               c.dec_err, resid, out, st));
         } else {
-            PROFILED("gateup", st, tg::launch_gateup(lp, s, T, c.idx, c.xq, c.xd, c.xs, c.hq, c.hd, c.hs, st));
-            PROFILED("down", st, tg::launch_down(lp, s, T, c.idx, c.w, c.hq, c.hd, c.hs, resid, out, st));
+            PROFILED("gateup", st, tg::launch_gateup(lp, s, T, idx, c.xq, c.xd, c.xs, c.hq, c.hd, c.hs, st));
+            PROFILED("down", st, tg::launch_down(lp, s, T, idx, w, c.hq, c.hd, c.hs, resid, out, st));
         }
     }
+    if (own) return TG_OK;
     const size_t n = (size_t)T * a->s.k;
     if (idx_out) HIP_TRY(hipMemcpyAsync(idx_out, c.idx, sizeof(int32_t) * n, hipMemcpyDeviceToDevice, st));
     if (w_out) HIP_TRY(hipMemcpyAsync(w_out, c.w, sizeof(float) * n, hipMemcpyDeviceToDevice, st));
@@ -753,18 +737,9 @@ static int moe_layer_launch(tg_arena *a, const Scratch &c, int layer, const floa
     return layer_kernels(a, c, layer, x, out, resid, T, eps, idx_out, w_out, st);
 }
 
-// x <- x + MoE_l(x) for layers [l0, l0+n), in place.  Up to three tokens go
-// through the routed launches one after another (tokens are independent; 13 us
-// a token and layer at the 30B shape where the grouped layer takes about 45).
+// x <- x + MoE_l(x) for layers [l0, l0+n), in place.
 static int stack_launch(tg_arena *a, const Scratch &c, float *x, int T, int l0, int n, float eps, hipStream_t st) {
-    if (routed_usable(a, T)) {
-        for (int t = 0; t < T; t++) {
-            float *xt = x + (size_t)t * a->s.H;
-            int rc = routed_layers(a, c, l0, n, xt, xt, xt, eps, c.idx, c.w, 0, st);
-            if (rc) return rc;
-        }
-        return TG_OK;
-    }
+    if (routed_usable(a, T)) return routed_layers(a, c, l0, n, x, x, x, eps, c.idx, c.w, 0, st);
     for (int l = l0; l < l0 + n; l++) {
         int rc = layer_kernels(a, c, l, x, x, x, T, eps, nullptr, nullptr, st);
         if (rc) return rc;

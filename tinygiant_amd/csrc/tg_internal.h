@@ -249,8 +249,7 @@ hipError_t launch_sample_all(const SmpBufs &b, const float *logits, int V, float
 bool layer_dec_ok(const Shape &s, int n_cu);
 size_t dec_part_floats(const Shape &s);
 size_t dec_ow_words(const Shape &s);
-// (one or two tokens; the generation advances by n_gen)
-hipError_t launch_dec_part(const float *Wr, const float *x, const Shape &s, int tokens, float *part, uint32_t *ctl, int n_gen,
+hipError_t launch_dec_part(const float *Wr, const float *x, const Shape &s, float *part, uint32_t *ctl, int n_layers,
                            hipStream_t st);
 hipError_t launch_layer_dec(const uint8_t *layer_pl, const Shape &s, int n_cu, const float *x, const float *gn,
                             const float *part_in, const float *wr_next, float *part_out, uint64_t *hw, uint64_t *ow,

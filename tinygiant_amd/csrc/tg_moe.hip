@@ -2041,13 +2041,9 @@ __global__ __launch_bounds__(FX_THREADS) void k_layer_dec(const float *__restric
 // call's first layer (block g: group g; thread e < E the chain of expert e,
 // thread E the chain of squares), and block 0 advances the generation word
 // by n_layers (one generation per layer launch of the call).
-// grid (H/32, tokens): token t's partials at part + t * half
 __global__ __launch_bounds__(256) void k_dec_part(const float *__restrict__ Wr, const float *__restrict__ x, int E,
-                                                  int H, float *__restrict__ part, uint32_t *ctl, int n_gen,
-                                                  size_t half) {
+                                                  int H, float *__restrict__ part, uint32_t *ctl, int n_layers) {
     const int g = blockIdx.x, tid = threadIdx.x, G = H / RG;
-    x += (size_t)blockIdx.y * H;
-    part += blockIdx.y * half;
     const float4 *x4 = reinterpret_cast<const float4 *>(x + (size_t)g * RG);
     float4 xv[RG / 4];
 #pragma unroll
@@ -2077,9 +2073,9 @@ __global__ __launch_bounds__(256) void k_dec_part(const float *__restrict__ Wr, 
         }
         part[(size_t)E * G + g] = aq;
     }
-    if (g == 0 && blockIdx.y == 0 && tid == 0) {
+    if (g == 0 && tid == 0) {
         uint32_t v = __hip_atomic_load(ctl + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        for (int i = 0; i < n_gen; i++) v = next_gen(v);
+        for (int i = 0; i < n_layers; i++) v = next_gen(v);
         __hip_atomic_store(ctl + 1, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 }
@@ -2940,11 +2936,9 @@ bool layer_dec_ok(const Shape &s, int n_cu) {
            RG - rd <= FX_THREADS && lds <= 160 * 1024;
 }
 
-hipError_t launch_dec_part(const float *Wr, const float *x, const Shape &s, int tokens, float *part, uint32_t *ctl,
-                           int n_gen, hipStream_t st) {
-    if (tokens < 1 || tokens > 2) return hipErrorInvalidValue;  // part holds two buffers
-    TG_LAUNCH(k_dec_part, dim3(s.H / RG, tokens), dim3(256), 0, st, Wr, x, s.E, s.H, part, ctl, n_gen,
-              dec_part_floats(s) / 2);
+hipError_t launch_dec_part(const float *Wr, const float *x, const Shape &s, float *part, uint32_t *ctl, int n_layers,
+                           hipStream_t st) {
+    TG_LAUNCH(k_dec_part, dim3(s.H / RG), dim3(256), 0, st, Wr, x, s.E, s.H, part, ctl, n_layers);
     return hipGetLastError();
 }
 
