@@ -287,8 +287,8 @@ def test_fused_gate_up_down_across_calls(O, tglib, H, I, E, k, Ts):
         a.close()
 
 
-# mean entries per expert on both sides of the one-tile / 16 x 16 line (32) and of 16-entry items (12), odd counts; experts over several
-# one-tile items (16 experts, mean 32) and a shape the fused launches do not take (I 160: the 32 x 32 kernels)
+# mean entries per expert on both sides of the one-tile / 16 x 16 line (32) and of 16-entry items (12), odd counts; small
+# layers and a shape the fused launches do not take (I 160), both on the 32 x 32 kernels
 @pytest.mark.parametrize("H,I,E,k,T", [(2048, 768, 128, 8, 333), (2048, 768, 128, 8, 512), (2048, 768, 128, 8, 513), (2048, 768, 128, 8, 192), (2048, 768, 128, 8, 193),
                                        (512, 256, 16, 4, 128), (512, 256, 16, 4, 129), (512, 256, 32, 8, 131),
                                        (256, 160, 16, 4, 150), (256, 160, 16, 4, 300)])
@@ -323,6 +323,37 @@ def test_one_tile_chunk_counts(O, tglib, H, I, T):
         out, idx, _ = MoEBlock(a).forward(0, dev(x), return_routing=True)
         assert np.array_equal(host(idx), ridx)
         assert np.array_equal(bits(host(out)), bits(ref))
+        assert tglib.tg_arena_status(a.handle) == 0
+    finally:
+        a.close()
+
+
+# fused: the one-tile (mean 17 to 32, from 48 MB of experts) and 16 x 16 kernels (33 to 64, from 96 MB), else the 32 x 32
+# kernels' two launches; from a mean of 65 the 16 x 16 kernels, up to 16 the one-tile, whatever the layer's size
+@pytest.mark.parametrize("H,I,E,k,T,fused", [(1024, 512, 32, 4, 128, True), (1024, 512, 32, 4, 129, False), (1024, 512, 32, 4, 512, False),
+                                             (1024, 512, 32, 4, 513, True), (1024, 512, 64, 6, 341, True), (1024, 512, 64, 6, 342, False),
+                                             (2048, 1024, 32, 4, 256, True), (2048, 1024, 32, 4, 257, True)])
+def test_item_size_rule_small_layers(O, tglib, H, I, E, k, T, fused):
+    gpu_note(f"grouped layer, item size by the layer's bytes H={H} I={I} E={E} T={T}")
+    import ctypes
+    from tinygiant_amd.moe import MoEBlock
+    a, layers, routers = make_arena(O, 1, H, I, E, k, seed=131)
+
+    def launches(role):
+        n, ms = ctypes.c_int(0), ctypes.c_double(0.0)
+        assert tglib.tg_prof_read(role, ctypes.byref(n), ctypes.byref(ms)) == 0
+        return n.value
+
+    try:
+        x = O.synth_normal(131, O.stream_id(0, T, 4), 1.0, T * H).reshape(T, H)
+        ref, _, _, _ = O.moe_layer(layers[0], routers[0], H, I, E, k, x)
+        assert tglib.tg_prof_enable(1) == 0
+        try:
+            out = host(MoEBlock(a).forward(0, dev(x)))
+            assert (launches(b"gu_down_mfma"), launches(b"gateup_mfma")) == ((1, 0) if fused else (0, 1))
+        finally:
+            tglib.tg_prof_enable(0)
+        assert np.array_equal(bits(out), bits(ref))
         assert tglib.tg_arena_status(a.handle) == 0
     finally:
         a.close()

@@ -1402,20 +1402,32 @@ int mfma_item_entries(const Shape &s, int mt) {
 }
 
 // Entries per expert in a work item, in M-tiles of 32 (0: 16 entries), from the
-// batch's mean entries per expert.  Where both fused gate/up + down launches take
-// the shape, the one-tile kernel up to a mean of 32 and the 16 x 16 kernel above
-// (us a layer, 30B shape: 420 tokens 173, 181; 512 tokens 201, 199; 640 tokens 236,
-// 211; 235B: 420 tokens 539, 611; 512 tokens 616, 648; 640 tokens 703, 701).
-// Items of 16 entries let three blocks share a CU instead of two: they pay once the gate/up blocks fill five a CU (30B 16 tokens 69 us, 73
-// with 16-entry items; 32 tokens 77, 75; 64 tokens 93, 84; 235B 8 tokens 122, 128;
-// 16 tokens 164, 152) and until experts with more than 16 entries, whose weights
-// they read twice, weigh more: a mean of 8, or 12 where K is at most 8 chunks (30B
-// 192 tokens 135, 130; 235B 160 tokens 356, 365).  Other shapes keep the 32 x 32
-// kernels (two launches).
+// batch's mean entries per expert and the layer's expert bytes.  The 32 x 32
+// kernels (two launches, items of 64 entries from a mean of 17) are the ones for
+// shapes that the fused gate/up + down launches do not take, and for small layers:
+// their blocks are many and short where the others leave CUs without one.
+// The one-tile kernel instead at a mean of 17 to 32, from 48 MB of experts, and
+// the 16 x 16 kernel instead at 33 to 64, from 96 MB (us a layer of a stack at
+// means of 20, 32, 40 and 64, uniform routing, first the 32 x 32 kernels, then these: H
+// 1024, I 512, 32 experts, 28 MB 53 / 61, 60 / 65, 61 / 63, 67 / 75; I 768, 42 MB
+// 59 / 68, 66 / 76, 68 / 77, 85 / 93; I 512, 64 experts, 57 MB 61 / 64, 68 / 63, 70 / 72,
+// 97 / 87; H 2048, I 768, 32 experts, 85 MB 93 / 89, 102 / 96, 106 / 112, 145 / 131; I
+// 1024, 113 MB 100 / 95, 110 / 92, 114 / 104, 158 / 122; skewed routing moves
+// the line at 33 to 64 from 57 to 96 MB: H 2048, I 1024, 16 experts 98 / 116 at 40).
+// Large layers change from the one-tile to the 16 x 16 kernel at 32 too (30B shape:
+// 420 tokens 173, 181; 512 tokens 201, 199; 640 tokens 236, 211; 235B: 420 tokens 539,
+// 611; 512 tokens 616, 648; 640 tokens 703, 701).
+// Items of 16 entries let three blocks share a CU instead of two: they pay once
+// the gate/up blocks fill five a CU (30B 16 tokens 69 us, 73 with 16-entry items; 32
+// tokens 77, 75; 64 tokens 93, 84; 235B 8 tokens 122, 128; 16 tokens 164, 152) and
+// until experts with more than 16 entries, whose weights they read twice, weigh
+// more: a mean of 8, or 12 where K is at most 8 chunks (30B 192 tokens 135, 130; 235B
+// 160 tokens 356, 365).
 int mfma_tiles(const Shape &s, int T) {
     const int avg = (T * s.k + s.E - 1) / s.E;
     if (mfma_item_entries(s, 4) > 128 && s.nbI % MF_KC == 0) {
-        if (avg > 32) return 4;
+        if (avg > 64 || (avg > 32 && s.LB >= ((size_t)96 << 20))) return 4;
+        if (avg > 32 || (avg > 16 && s.LB < ((size_t)48 << 20))) return 2;
         // experts that T tokens select, each missed by a token with chance 1 - k / E
         const double distinct = s.E * (1.0 - std::pow(1.0 - (double)s.k / s.E, T));
         const int gxg = (s.I + 63) / 64;
