@@ -357,3 +357,30 @@ def test_item_size_rule_small_layers(O, tglib, H, I, E, k, T, fused):
         assert tglib.tg_arena_status(a.handle) == 0
     finally:
         a.close()
+
+
+# down K of 1 to 12 chunks with a last one of 1 to 7 blocks (odd block counts: row scales on 2-byte addresses)
+@pytest.mark.parametrize("H,I", [(256, 32), (512, 160), (256, 288), (768, 480), (512, 736), (256, 1056), (512, 1184), (256, 1408),
+                                 (512, 1504), (256, 2080), (512, 2880)])
+@pytest.mark.parametrize("T", [3, 9, 50])
+def test_one_tile_ragged_down(O, tglib, H, I, T):
+    """The one-tile down launch where K is not whole chunks of 8 blocks, with the combine after it and inside it."""
+    import os
+    gpu_note(f"one-tile down, ragged K, H={H} I={I} T={T}")
+    from tinygiant_amd.moe import MoEBlock
+    E, k = 16, 4
+    a, layers, routers = make_arena(O, 1, H, I, E, k, seed=137)
+    old = os.environ.pop("TG_FUSE_COMBINE", None)
+    try:
+        a.set_batch_path(a.BATCH_GROUPED)
+        x = O.synth_normal(137, O.stream_id(0, T, 4), 1.0, T * H).reshape(T, H)
+        ref, _, _, _ = O.moe_layer(layers[0], routers[0], H, I, E, k, x)
+        for fuse in ("0", "1"):
+            os.environ["TG_FUSE_COMBINE"] = fuse
+            assert np.array_equal(bits(host(MoEBlock(a).forward(0, dev(x)))), bits(ref)), f"combine inside: {fuse}"
+        assert tglib.tg_arena_status(a.handle) == 0
+    finally:
+        os.environ.pop("TG_FUSE_COMBINE", None)
+        if old is not None:
+            os.environ["TG_FUSE_COMBINE"] = old
+        a.close()

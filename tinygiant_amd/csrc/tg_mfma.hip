@@ -501,13 +501,17 @@ TG_DEV int half_sum(int v) {
     return v;
 }
 
-// One block of the one-tile kernels: item wi, row tile bx; K a whole number of
-// chunks.  GD: gate/up and down blocks of the same launch (k_mfma_small_gd): a
+// One block of the one-tile kernels: item wi, row tile bx.  K is a whole number
+// of chunks, or with RAG (down) any number of blocks: the row scales then go
+// through registers (a row's are 2-byte aligned), and the last chunk runs only
+// its blocks.  (With the 32 x 32 kernel's one tile for these K, us a layer of a
+// stack: H 2048, I 1408, 6 of 64 experts, 4 tokens 64, now 53; 64 tokens 134, 108;
+// H 2816, I 2880, 4 of 32: 116, 81 and 186, 144.)  GD: gate/up and down blocks of the same launch (k_mfma_small_gd): a
 // gate/up block stores h with agent-scope stores and, once they are
 // acknowledged, counts itself in at rdy[wi]; a down block waits (bounded)
 // until all `need` gate/up blocks of its item have, its first weights in
 // flight meanwhile, then stages h at agent scope.
-template <int M, bool PAIR, bool GD>
+template <int M, bool PAIR, bool GD, bool RAG = false>
 TG_DEV __attribute__((always_inline)) void ms_item(const uint8_t *__restrict__ layer_pl, const Shape s,
                                                    const int32_t *__restrict__ work,
                                                    const int32_t *__restrict__ entries,
@@ -524,11 +528,12 @@ TG_DEV __attribute__((always_inline)) void ms_item(const uint8_t *__restrict__ l
     constexpr int JA = FA / (NT * 16);               // DMA rounds of a chunk's rows
     constexpr int ND = FD / 256;                     // waves that stage a chunk's scales
     static_assert((M == 16 || M == 32) && JA * NT * 16 == FA && MF_KC == 8, "staging map");
+    static_assert(!RAG || (!PAIR && !GD), "gate/up rows are whole chunks");
     const int e = work[3 * wi], o = work[3 * wi + 1], c = work[3 * wi + 2];
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, n = lane & 31,
               h = lane >> 5;
     const int K = PAIR ? s.H : s.I, nb = K / QK, rows = PAIR ? s.I : s.H, k = s.k;
-    const int nch = nb / MF_KC;
+    const int nch = RAG ? (nb + MF_KC - 1) / MF_KC : nb / MF_KC;
 
     // this wave's 32 weight rows; an out-of-range tile computes on the first
     // and stores nothing
@@ -541,7 +546,8 @@ TG_DEV __attribute__((always_inline)) void ms_item(const uint8_t *__restrict__ l
     // chunk ch of the rows: load i takes rows 8i .. 8i+7, lane l row l / 8,
     // piece l % 8.  Chunks past the last are out of the buffer's range: such a
     // load moves nothing, and every step issues the same number of loads, so
-    // the waits stay exact
+    // the waits stay exact.  (RAG: pieces past a row's end are the next row's
+    // or out of range; no block uses them)
     const auto wrs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(tb + (size_t)r0 * nb * 16), 0, 32 * nb * 16,
                                                        0x00020000);
     const uint32_t wof = (uint32_t)((lane >> 3) * nb * 16 + (lane & 7) * 16);
@@ -551,8 +557,28 @@ TG_DEV __attribute__((always_inline)) void ms_item(const uint8_t *__restrict__ l
         for (int i = 0; i < 4; i++)
             w[i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wrs, (int)v, i * 8 * nb * 16, 0));
     };
-    // the rows' scales of chunks 4g .. 4g+3 (past the last chunk: its again)
+    // the rows' scales of chunks 4g .. 4g+3 (past the last chunk: its again).
+    // RAG: lane (n, h) loads row n's 16 of chunks 4g + 2h, 4g + 2h + 1 (past the
+    // last block: its again), and put_ws stores them once they are in
+    uint32_t wsv[RAG ? 16 : 1];
+    auto put_ws = [&](int g) {
+        if constexpr (RAG) {
+            uint8_t *row = smem + Lds::WS + wave * 4096 + (g & 1) * 2048 + n * 64;
+#pragma unroll
+            for (int q = 0; q < 2; q++) {
+                const uint32_t *v = wsv + 8 * q;
+                *reinterpret_cast<uint4 *>(row + (((2 * h + q) ^ ((n >> 1) & 3)) << 4)) =
+                    make_uint4(v[0] | v[1] << 16, v[2] | v[3] << 16, v[4] | v[5] << 16, v[6] | v[7] << 16);
+            }
+        }
+    };
     auto stage_ws = [&](int g) {
+        if constexpr (RAG) {
+            const uint16_t *row = reinterpret_cast<const uint16_t *>(wsc) + (size_t)n * nb;
+#pragma unroll
+            for (int j = 0; j < 16; j++) wsv[j] = row[min(32 * g + 16 * h + j, nb - 1)];
+            return;
+        }
 #pragma unroll
         for (int j = 0; j < 2; j++) {
             const int r = j * 16 + (lane >> 2), p = (lane & 3) ^ ((r >> 1) & 3);
@@ -599,14 +625,20 @@ TG_DEV __attribute__((always_inline)) void ms_item(const uint8_t *__restrict__ l
     // the activations and activation scales of chunks 2q, 2q+1 into slots
     // ch % 4.  Groups of 4 rows without an entry of the item are left out
     // (their sums are never stored).
+    // (RAG: past the row's end its last piece or scale again)
     const int8_t *asrc[JA];
+    int apc[JA];
 #pragma unroll
     for (int j = 0; j < JA; j++) {
         const int L = (j * NW + wave) * 64 + lane;  // 16-byte slot of a chunk's rows
-        const int t = L >> 4, pc = ((L & 15) - t) & 15;
-        asrc[j] = aq + (size_t)(PAIR ? ea[j] / k : ea[j]) * K + pc * 16;
+        const int t = L >> 4;
+        apc[j] = (((L & 15) - t) & 15) * 16;
+        asrc[j] = aq + (size_t)(PAIR ? ea[j] / k : ea[j]) * K;
+        if (!RAG) asrc[j] += apc[j];
     }
-    const float *dsrc = ad + (size_t)(PAIR ? ed / k : ed) * nb + (wave * 64 + lane) / M;
+    const int dbl = (wave * 64 + lane) / M;
+    const float *dsrc = ad + (size_t)(PAIR ? ed / k : ed) * nb;
+    if (!RAG) dsrc += dbl;
     auto stage_act = [&](int q) {
 #pragma unroll
         for (int cc = 0; cc < 2; cc++) {
@@ -616,24 +648,27 @@ TG_DEV __attribute__((always_inline)) void ms_item(const uint8_t *__restrict__ l
                 for (int j = 0; j < JA; j++) {
                     if (4 * (j * NW + wave) < c) {  // uniform
                         const uint32_t m0 = lds_addr(smem, Lds::ACT + (ch & 3) * FA + (j * NW + wave) * 1024);
+                        const int at = RAG ? min(apc[j] + ch * MF_KC * 32, K - 16) : ch * MF_KC * 32;
                         if constexpr (GD && !PAIR)
-                            lds_dma16_coh(asrc[j] + ch * MF_KC * 32, m0);
+                            lds_dma16_coh(asrc[j] + at, m0);
                         else
-                            lds_dma16(asrc[j] + ch * MF_KC * 32, m0);
+                            lds_dma16(asrc[j] + at, m0);
                     }
                 }
                 if (wave < ND) {  // uniform
                     const uint32_t m0 = lds_addr(smem, Lds::DX + (ch & 3) * FD + wave * 256);
+                    const int at = RAG ? min(dbl + ch * MF_KC, nb - 1) : ch * MF_KC;
                     if constexpr (GD && !PAIR)
-                        lds_dma4_coh(dsrc + ch * MF_KC, m0);
+                        lds_dma4_coh(dsrc + at, m0);
                     else
-                        lds_dma4(dsrc + ch * MF_KC, m0);
+                        lds_dma4(dsrc + at, m0);
                 }
             }
         }
     };
     stage_act(0);
     stage_act(1);
+    put_ws(0);
     if constexpr (GD && !PAIR) {
         __builtin_amdgcn_s_waitcnt(VMCNT0);
     } else {
@@ -667,13 +702,10 @@ TG_DEV __attribute__((always_inline)) void ms_item(const uint8_t *__restrict__ l
             __builtin_amdgcn_sched_barrier(0);
             wave_lds_sync();
             if (ch < nch) {  // uniform
-                const uint4 sc =
-                    *reinterpret_cast<const uint4 *>(ws_row + ((ch >> 2) & 1) * 2048 + (((ch & 3) ^ ((n >> 1) & 3)) << 4));
-                const uint32_t scw[4] = {sc.x, sc.y, sc.z, sc.w};
+                const uint8_t *scp = ws_row + ((ch >> 2) & 1) * 2048 + (((ch & 3) ^ ((n >> 1) & 3)) << 4);
                 const uint8_t *tq = smem + Lds::ACT + (ch & 3) * FA + (n & (M - 1)) * 256;
                 const float *xq = reinterpret_cast<const float *>(smem + Lds::DX + (ch & 3) * FD) + 4 * h;
-#pragma unroll
-                for (int bl = 0; bl < MF_KC; bl++) {
+                auto block = [&](int bl, uint32_t dwh) {
                     const uint4 blk = *reinterpret_cast<const uint4 *>(wb_row + ((bl ^ (n & 7)) << 4));
                     // 16 (q - 8) per byte: ((q << 4) & 0xF0) ^ 0x80, exact in int8
                     v4i wq;
@@ -682,7 +714,7 @@ TG_DEV __attribute__((always_inline)) void ms_item(const uint8_t *__restrict__ l
                     wq.z = (int)(((blk.z << nsh) & 0xF0F0F0F0u) ^ 0x80808080u);
                     wq.w = (int)(((blk.w << nsh) & 0xF0F0F0F0u) ^ 0x80808080u);
                     const v4i ta = *reinterpret_cast<const v4i *>(tq + (((2 * bl + h + n) & 15) << 4));
-                    const float dw = h2f((uint16_t)(scw[bl >> 1] >> (16 * (bl & 1)))) * 0.0625f;
+                    const float dw = h2f((uint16_t)dwh) * 0.0625f;
                     float4 dx[NG];
 #pragma unroll
                     for (int g = 0; g < NG; g++) dx[g] = *reinterpret_cast<const float4 *>(xq + bl * M + 8 * g);
@@ -698,6 +730,16 @@ TG_DEV __attribute__((always_inline)) void ms_item(const uint8_t *__restrict__ l
                             acc[r] = __builtin_fmaf(u, dxa[rr], acc[r]);
                         }
                     }
+                };
+                if (!RAG || ch + 1 < nch) {  // uniform
+                    const uint4 sc = *reinterpret_cast<const uint4 *>(scp);
+                    const uint32_t scw[4] = {sc.x, sc.y, sc.z, sc.w};
+#pragma unroll
+                    for (int bl = 0; bl < MF_KC; bl++) block(bl, scw[bl >> 1] >> (16 * (bl & 1)));
+                } else {
+#pragma unroll 1
+                    for (int bl = 0; bl < nb - ch * MF_KC; bl++)
+                        block(bl, *reinterpret_cast<const uint16_t *>(scp + 2 * bl));
                 }
                 // the sums formed here (sunk past the branches below, they would
                 // keep every block's MFMA result live and spill)
@@ -710,6 +752,7 @@ TG_DEV __attribute__((always_inline)) void ms_item(const uint8_t *__restrict__ l
                 // after it
                 if (nch > 4 && (ch & 1) && ch + 1 < nch) {
                     __builtin_amdgcn_s_waitcnt(VMCNT0 | 8);
+                    if (RAG && (ch & 3) == 3) put_ws((ch >> 2) + 1);
                     if ((ch & 3) == 3 && ch + 5 < nch) stage_ws((ch >> 2) + 2);
                     lds_barrier();
                     if (ch + 3 < nch) stage_act((ch >> 1) + 2);
@@ -809,7 +852,7 @@ TG_DEV __attribute__((always_inline)) void ms_item(const uint8_t *__restrict__ l
     }
 }
 
-template <int M, bool PAIR>
+template <int M, bool PAIR, bool RAG>
 __global__ __launch_bounds__(MS_NW * 64, ms_blocks(M)) void k_mfma_small(const uint8_t *__restrict__ layer_pl, Shape s,
                                                               const int32_t *__restrict__ work,
                                                               const int32_t *__restrict__ work_n,
@@ -819,8 +862,8 @@ __global__ __launch_bounds__(MS_NW * 64, ms_blocks(M)) void k_mfma_small(const u
                                                               float *__restrict__ od, int *__restrict__ os,
                                                               float *__restrict__ D, FuseArgs F) {
     if ((int)blockIdx.y >= work_n[0]) return;  // uniform over the block
-    ms_item<M, PAIR, false>(layer_pl, s, work, entries, aq, ad, oq, od, os, D, F, (int)blockIdx.y, (int)blockIdx.x,
-                         GdArgs());
+    ms_item<M, PAIR, false, RAG>(layer_pl, s, work, entries, aq, ad, oq, od, os, D, F, (int)blockIdx.y, (int)blockIdx.x,
+                                 GdArgs());
 }
 
 // Gate/up and down of the one-tile items in one launch: with n items (work_n,
@@ -1458,23 +1501,19 @@ static hipError_t mf_go(const uint8_t *layer_pl, const Shape &s, int wmax, const
     return hipGetLastError();
 }
 
-template <int M, bool PAIR>
+template <int M, bool PAIR, bool RAG = false>
 static hipError_t ms_go(const uint8_t *layer_pl, const Shape &s, int wmax, const int32_t *work, const int32_t *work_n,
                         const int32_t *entries, const int8_t *aq, const float *ad, int8_t *oq, float *od, int *os,
                         float *D, const FuseArgs &F, hipStream_t st) {
     static_assert(MS_NW * 32 == FC_ROWS && XT_NW * 32 == FC_ROWS, "one down block per output tile");
     const int rows = PAIR ? s.I : s.H, nb = (PAIR ? s.H : s.I) / QK;
-    // whole chunks of K (the row scales are staged in 16-byte pieces); other shapes take the 32 x 32 kernel's one tile
-    if (nb % MF_KC != 0) {
-        if (F.cnt) return hipErrorInvalidValue;
-        return mf_go<1, PAIR>(layer_pl, s, wmax, work, work_n, entries, aq, ad, oq, od, os, D, st);
-    }
+    if (RAG == (nb % MF_KC == 0)) return hipErrorInvalidValue;
     const unsigned gx = PAIR ? mf_cdiv((size_t)rows, 32 * (MS_NW / 2)) : mf_cdiv((size_t)rows, 32 * MS_NW);
     static std::atomic<uint64_t> attr{0};
-    hipError_t e = lds_attr(reinterpret_cast<const void *>(&k_mfma_small<M, PAIR>), MsLds<M>::BYTES, attr);
+    hipError_t e = lds_attr(reinterpret_cast<const void *>(&k_mfma_small<M, PAIR, RAG>), MsLds<M>::BYTES, attr);
     if (e != hipSuccess) return e;
-    TG_LAUNCH((k_mfma_small<M, PAIR>), dim3(gx, wmax), dim3(MS_NW * 64), MsLds<M>::BYTES, st, layer_pl, s, work, work_n,
-              entries, aq, ad, oq, od, os, D, F);
+    TG_LAUNCH((k_mfma_small<M, PAIR, RAG>), dim3(gx, wmax), dim3(MS_NW * 64), MsLds<M>::BYTES, st, layer_pl, s, work,
+              work_n, entries, aq, ad, oq, od, os, D, F);
     return hipGetLastError();
 }
 
@@ -1525,7 +1564,7 @@ hipError_t launch_gateup_mfma(const uint8_t *layer_pl, const Shape &s, int mt, i
 bool down_fuses(const Shape &s, int mt, int T) {
     const char *v = getenv("TG_FUSE_COMBINE");
     const bool on = v && v[0] == '1';
-    const bool kern = (mt <= 1 && s.nbI % MF_KC == 0) || (mt == 4 && mfma_item_entries(s, mt) > 128);
+    const bool kern = mt <= 1 || (mt == 4 && mfma_item_entries(s, mt) > 128);
     return on && kern && s.H % FC_ROWS == 0 && (size_t)T * s.k * s.H < ((size_t)1 << 31);
 }
 
@@ -1536,6 +1575,9 @@ hipError_t launch_down_mfma(const uint8_t *layer_pl, const Shape &s, int mt, int
     (void)hs;
     if (mt == 0) return ms_go<16, false>(layer_pl, s, wmax, work, work_n, entries, hq, hd, nullptr, nullptr, nullptr,
                                          D, F, st);
+    if (mt == 1 && s.nbI % MF_KC != 0)
+        return ms_go<32, false, true>(layer_pl, s, wmax, work, work_n, entries, hq, hd, nullptr, nullptr, nullptr, D, F,
+                                      st);
     if (mt == 1) return ms_go<32, false>(layer_pl, s, wmax, work, work_n, entries, hq, hd, nullptr, nullptr, nullptr,
                                          D, F, st);
     if (mt == 4 && mfma_item_entries(s, mt) > 128)
