@@ -30,8 +30,7 @@
 // Launches of one call (one host synchronisation at the end):
 //   k_smp_max     per-block max of the logits and a non-finite flag; clears
 //                 the histogram
-//   k_smp_exp     p
-//   k_smp_chunks  one block per 8192-value buffer: its pairwise sum
+//   k_smp_exp_chunks  p, and the pairwise sum of each 8192-value buffer
 //   k_smp_norm_select  S from the buffer sums; q = p / S; a histogram of q in
 //                 1/16 binades with counts and exact mass (units of 2^-40),
 //                 and from it the fewest top buckets whose mass provably
@@ -415,11 +414,21 @@ __global__ __launch_bounds__(SMP_T) void k_smp_max(const float *__restrict__ l, 
     }
 }
 
-__global__ __launch_bounds__(SMP_T) void k_smp_exp(const float *__restrict__ l, int V, const float *__restrict__ pmax,
-                                                   const int *__restrict__ pbad, int nb, float T,
-                                                   float *__restrict__ p, SmpCtl *ctl) {
+// One block per 8192-value buffer: p = exp((l - max) / T) and its pairwise sum,
+// read from LDS.  Few candidates leave a call bound by the host's launches, so the
+// two are one (a call over 8192 tokens with few candidates 50 us; as two launches 62).
+__global__ __launch_bounds__(1024) void k_smp_exp_chunks(const float *__restrict__ l, int V,
+                                                         const float *__restrict__ pmax, const int *__restrict__ pbad,
+                                                         int nb, float T, float *__restrict__ p,
+                                                         float *__restrict__ sums, SmpCtl *ctl) {
+    constexpr int R = NP_BUFSIZE / 1024;
+    __shared__ float ps[NP_BUFSIZE];
+    __shared__ PwTree t;
     __shared__ float s_m;
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, c0 = blockIdx.x * NP_BUFSIZE;
+    float x[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) x[r] = l[min(c0 + r * 1024 + tid, V - 1)];
     if (tid < WAVE) {
         float m = -INFINITY;
         int bad = 0;
@@ -435,22 +444,26 @@ __global__ __launch_bounds__(SMP_T) void k_smp_exp(const float *__restrict__ l, 
     }
     __syncthreads();
     const float m = s_m;
-    for (int i = blockIdx.x * SMP_T + tid; i < V; i += gridDim.x * SMP_T) {
-        const float z = (l[i] - m) / T;
-        p[i] = (float)exp((double)z);
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const int j = r * 1024 + tid;
+        if (c0 + j < V) {
+            const float z = (x[r] - m) / T, e = (float)exp((double)z);
+            p[c0 + j] = e;
+            ps[j] = e;
+        }
     }
+    __syncthreads();
+    const float s = block_pw_sum(ps, min(NP_BUFSIZE, V - c0), t);
+    if (tid == 0) sums[blockIdx.x] = s;
 }
 
-// One block per 8192-value buffer of v[0..n): its pairwise sum.  n is the
-// argument, or, when n_from_ctl, the candidate count ctl->cut.
-__global__ __launch_bounds__(1024) void k_smp_chunks(const float *__restrict__ v, int n, int n_from_ctl,
-                                                     const SmpCtl *ctl, float *__restrict__ sums) {
+// One block per 8192-value buffer of the candidates v[0..ctl->cut): its pairwise sum.
+__global__ __launch_bounds__(1024) void k_smp_chunks(const float *__restrict__ v, const SmpCtl *ctl,
+                                                     float *__restrict__ sums) {
     __shared__ PwTree t;
-    if (n_from_ctl) {
-        if (ctl->status != SMP_ST_PENDING) return;
-        n = ctl->cut;
-    }
-    const int c0 = blockIdx.x * NP_BUFSIZE;
+    if (ctl->status != SMP_ST_PENDING) return;
+    const int n = ctl->cut, c0 = blockIdx.x * NP_BUFSIZE;
     if (c0 >= n) return;
     const float s = block_pw_sum(v + c0, min(NP_BUFSIZE, n - c0), t);
     if (threadIdx.x == 0) sums[blockIdx.x] = s;
@@ -815,9 +828,8 @@ static void launch_probs(const SmpBufs &b, const float *logits, int V, float T, 
     const unsigned nb = smp_grid(V, SMP_T * 4);
     const int nchunks = (V + NP_BUFSIZE - 1) / NP_BUFSIZE;
     TG_LAUNCH(k_smp_max, dim3(nb), dim3(SMP_T), 0, st, logits, V, b.pmax, b.pbad, b.hcnt, b.hmass, b.ctl);
-    TG_LAUNCH(k_smp_exp, dim3(smp_grid(V, SMP_T * 2)), dim3(SMP_T), 0, st, logits, V, b.pmax, b.pbad, (int)nb, T,
-              b.p, b.ctl);
-    TG_LAUNCH(k_smp_chunks, dim3(nchunks), dim3(1024), 0, st, b.p, V, 0, b.ctl, b.sums);
+    TG_LAUNCH(k_smp_exp_chunks, dim3(nchunks), dim3(1024), 0, st, logits, V, b.pmax, b.pbad, (int)nb, T, b.p, b.sums,
+              b.ctl);
     if (select)
         TG_LAUNCH(k_smp_norm_select, dim3((unsigned)((V + SL_T * SL_R - 1) / (SL_T * SL_R))), dim3(SL_T), 0, st, b.p,
                   V, b.sums, nchunks, top_p, b.ctl, b.q, b.hcnt, b.hmass);
@@ -848,7 +860,7 @@ hipError_t launch_sample_large(const SmpBufs &b, int V, double top_p, double u, 
     TG_LAUNCH(k_rs_place<2>, grid, block, 0, st, b.q, b.keys2, V, b.table, b.keys, b.sq, b.sid);
     const int nchunks = (V + NP_BUFSIZE - 1) / NP_BUFSIZE;
     TG_LAUNCH(k_smp_cut, dim3(1), dim3(1024), 0, st, b.sq, V, top_p, b.ctl);
-    TG_LAUNCH(k_smp_chunks, dim3(nchunks), dim3(1024), 0, st, b.sq, 0, 1, b.ctl, b.sums);
+    TG_LAUNCH(k_smp_chunks, dim3(nchunks), dim3(1024), 0, st, b.sq, b.ctl, b.sums);
     TG_LAUNCH(k_smp_draw, dim3(1), dim3(1024), 0, st, b.sq, b.sid, b.sums, u, b.ctl);
     return hipGetLastError();
 }
