@@ -1249,6 +1249,7 @@ static hipStream_t g_lg_kv_st = nullptr;  // the KV cache's copy (lg_kv_in) and 
 static hipEvent_t g_lg_kv_ev = nullptr;
 static bool g_lg_kv_busy = false;         // copies issued on it that g_lg_st does not wait for
 static size_t g_lg_pin_off = 0;  // bounce bytes handed out since the last wait (pinned buffer below)
+static bool g_lg_open = false;   // a call has begun and nothing has waited for the streams since
 static int lg_sync();
 
 static int lg_reserve(size_t bytes) {
@@ -1268,10 +1269,10 @@ static int lg_reserve(size_t bytes) {
     }
     g_lg_dev = dev;
     if (!g_lg_st) HIP_TRY(hipStreamCreateWithFlags(&g_lg_st, hipStreamNonBlocking));
-    if (g_lg_pin_off || g_lg_kv_busy) {  // a call that failed before its closing wait left bounce slots taken
-        int rc2 = lg_sync();
-        if (rc2) return rc2;
-    }
+    // a call that failed before its closing wait left its work running: the scratch and the bounce slots are
+    // still in use, and the KV copies of the next call run beside the stream that this work is on
+    if (g_lg_open && (rc = lg_sync())) return rc;
+    g_lg_open = true;
     if (bytes > g_lg_cap) {
         if (g_lg_buf) HIP_TRY(hipFree(g_lg_buf));
         g_lg_buf = nullptr;
@@ -1291,7 +1292,7 @@ static int lg_reserve(size_t bytes) {
 // DMA from pinned memory instead of the runtime's staging of pageable
 // memory).  A call's bounce slots are handed out in order and reused only
 // after the call's closing synchronisation; a call that fails before it
-// leaves them taken until the next call that finishes, and copies that do
+// leaves them taken until the next call begins, and copies that do
 // not fit go straight from pageable memory.  Kept until process exit.
 static uint8_t *g_lg_pin = nullptr;
 constexpr size_t LG_PIN_BYTES = (size_t)1 << 20, LG_PIN_MAX = (size_t)256 << 10;
@@ -1319,12 +1320,14 @@ static int lg_h2d(void *dst, const void *src, size_t n) {
     return TG_OK;
 }
 
-// Waits for the legacy stream; every bounce slot handed out before is free
-// again afterwards.
+// Waits for the legacy stream, and for the KV copies where a call failed before
+// the stream waited for them; every bounce slot handed out before is free again
+// afterwards.
 static int lg_sync() {
     HIP_TRY(hipStreamSynchronize(g_lg_st));
-    if (g_lg_kv_busy) HIP_TRY(hipStreamSynchronize(g_lg_kv_st));  // a call failed on the way
+    if (g_lg_kv_busy) HIP_TRY(hipStreamSynchronize(g_lg_kv_st));
     g_lg_kv_busy = false;
+    g_lg_open = false;
     g_lg_pin_off = 0;  // every copy issued so far has completed
     return TG_OK;
 }
@@ -1931,15 +1934,15 @@ static LgAttnBufs lg_attn_bufs(LgCarve &c, const LgAttn &g) {
     return b;
 }
 
-// Host cache rows 0 .. kv_len-1 of every kv head into the device caches
-// [n_kv][seq][hd], and this position's RoPE table rows.
+// This position's RoPE table rows.
 static int lg_rope_in(const LgAttn &g, const LgAttnBufs &b, const float *rope_cos, const float *rope_sin) {
     const size_t half = 4 * (size_t)(g.hd / 2);
     int rc = lg_h2d(b.cs, rope_cos + (size_t)g.pos * (g.hd / 2), half);
     return rc ? rc : lg_h2d(b.sn, rope_sin + (size_t)g.pos * (g.hd / 2), half);
 }
 
-// The cached rows on a stream of their own: the host copies them out of pageable
+// Host cache rows 0 .. kv_len-1 of every kv head into the device caches
+// [n_kv][seq][hd], on a stream of their own: the host copies them out of pageable
 // memory while the projections run (4.2 MB at 1024 positions of 4 x 128: 80-100
 // us on the host either way), and the attention waits for them.
 static int lg_kv_in(const LgAttn &g, const LgAttnBufs &b, const float *kv_k, const float *kv_v) {
