@@ -1716,10 +1716,17 @@ static int lg_moe_all(const uint8_t **expert_ptrs, const float *weights, int n_e
     }
     tg::LgMoeOps P;
     int rc;
-    if ((rc = lg_moe_ops(n_experts, gp, up, dp, weights, gb, eb - 2 * gb, m.stage, P)) ||
-        (rc = lg_moe_run(P, n_experts, dx, dout, embed, inter, b, m)))
-        return rc;
-    return lg_finish(output, dout, 4 * (size_t)embed);
+    if ((rc = lg_moe_ops(n_experts, gp, up, dp, weights, gb, eb - 2 * gb, m.stage, P))) return rc;
+    // the down launch writes the bounce slot itself (pinned memory, each row once; a copy behind it took
+    // 1.7 us a call more)
+    const size_t n = 4 * (size_t)embed;
+    if (void *p = lg_pin_take(n)) {
+        if ((rc = lg_moe_run(P, n_experts, dx, static_cast<float *>(p), embed, inter, b, m)) || (rc = lg_sync())) return rc;
+        memcpy(output, p, n);
+        return TG_OK;
+    }
+    if ((rc = lg_moe_run(P, n_experts, dx, dout, embed, inter, b, m))) return rc;
+    return lg_finish(output, dout, n);
 }
 
 extern "C" void tg_moe_forward(const uint8_t **expert_ptrs, const float *weights, int n_experts, const float *input,
