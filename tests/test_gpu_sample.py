@@ -204,3 +204,30 @@ def test_sample_ordered_sum_edges(tglib, sampler_factory, V):
         check_case(tglib, s, logit_set(name, V, V + 1), T, 1.0, us=(0.0, 0.3, 0.77, 0.9999999))
         check_case(tglib, s, logit_set(name, V, V + 1), T, 0.97, us=(0.5,))
     check_case(tglib, s, np.zeros(V, np.float32), 1.0, 1.0, us=(0.25, 0.9999999))
+
+
+@pytest.mark.parametrize("top_p", [1.0, 1.5, float("nan")])
+def test_sample_full_sort_errors(tglib, sampler_factory, top_p):
+    """Bad logits where no candidate selection runs (top_p >= 1 or NaN, more than 8192 tokens): refused, and the next
+    good call on the same sampler is right."""
+    gpu_note(f"tg_sampler_run bad logits at top_p {top_p}")
+    V = 20001
+    s = sampler_factory(V)
+    l = logit_set("llm", V, 7)
+    for bad in (np.nan, np.inf):
+        for at in ((0,), (777, V - 1)):
+            b = l.copy()
+            b[list(at)] = bad
+            assert run(tglib, s, b, np.float32(1.0), top_p, 0.5)[0] == TG_E_INVALID
+    assert run(tglib, s, np.full(V, -np.inf, np.float32), np.float32(1.0), top_p, 0.5)[0] == TG_E_INVALID
+    rc, tok = run(tglib, s, l, np.float32(1.0), top_p, 0.5)
+    assert rc == 0 and tok == S.sample(l, 1.0, top_p, 0.5)[0]
+
+
+@pytest.mark.parametrize("V", [7, 8, 128, 129, 8191, 8193, 16384, 16391])
+def test_sample_buffer_edges(tglib, sampler_factory, V):
+    """The probabilities' sum at the edges of the 8192-value buffers and of the pairwise tree, few and many candidates."""
+    gpu_note(f"tg_sampler_run buffer edges V={V}")
+    s = sampler_factory(V)
+    for name, T, top_p in (("llm", 1.0, 0.9), ("flat", 0.5, 0.99), ("peaked", 0.7, 0.6)):
+        check_case(tglib, s, logit_set(name, V, V), T, top_p, us=(0.0, 0.5, 0.9999999))

@@ -2339,7 +2339,7 @@ static int sampler_new(int vocab, tg_sampler **out) {
         s->b.keys = c.take<unsigned long long>(sizeof(unsigned long long) * V);
         s->b.keys2 = c.take<unsigned long long>(sizeof(unsigned long long) * V);
         s->b.table = c.take<uint32_t>(sizeof(uint32_t) * tg::SMP_RS_TABLE);
-        s->b.sq = c.take<float>(sizeof(float) * V);
+        s->b.sq = c.take<float>(sizeof(float) * ((V + tg::SMP_PAD - 1) / tg::SMP_PAD * tg::SMP_PAD));
         s->b.sid = c.take<uint32_t>(sizeof(uint32_t) * V);
         s->b.ctl = c.take<tg::SmpCtl>(sizeof(tg::SmpCtl));
         s->dl = c.take<float>(sizeof(float) * V);

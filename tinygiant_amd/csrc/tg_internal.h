@@ -208,6 +208,7 @@ constexpr int SMP_BUCKET_SHIFT = 19, SMP_BUCKET_LOW = (127 - 63) << 4;
 constexpr int SMP_SMALL = 8192;          // candidates ranked by counting
 constexpr int SMP_RS_TABLE = (SMP_VMAX / 4096) * 1024;  // 128 blocks x 1024 digits
 constexpr int NP_BUFSIZE = 8192;         // np.sum reduces in buffers of this many values
+constexpr int SMP_PAD = 16;              // sq is read in whole groups of this many values
 constexpr int SMP_ST_PENDING = -1, SMP_ST_OK = 0, SMP_ST_INPUT = 1, SMP_ST_BOUND = 2;
 struct SmpCtl {
     float m, S;        // max logit, np.sum of p
@@ -230,7 +231,7 @@ struct SmpBufs {
     unsigned long long *hmass;    // SMP_BUCKETS
     unsigned long long *keys, *keys2;  // vocab each: the candidates' keys, the sort's passes
     uint32_t *table;              // SMP_RS_TABLE: the sort's digit counts per block
-    float *sq;                    // vocab: sorted probabilities (more than SMP_SMALL candidates)
+    float *sq;                    // vocab, rounded up to SMP_PAD: the candidates' probabilities in descending order
     uint32_t *sid;                // vocab: their token ids
     SmpCtl *ctl;
 };

@@ -236,6 +236,7 @@ template <class F> TG_DEV Hop<F> hop_scan(F c, Hop<F> v) {
 // values per lane and scan: by a block (8: cut 36, draw 72 us instead of 25 and
 // 56 at 151,936 values), by one wave (which scans its values once per binade)
 constexpr int ORD_R = 16, ORD_R1 = 8;
+static_assert(SMP_PAD % ORD_R == 0 && SMP_PAD % ORD_R1 == 0, "loads of whole runs stay in sq");
 constexpr int ORD_NW = 16;      // waves of a block scan
 constexpr int ORD_HEAD = 1024;  // values summed by one wave first (most of the binades lie there)
 constexpr int ORD_TILE = ORD_NW * WAVE * ORD_R;
@@ -800,6 +801,10 @@ __global__ __launch_bounds__(RS_T) void k_rs_place(const float *__restrict__ q,
 
 __global__ __launch_bounds__(1024) void k_smp_cut(const float *__restrict__ sq, int V, double top_p, SmpCtl *ctl) {
     __shared__ OrdLds ord;
+    if (ctl->bad) {  // (the sort ran on what the bad logits gave)
+        if (threadIdx.x == 0) ctl->status = SMP_ST_INPUT;
+        return;
+    }
     float s;
     const int c = ord_block<float, false>(sq, 1.0f, V, s, [=](float r) { return (double)r >= top_p; }, ord, nullptr);
     if (threadIdx.x == 0) ctl->cut = c >= 0 ? c + 1 : V;
