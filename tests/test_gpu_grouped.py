@@ -309,6 +309,7 @@ def test_item_size_rule_edges(O, tglib, H, I, E, k, T):
 
 # the one-tile kernels' staging rings: K of 1, 2, 3, 4, 5, 6, 9 and 12 chunks of 8 blocks (gate/up from H, down from I);
 # rows that fill no block (I 288: 9 tiles of 32, and not whole chunks); T gives items of 1 to 32 entries and split experts
+# (32-entry items throughout: 16 experts fill too few blocks for 16-entry ones)
 @pytest.mark.parametrize("H,I", [(256, 256), (512, 768), (768, 512), (1024, 1280), (1280, 1024), (1536, 256),
                                  (2304, 1536), (3072, 288)])
 @pytest.mark.parametrize("T", [2, 9, 70])
@@ -318,6 +319,7 @@ def test_one_tile_chunk_counts(O, tglib, H, I, T):
     E, k = 16, 4
     a, layers, routers = make_arena(O, 1, H, I, E, k, seed=103)
     try:
+        a.set_batch_path(a.BATCH_GROUPED)
         x = O.synth_normal(103, O.stream_id(0, T, 4), 1.0, T * H).reshape(T, H)
         ref, ridx, _, _ = O.moe_layer(layers[0], routers[0], H, I, E, k, x)
         out, idx, _ = MoEBlock(a).forward(0, dev(x), return_routing=True)
@@ -383,4 +385,22 @@ def test_one_tile_ragged_down(O, tglib, H, I, T):
         os.environ.pop("TG_FUSE_COMBINE", None)
         if old is not None:
             os.environ["TG_FUSE_COMBINE"] = old
+        a.close()
+
+
+# the 16-entry items' kernel (from five gate/up blocks a CU of 256) at odd chunk counts above 4: K of 9 and 5 chunks each way
+@pytest.mark.parametrize("H,I,E,k,T", [(2304, 1280, 80, 8, 50), (1280, 2304, 40, 4, 40)])
+def test_16_entry_items_chunk_counts(O, tglib, H, I, E, k, T):
+    gpu_note(f"16-entry items H={H} I={I} E={E} T={T}")
+    from tinygiant_amd.moe import MoEBlock
+    assert E * (1 - (1 - k / E) ** T) * ((I + 63) // 64) >= 5 * 256 and T * k <= 8 * E  # the item rule's condition
+    a, layers, routers = make_arena(O, 1, H, I, E, k, seed=139)
+    try:
+        x = O.synth_normal(139, O.stream_id(0, T, 4), 1.0, T * H).reshape(T, H)
+        ref, ridx, _, _ = O.moe_layer(layers[0], routers[0], H, I, E, k, x)
+        out, idx, _ = MoEBlock(a).forward(0, dev(x), return_routing=True)
+        assert np.array_equal(host(idx), ridx)
+        assert np.array_equal(bits(host(out)), bits(ref))
+        assert tglib.tg_arena_status(a.handle) == 0
+    finally:
         a.close()

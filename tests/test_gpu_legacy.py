@@ -361,3 +361,25 @@ def run_transformer_layer(O, L, rng, embed, n_heads, n_kv, hd, kv_max, kv_len, i
     assert_exact(gx, rx, "transformer layer x")
     assert np.array_equal(gk.view(np.uint32), rk.view(np.uint32)), "key cache"
     assert np.array_equal(gv.view(np.uint32), rv.view(np.uint32)), "value cache"
+
+
+@pytest.mark.parametrize("what", ["attention", "layer"])
+def test_large_return(O, L, what):
+    """Outputs and new cache rows of more than 256 KB: strided copies back instead of the pinned buffer."""
+    gpu_note(f"{what}, E=256 H=64/64 hd=512")
+    rng = np.random.default_rng(64)
+    embed, n_heads, n_kv, hd, kv_max, kv_len = 256, 64, 64, 512, 3, 2
+    assert 4 * (embed + 2 * n_kv * hd) > 256 << 10
+    if what == "layer":
+        run_transformer_layer(O, L, rng, embed, n_heads, n_kv, hd, kv_max, kv_len, 256, [0, 0])
+        return
+    wq, wk, wv, wo, qn, kn, c, s, kv_k, kv_v, x = attn_case(rng, False, embed, n_heads, n_kv, hd, kv_max)
+    gk, gv, out = kv_k.copy(), kv_v.copy(), np.zeros(embed, np.float32)
+    L.tg_attention_decode(ptr(wq), ptr(wk), ptr(wv), ptr(wo), ptr(qn), ptr(kn), ptr(gk), ptr(gv), kv_len, kv_max, ptr(c),
+                          ptr(s), ptr(x), ptr(out), embed, n_heads, n_kv, hd, kv_len)
+    rk, rv = kv_k.copy(), kv_v.copy()
+    ref = O.attention_decode(False, wq, wk, wv, wo, qn, kn, rk, rv, kv_len, kv_max, c, s, x, embed, n_heads, n_kv, hd,
+                             kv_len)
+    assert_exact(out, ref, "attention output")
+    assert np.array_equal(gk.view(np.uint32), rk.view(np.uint32)), "key cache"
+    assert np.array_equal(gv.view(np.uint32), rv.view(np.uint32)), "value cache"

@@ -568,7 +568,7 @@ static int layer_kernels_grouped(tg_arena *a, const Scratch &c, int layer, const
     // saves: 2048 tokens, route_q8 10.6 -> 32.4 us for group 12.6 -> 7.1 us)
     const bool mfma = mfma_usable(a, T), placed = mfma && chains;
     const int n = T * s.k;
-    const int mt = mfma ? tg::mfma_tiles(s, T) : 0, ch = mfma ? tg::mfma_item_entries(s, mt) : 0;
+    const int mt = mfma ? tg::mfma_tiles(s, T, a->n_cu) : 0, ch = mfma ? tg::mfma_item_entries(s, mt) : 0;
     const int wmax = mfma ? tg::group_work_max(s, n, ch) : 0;
     // gate/up and down in one launch where the one-tile kernels take it
     // (the combine stays a launch of its own)

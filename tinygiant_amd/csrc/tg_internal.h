@@ -321,7 +321,7 @@ hipError_t launch_group_placed(const Shape &s, int n, int ch, int cap, int32_t *
                                int32_t *offsets, int32_t *work, int32_t *work_n, int32_t *rdy, hipStream_t st);
 // int8-MFMA grouped gate/up and down (mt = M-tiles of 32 entries per item; 0: items of 16)
 bool mfma_shape_ok(const Shape &s);
-int mfma_tiles(const Shape &s, int T);
+int mfma_tiles(const Shape &s, int T, int n_cu);
 // entries per work item for the MFMA launches at mt M-tiles
 int mfma_item_entries(const Shape &s, int mt);
 hipError_t launch_gateup_mfma(const uint8_t *layer_pl, const Shape &s, int mt, int wmax, const int32_t *work,
@@ -352,8 +352,8 @@ struct GdArgs {
     int drop = -1;      // failure-channel hook: the item whose gate/up blocks never count in
     int need = 0;       // gate/up blocks per item (set by the launcher)
 };
-// the fused launch applies: one-tile items (mt == 1), the down K at most 8
-// chunks of 8 blocks, and TG_FUSE_GD not 0 (read per call)
+// the fused launch applies: one-tile items (mt 0 or 1), both K whole chunks of 8
+// blocks, and TG_FUSE_GD not 0 (read per call)
 bool gd_fuses(const Shape &s, int mt);
 hipError_t launch_gu_down_ms(const uint8_t *layer_pl, const Shape &s, int mt, int wmax, const int32_t *work,
                              const int32_t *work_n, const int32_t *entries, const int8_t *xq, const float *xd,

@@ -453,12 +453,15 @@ TG_DEV void fused_combine(const FuseArgs &F, const Shape &s, const int32_t *__re
 // doubled the L1's fill traffic.  The activations of a pair of chunks are
 // staged in one of two LDS slots while the pair before is used; one barrier
 // per pair, none when K spans at most 4 chunks.  68 KB of LDS: two blocks per CU.
-// A layer (30B / 235B shape, weights from HBM), before and after: 5 tokens 75.9 ->
-// 60.7 / 122.9 -> 103 us, 64 tokens 108.5 -> 92.7 / 314 -> 260 us.
+// With 32-entry items a layer of a stack (30B / 235B shape, weights from HBM) went
+// from 75.9 to 60.7 / 122.9 to 103 us at 5 tokens and from 108.5 to 92.7 / 314 to 260
+// at 64; one layer again and again, its experts in the last-level cache, from 60.8
+// to 54.2 us at 5 tokens (30B), 95.5 to 81.1 at 64 and 204 to 169 at 32 (235B).
 constexpr int MS_NW = 4;    // waves per block
-// weight chunks in flight per wave (with four or with the LDS reads and MFMAs of
-// the next blocks issued ahead of a block's epilogue, 16-entry items took the
-// same time and spilled)
+// weight chunks in flight per wave.  32-entry gate/up items have four: in this
+// kernel 2, 3 and 4 measured the same, where the one before it was slower with
+// four.  16-entry items with four, or with the LDS reads and MFMAs of the next
+// blocks issued ahead of a block's epilogue, took the same time and spilled.
 constexpr int ms_pf(int m, bool pair) { return m == 16 ? 2 : pair ? 4 : 3; }
 template <int M> struct MsLds {
     static constexpr int ACT = 0;                    // [4 chunks][M entries][256 bytes, 16-byte pieces rotated by the entry]
@@ -467,7 +470,7 @@ template <int M> struct MsLds {
     static constexpr int WS = WB + MS_NW * 4096;     // [wave][2][32 rows][4 chunks' scales, chunk p at p ^ (r/2 & 3)]
     static constexpr int BYTES = WS + MS_NW * 4096;
 };
-// blocks per CU (the LDS allows no more; 168 or 256 VGPRs)
+// blocks per CU (the LDS allows no more; 156 of 168 and 224, with RAG 235, of 256 VGPRs)
 constexpr int ms_blocks(int m) { return m == 16 ? 3 : 2; }
 static_assert((MsLds<16>::BYTES + 1280) * 3 <= 160 * 1024 && (MsLds<32>::BYTES + 1280) * 2 <= 160 * 1024, "LDS per CU");
 
@@ -1458,15 +1461,17 @@ int mfma_item_entries(const Shape &s, int mt) {
 // 1024, 113 MB 100 / 95, 110 / 92, 114 / 104, 158 / 122; skewed routing moves
 // the line at 33 to 64 from 57 to 96 MB: H 2048, I 1024, 16 experts 98 / 116 at 40).
 // Large layers change from the one-tile to the 16 x 16 kernel at 32 too (30B shape:
-// 420 tokens 173, 181; 512 tokens 201, 199; 640 tokens 236, 211; 235B: 420 tokens 539,
-// 611; 512 tokens 616, 648; 640 tokens 703, 701).
+// 420 tokens 173, 181; 512 tokens 201, 199, within the runs' differences; 640 tokens
+// 236, 211; 235B: 420 tokens 539, 611; 512 tokens 616, 648; 640 tokens 703, 701).
 // Items of 16 entries let three blocks share a CU instead of two: they pay once
-// the gate/up blocks fill five a CU (30B 16 tokens 69 us, 73 with 16-entry items; 32
+// the gate/up blocks of the experts that uniform routing is expected to select fill
+// five a CU (us a layer of a stack, uniform routing: 30B 16 tokens 69 us, 73 with 16-entry items; 32
 // tokens 77, 75; 64 tokens 93, 84; 235B 8 tokens 122, 128; 16 tokens 164, 152) and
 // until experts with more than 16 entries, whose weights they read twice, weigh
-// more: a mean of 8, or 12 where K is at most 8 chunks (30B 192 tokens 135, 130; 235B
-// 160 tokens 356, 365).
-int mfma_tiles(const Shape &s, int T) {
+// more: a mean of 8, or 12 where K is at most 8 chunks, a line between the two shapes
+// that were timed (30B, K 8 chunks, 192 tokens 135, 130; 235B, 16 chunks, 160 tokens
+// 356, 365).  With skewed routing they pay from fewer tokens and to fewer.
+int mfma_tiles(const Shape &s, int T, int n_cu) {
     const int avg = (T * s.k + s.E - 1) / s.E;
     if (mfma_item_entries(s, 4) > 128 && s.nbI % MF_KC == 0) {
         if (avg > 64 || (avg > 32 && s.LB >= ((size_t)96 << 20))) return 4;
@@ -1474,7 +1479,7 @@ int mfma_tiles(const Shape &s, int T) {
         // experts that T tokens select, each missed by a token with chance 1 - k / E
         const double distinct = s.E * (1.0 - std::pow(1.0 - (double)s.k / s.E, T));
         const int gxg = (s.I + 63) / 64;
-        return avg <= (s.nbH <= 8 * MF_KC ? 12 : 8) && distinct * gxg >= 1280.0 ? 0 : 1;
+        return avg <= (s.nbH <= 8 * MF_KC ? 12 : 8) && distinct * gxg >= 5.0 * n_cu ? 0 : 1;
     }
     return avg > 64 ? 4 : (avg > 16 ? 2 : 1);
 }
