@@ -509,7 +509,8 @@ TG_DEV int half_sum(int v) {
 // through registers (a row's are 2-byte aligned), and the last chunk runs only
 // its blocks.  (With the 32 x 32 kernel's one tile for these K, us a layer of a
 // stack: H 2048, I 1408, 6 of 64 experts, 4 tokens 64, now 53; 64 tokens 134, 108;
-// H 2816, I 2880, 4 of 32: 116, 81 and 186, 144.)  GD: gate/up and down blocks of the same launch (k_mfma_small_gd): a
+// H 2816, I 2880, 4 of 32: 116, 81 and 186, 144.)
+// GD: gate/up and down blocks of the same launch (k_mfma_small_gd): a
 // gate/up block stores h with agent-scope stores and, once they are
 // acknowledged, counts itself in at rdy[wi]; a down block waits (bounded)
 // until all `need` gate/up blocks of its item have, its first weights in
